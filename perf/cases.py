@@ -53,8 +53,8 @@ def listed():
         dict(name="line-start", kind="run", nx=256, ny=256, nz=512, K=8, grains=5000, steps=100),
         # the same configuration on through competitive growth
         dict(name="line-run", kind="run", nx=256, ny=256, nz=512, K=8, grains=5000, steps=2000),
-        # late in a line run: most of the window is solid and the frame follows the front
-        dict(name="window-late", kind="window", nx=256, ny=256, nz=256, K=8, grains=5000, R=0.5, front=0.78,
+        # late in a line run: most of the window is solid, the grains have coarsened, the frame follows the front
+        dict(name="window-late", kind="window", nx=256, ny=256, nz=256, K=8, grains=600, R=0.5, front=0.78,
              warm=240, steps=40),
         # a shallow window of the same kind with the reference's slot count
         dict(name="window-k5", kind="window", nx=160, ny=96, nz=80, K=5, grains=375, R=0.5, front=0.75, warm=300,
