@@ -520,287 +520,208 @@ __device__ __forceinline__ void rhs_point(const StepArgs& a, int i, int j, int k
 // Overflow policy for a point whose neighbourhood holds more than K distinct
 // ids (undefined behaviour in the reference, 3DgrainMPI/APTPhaseField.cu:222-231).
 // Kept set: the K ids ranked first by (largest phi over their entries, then
-// earliest entry reaching it).  Computed in one streaming pass over the
-// entries with a K-candidate list: a newcomer replaces the worst candidate
-// only if its phi is strictly larger.  The worst candidate's key never
-// decreases, so no id left outside can outrank it and the list ends as the
-// exact top K.  Kept ids then take slots in first-appearance order (pass A
-// again, filtered).
-template <int K>
-struct TopK {
-    int id[K];
-    float mx[K];
-    int pos[K];
-    int n;
+// earliest entry reaching it), in first-appearance order.
+//
+// A group of lanes settles one point: lane l holds the K (id, phi) entries of
+// neighbour l (8 lanes for the 7 points; 16 lanes with up to two positions
+// each, l and l + 16, for the 27), all loaded in one round trip.  K rounds
+// each pick the entry of largest phi (earliest among equals) that is left,
+// which names the next id of the ranking, and drop that id's entries; lanes
+// reduce by DPP within the group.  Then lane q updates slot q.
+//
+// Bound by latency for short lists and by VALU for long ones (~950
+// instructions per wave of 8 points).  One point per lane with a streaming
+// top-K (56 dependent pushes and a second pass over the neighbours) was one
+// long chain of loads and compares, and left all but a few CUs idle: the
+// fix-up of a 64^3 K=8 start-up fell from 53-62 to 12-13 us, of 32^3 K=5 from
+// 27 to 9 us, of 96x96x128 K=5 with the 27-point gather from 121-148 to
+// 51-122 us.  It gathers from the state; the records of the neighbours'
+// entries that the step kernel used to write for it (448 B a point at K=8)
+// cost the step more than they saved (256x256x512 start-up: step kernel 530 ->
+// 449 us without them, fix-up 93 -> 127 us).
+template <bool G27>
+struct FixGroup {
+    static constexpr int kLanes = G27 ? 16 : 8;   // lanes per point
+    static constexpr int kPos = G27 ? 2 : 1;      // neighbour positions per lane
+    static constexpr int kPoints = 64 / kLanes;   // points per wave
 };
 
-template <int K>
-__device__ __forceinline__ void topk_push(TopK<K>& c, int id, float v, int pos)
+// LDS words of one group: the kept ids' phi at the 7 stencil rows by rank
+// (8 x 8), then four rows of 8: ids and first positions by rank, rank by slot,
+// repulsion by slot.  The stride keeps a wave's groups on different banks.
+constexpr int kFixVal = 0, kFixId = 64, kFixPos = 72, kFixRank = 80, kFixRep = 88, kFixStride = 104;
+
+template <int CTRL>
+__device__ __forceinline__ int dpp_get(int v)
 {
-    // kept id: raise its maximum (empty entries hold id -1, which never
-    // reaches here)
-    bool hit = false;
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        const bool h = c.id[q] == id;
-        const bool u = h && v > c.mx[q];
-        c.mx[q] = u ? v : c.mx[q];
-        c.pos[q] = u ? pos : c.pos[q];
-        hit |= h;
-    }
-    if (hit) return;
-    // new id: append while there is room, else replace the worst candidate
-    // (smallest phi, latest position among equals) if v beats it
-    int w = 0;
-    float wm = c.mx[0];
-    int wp = c.pos[0];
-#pragma unroll
-    for (int q = 1; q < K; ++q) {
-        const bool worse = c.mx[q] < wm || (c.mx[q] == wm && c.pos[q] > wp);
-        w = worse ? q : w;
-        wm = worse ? c.mx[q] : wm;
-        wp = worse ? c.pos[q] : wp;
-    }
-    const bool full = c.n >= K;
-    const int tgt = full ? w : c.n;
-    const bool upd = !full || v > wm;
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        const bool t = upd && q == tgt;
-        c.id[q] = t ? id : c.id[q];
-        c.mx[q] = t ? v : c.mx[q];
-        c.pos[q] = t ? pos : c.pos[q];
-    }
-    c.n += full ? 0 : 1;
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false);
 }
 
-// Candidates of one neighbour point, entry p at arg/ph[base + p * L]; P is
-// the point's position in the scan order.
-template <int K>
-__device__ __forceinline__ void topk_point(const int* __restrict__ arg, const float* __restrict__ ph,
-                                           int base, int L, int P, TopK<K>& c)
+// Largest / smallest value over a group of 8 or 16 lanes, on every lane of it
+// (all lanes of the wave active): xor 1, xor 2, half-row mirror, row mirror.
+template <bool G27>
+__device__ __forceinline__ int group_max(int v)
 {
-    int ids[K];  // all 2K loads first, as in scan_point
-    float phs[K];
-#pragma unroll
-    for (int p = 0; p < K; ++p) {
-        ids[p] = arg[base + p * L];
-        phs[p] = ph[base + p * L];
-    }
-#pragma unroll
-    for (int p = 0; p < K; ++p) {
-        if (ids[p] == -1) continue;
-        topk_push(c, ids[p], phs[p], P * K + p);
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    v = max(v, dpp_get<0xB1>(v));
+    v = max(v, dpp_get<0x4E>(v));
+    v = max(v, dpp_get<0x141>(v));
+    return G27 ? max(v, dpp_get<0x140>(v)) : v;
+}
+template <bool G27>
+__device__ __forceinline__ int group_min(int v)
+{
+    v = min(v, dpp_get<0xB1>(v));
+    v = min(v, dpp_get<0x4E>(v));
+    v = min(v, dpp_get<0x141>(v));
+    return G27 ? min(v, dpp_get<0x140>(v)) : v;
 }
 
-// The K (id, phi) entries of one neighbour point, loaded one neighbour ahead
-// of their top-K pushes so that the fix-up's chain of neighbour loads
-// overlaps the pushes instead of taking one memory round trip per neighbour.
-template <int K>
-struct NbrEntries {
-    int id[K];
-    float ph[K];
-};
-
-template <int K>
-__device__ __forceinline__ void entries_load(const int* __restrict__ arg, const float* __restrict__ ph,
-                                             int base, int L, NbrEntries<K>& e)
+// phi as an integer of the same order (-0 as +0, below every float: kNoKey).
+constexpr int kNoKey = (int)0x80000000;
+__device__ __forceinline__ int phi_key(float x)
 {
-#pragma unroll
-    for (int p = 0; p < K; ++p) {
-        e.id[p] = arg[base + p * L];
-        e.ph[p] = ph[base + p * L];
-    }
+    const int b = __float_as_int(x + 0.0f);
+    return b ^ ((b >> 31) & 0x7fffffff);
 }
 
-// topk_point's pushes for entries loaded earlier; P: the point's position in
-// the scan order.
-template <int K>
-__device__ __forceinline__ void entries_push(const NbrEntries<K>& e, int P, TopK<K>& c)
+// Orders a wave's LDS accesses (DS operations of a wave complete in order).
+__device__ __forceinline__ void wave_lds_fence()
 {
-#pragma unroll
-    for (int p = 0; p < K; ++p) {
-        if (e.id[p] == -1) continue;
-        topk_push(c, e.id[p], e.ph[p], P * K + p);
-    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-// Pass A restricted to the kept ids, on one neighbour's K ids loaded earlier.
-template <int K, int S>
-__device__ __forceinline__ void ids_kept(const int (&ids)[K], Gather<K>& g, const TopK<K>& kept)
-{
-#pragma unroll
-    for (int p = 0; p < K; ++p) {
-        const int id = ids[p];
-        if (id == -1) continue;
-        bool ok = false;
-#pragma unroll
-        for (int u = 0; u < K; ++u) ok |= (kept.id[u] == id);
-        if (!ok) continue;
-        int pos = g.n;
-#pragma unroll
-        for (int q = 0; q < K; ++q) pos = (g.la[q] == id) ? q : pos;
-#pragma unroll
-        for (int q = 0; q < K; ++q) g.la[q] = (q == pos) ? id : g.la[q];
-        g.n += (pos == g.n) ? 1 : 0;
-        if (S >= 0) {
-            const uint32_t sh = 4u * (uint32_t)pos;
-            g.pm[S] = (g.pm[S] & ~(15u << sh)) | ((uint32_t)p << sh);
-        }
-    }
-}
-
-template <int K>
-__device__ __forceinline__ void ids_load(const int* __restrict__ arg, int base, int L, int (&ids)[K])
-{
-#pragma unroll
-    for (int p = 0; p < K; ++p) ids[p] = arg[base + p * L];
-}
-
-// Pass A restricted to the kept ids.
-template <int K, int S>
-__device__ __forceinline__ void scan_point_kept(const int* __restrict__ arg, int base, int L,
-                                                Gather<K>& g, const TopK<K>& kept)
-{
-    int ids[K];  // the K loads first, as in scan_point
-    ids_load<K>(arg, base, L, ids);
-    ids_kept<K, S>(ids, g, kept);
-    __builtin_amdgcn_sched_barrier(0);
-}
-
-// Pass A restricted to the kept ids over the 7 stencil points D,B,L,C,R,T,U
-// (point u at arg[bases[u] + p * L]), each point's ids loaded while the
-// previous point's are scanned.
-template <int K>
-__device__ __forceinline__ void kept_pass7(const int* __restrict__ arg, const int (&bases)[7], int L,
-                                           Gather<K>& g, const TopK<K>& c)
-{
-    int x[K], y[K];
-    ids_load<K>(arg, bases[0], L, x);
-    ids_load<K>(arg, bases[1], L, y);
-    ids_kept<K, 0>(x, g, c);
-    __builtin_amdgcn_sched_barrier(0);
-    ids_load<K>(arg, bases[2], L, x);
-    ids_kept<K, 1>(y, g, c);
-    __builtin_amdgcn_sched_barrier(0);
-    ids_load<K>(arg, bases[3], L, y);
-    ids_kept<K, 2>(x, g, c);
-    __builtin_amdgcn_sched_barrier(0);
-    ids_load<K>(arg, bases[4], L, x);
-    ids_kept<K, 3>(y, g, c);
-    __builtin_amdgcn_sched_barrier(0);
-    ids_load<K>(arg, bases[5], L, y);
-    ids_kept<K, 4>(x, g, c);
-    __builtin_amdgcn_sched_barrier(0);
-    ids_load<K>(arg, bases[6], L, x);
-    ids_kept<K, 5>(y, g, c);
-    __builtin_amdgcn_sched_barrier(0);
-    ids_kept<K, 6>(x, g, c);
-    __builtin_amdgcn_sched_barrier(0);
-}
-
-// Rolled runs of z-major positions [from, to) through pass A restricted to
-// the kept ids (ids only).
-template <int K>
-__device__ __forceinline__ void kept_run(const StepArgs& a, const Nbr& nb, int from, int to,
-                                         Gather<K>& g, const TopK<K>& c)
-{
-#pragma unroll 1
-    for (int q = from; q < to; ++q) scan_point_kept<K, -1>(a.arg, nbase_q(a, nb, q), a.L, g, c);
-}
-
+// The overflow policy and pass B for one point per group; every lane of the
+// wave calls it.  on: the group has a point (C, its element index).
 template <int K, bool G27>
-__device__ __forceinline__ void gather_overflow(const StepArgs& a, const Nbr& nb, Gather<K>& g)
+__device__ __forceinline__ void fixup_group(const StepArgs& a, unsigned C, bool on, int l, unsigned* sc,
+                                            float a_s, float epsv)
 {
-    TopK<K> c;
-    c.n = 0;
+    using F = FixGroup<G27>;
+    constexpr int E = F::kPos * K;
+    const int A = a.fnx * a.fny;
+    const int k = (int)C / A;
+    const int rem = (int)C - k * A;
+    const int j = rem / a.fnx;
+    const int i = rem - j * a.fnx;
+    int id[E], key[E];
+    float ph[E];
+    int row = -1, rowpos = 0;  // the lane's stencil row (D,B,L,C,R,T,U) and which of its positions it is
 #pragma unroll
-    for (int q = 0; q < K; ++q) {
-        c.id[q] = -1;
-        c.mx[q] = 0.0f;
-        c.pos[q] = 0;
-    }
-    gather_init(g);
-    if (!G27) {
-        const int nbs[7] = {nbase(a, nb, 1, 1, 0), nbase(a, nb, 1, 0, 1), nbase(a, nb, 0, 1, 1),
-                            nbase(a, nb, 1, 1, 1), nbase(a, nb, 2, 1, 1), nbase(a, nb, 1, 2, 1),
-                            nbase(a, nb, 1, 1, 2)};
-        NbrEntries<K> e[2];
-        entries_load<K>(a.arg, a.ph, nbs[0], a.L, e[0]);
-#pragma unroll
-        for (int u = 0; u < 7; ++u) {
-            if (u + 1 < 7) entries_load<K>(a.arg, a.ph, nbs[u + 1], a.L, e[(u + 1) & 1]);
-            entries_push<K>(e[u & 1], u, c);
-            __builtin_amdgcn_sched_barrier(0);
+    for (int t = 0; t < F::kPos; ++t) {
+        const int u = l + 16 * t;  // scan position
+        int dx, dy, dz, s;
+        bool in;
+        if (!G27) {
+            dx = u == 2 ? -1 : u == 4 ? 1 : 0;
+            dy = u == 1 ? -1 : u == 5 ? 1 : 0;
+            dz = u == 0 ? -1 : u == 6 ? 1 : 0;
+            s = u;
+            in = u < 7;
+        } else {  // z-major 27-point order (3Dgrain/APTPhaseField.cu:241-268)
+            dx = u % 3 - 1;
+            dy = u / 3 % 3 - 1;
+            dz = u / 9 - 1;
+            s = u == 4 ? 0 : u == 10 ? 1 : (u >= 12 && u <= 14) ? u - 10 : u == 16 ? 5 : u == 22 ? 6 : -1;
+            in = u < 27;
         }
-        kept_pass7<K>(a.arg, nbs, a.L, g, c);
-    } else {
-#pragma unroll 1
-        for (int q = 0; q < 27; ++q) topk_point<K>(a.arg, a.ph, nbase_q(a, nb, q), a.L, q, c);
-        kept_run<K>(a, nb, 0, 4, g, c);
-        scan_point_kept<K, 0>(a.arg, nbase_q(a, nb, 4), a.L, g, c);
-        kept_run<K>(a, nb, 5, 10, g, c);
-        scan_point_kept<K, 1>(a.arg, nbase_q(a, nb, 10), a.L, g, c);
-        kept_run<K>(a, nb, 11, 12, g, c);
-        scan_point_kept<K, 2>(a.arg, nbase_q(a, nb, 12), a.L, g, c);
-        scan_point_kept<K, 3>(a.arg, nbase_q(a, nb, 13), a.L, g, c);
-        scan_point_kept<K, 4>(a.arg, nbase_q(a, nb, 14), a.L, g, c);
-        kept_run<K>(a, nb, 15, 16, g, c);
-        scan_point_kept<K, 5>(a.arg, nbase_q(a, nb, 16), a.L, g, c);
-        kept_run<K>(a, nb, 17, 22, g, c);
-        scan_point_kept<K, 6>(a.arg, nbase_q(a, nb, 22), a.L, g, c);
-        kept_run<K>(a, nb, 23, 27, g, c);
-    }
-}
-
-// The record buffer named by the fix-up list's header (kFixHeader): entry
-// f = s*K + p of record q has its id at id[f * cap + q] and its phi at
-// ph[f * cap + q]; ph follows the 7 * K * cap ids in the same allocation.
-struct RecView {
-    int* id;
-    float* ph;
-    int cap;
-};
-
-template <int K>
-__device__ __forceinline__ RecView rec_view(const StepArgs& a)
-{
-    RecView r;
-    r.cap = (int)a.fix_list[-4];
-    r.id = *reinterpret_cast<int* const*>(a.fix_list - 2);
-    r.ph = reinterpret_cast<float*>(r.id + (size_t)7 * K * (size_t)r.cap);
-    return r;
-}
-
-// The same policy on a fix-up record: the point's 7 x K entries in scan order
-// (D,B,L,C,R,T,U, then slot), entry f = s*K + p at rid/rph[f * cap + q]
-// (written by the tile from its LDS ring, see rec_store).
-template <int K>
-__device__ __forceinline__ void gather_overflow_rec(const int* rid, const float* rph, int cap, int q,
-                                                    Gather<K>& g)
-{
-    TopK<K> c;
-    c.n = 0;
+        if (in && s >= 0) {  // at most one position of a lane
+            row = s;
+            rowpos = t;
+        }
+        in = in && on;
+        const int b = in ? bc_map(i + dx, a.fnx, a.bcx) + bc_map(j + dy, a.fny, a.bcy) * a.fnx +
+                               bc_map(k + dz, a.fnz, a.bcz) * A
+                         : (int)C;
 #pragma unroll
-    for (int u = 0; u < K; ++u) {
-        c.id[u] = -1;
-        c.mx[u] = 0.0f;
-        c.pos[u] = 0;
+        for (int p = 0; p < K; ++p) {
+            const int x = a.arg[b + p * a.L];
+            ph[t * K + p] = a.ph[b + p * a.L];
+            id[t * K + p] = in ? x : -1;
+        }
     }
-    gather_init(g);
-    NbrEntries<K> cur, nxt;
-    entries_load<K>(rid, rph, q, cap, cur);
+#pragma unroll
+    for (int e = 0; e < E; ++e) key[e] = id[e] != -1 ? phi_key(ph[e]) : kNoKey;
+    const int pos0 = l * K;  // scan position of entry e: pos0 + (16 K for the second position) + slot
+    int nk = 0;
 #pragma unroll 1
-    for (int s = 0; s < 7; ++s) {
-        if (s + 1 < 7) entries_load<K>(rid + (s + 1) * K * cap, rph + (s + 1) * K * cap, q, cap, nxt);
-        entries_push<K>(cur, s, c);
-        cur = nxt;
+    for (int r = 0; r < K; ++r) {
+        int m = key[0];
+#pragma unroll
+        for (int e = 1; e < E; ++e) m = max(m, key[e]);
+        m = group_max<G27>(m);
+        int first = 0x7fffffff;
+#pragma unroll
+        for (int e = E - 1; e >= 0; --e)
+            first = key[e] == m ? pos0 + (e / K) * 16 * K + e % K : first;
+        first = group_min<G27>(first);
+        int kid = kNoKey;
+#pragma unroll
+        for (int e = 0; e < E; ++e) kid = pos0 + (e / K) * 16 * K + e % K == first ? id[e] : kid;
+        kid = group_max<G27>(kid);
+        const bool live = m != kNoKey;
+        nk += live ? 1 : 0;
+        // the id's entries leave the ranking; its phi at this lane's stencil
+        // row is the last entry's, as the reference's overwrite gives it
+        float v = -1.0f;
+        int fp = 0x7fffffff;
+#pragma unroll
+        for (int e = E - 1; e >= 0; --e) {
+            const bool h = live && id[e] == kid;
+            fp = h ? pos0 + (e / K) * 16 * K + e % K : fp;
+            key[e] = h ? kNoKey : key[e];
+        }
+#pragma unroll
+        for (int t = 0; t < F::kPos; ++t)
+#pragma unroll
+            for (int p = 0; p < K; ++p)
+                v = live && id[t * K + p] == kid && (F::kPos == 1 || rowpos == t) ? ph[t * K + p] : v;
+        fp = group_min<G27>(fp);
+        if (row >= 0) sc[kFixVal + 8 * r + row] = __float_as_uint(v);
+        if (l == 0) {
+            sc[kFixId + r] = (unsigned)kid;
+            sc[kFixPos + r] = (unsigned)fp;
+        }
     }
-    const int bases[7] = {q, q + K * cap, q + 2 * K * cap, q + 3 * K * cap, q + 4 * K * cap,
-                          q + 5 * K * cap, q + 6 * K * cap};
-    kept_pass7<K>(rid, bases, cap, g, c);
+    wave_lds_fence();
+    if (l < K) {  // lane r: the slot of rank r
+        const unsigned mine = sc[kFixPos + l];
+        int slot = 0;
+#pragma unroll
+        for (int r = 0; r < K; ++r) slot += sc[kFixPos + r] < mine ? 1 : 0;
+        sc[kFixRank + slot] = (unsigned)l;
+    }
+    wave_lds_fence();
+    // lane q: slot q
+    const int q = min(l, K - 1);
+    const bool in = on && l < nk;
+    const int r = in ? (int)sc[kFixRank + q] : 0;
+    float v[7];
+#pragma unroll
+    for (int s = 0; s < 7; ++s) v[s] = __uint_as_float(sc[kFixVal + 8 * r + s]);
+    const int gid = (int)sc[kFixId + r];
+    const float w = v[3] + 1.0f;
+    if (l < K) sc[kFixRep + l] = in ? __float_as_uint(0.25f * w * w) : 0u;
+    wave_lds_fence();
+    float repul = 0.0f;  // empty slots add exactly +0
+#pragma unroll
+    for (int p = 0; p < K; ++p) repul += p != q ? __uint_as_float(sc[kFixRep + p]) : 0.0f;
+    wave_lds_fence();  // the words are rewritten for the group's next point
+    if (on && l < K) {
+        const int o = (int)C + l * a.L;
+        if (!in) {
+            a.arg_new[o] = -1;
+            a.ph_new[o] = -1.0f;
+        } else {
+            float T;
+            if (!thermal_T(a, i, j, k, T)) {
+                const float nv = slot_update(a, gid, v[0], v[1], v[2], v[3], v[4], v[5], v[6], repul,
+                                             T / a.L_cp, a_s, epsv);
+                a.ph_new[o] = nv;
+                a.arg_new[o] = (nv < kKillf) ? -1 : gid;
+            }
+        }
+    }
 }
 
 // One interior point: pass A, then pass B.  Returns 0 if no neighbour holds a
@@ -820,48 +741,6 @@ __device__ __forceinline__ int apt_point(const StepArgs& a, int i, int j, int k,
     stencil_bases(a, nb, b);
     rhs_point<K>(a, i, j, k, b, g, a_s, epsv);
     return g.n > 0 ? 1 : 0;
-}
-
-// Overflowed fix-up list entry q (fix-up kernels only): point index, and
-// whether the tile left the point's entries in the record buffer.
-__device__ __forceinline__ void fixup_point(const StepArgs& a, unsigned q, int& i, int& j, int& k,
-                                            bool& rec)
-{
-    const unsigned e = a.fix_list[q];
-    rec = (e & kRecFlag) != 0u;
-    const int C = (int)(e & ~kRecFlag);
-    const int A = a.fnx * a.fny;
-    k = C / A;
-    const int r = C - k * A;
-    j = r / a.fnx;
-    i = r - j * a.fnx;
-}
-
-// The overflow policy and pass B for a point whose entries are in record q.
-template <int K>
-__device__ __forceinline__ void apt_point_overflow_rec(const StepArgs& a, int i, int j, int k, int q,
-                                                       float a_s, float epsv)
-{
-    const RecView r = rec_view<K>(a);
-    Gather<K> g;
-    gather_overflow_rec<K>(r.id, r.ph, r.cap, q, g);
-    const int C = i + j * a.fnx + k * a.fnx * a.fny;
-    rhs_point<K>(a, i, j, k, C, g, a_s, epsv, [&](int s, uint32_t p) {
-        return r.ph[(s * K + (int)p) * r.cap + q];
-    });
-}
-
-// The same point under the overflow policy (fix-up kernel only).
-template <int K, bool G27>
-__device__ __forceinline__ void apt_point_overflow(const StepArgs& a, int i, int j, int k,
-                                                   float a_s, float epsv)
-{
-    const Nbr nb = make_nbr(a, i, j, k);
-    Gather<K> g;
-    gather_overflow<K, G27>(a, nb, g);
-    int b[7];
-    stencil_bases(a, nb, b);
-    rhs_point<K>(a, i, j, k, b, g, a_s, epsv);
 }
 
 // ---------------------------------------------------------------- tiled ---
@@ -1140,50 +1019,17 @@ __device__ __forceinline__ bool overflow_keeps_list(const int* iD, const int* iC
     return outside < low;
 }
 
-constexpr unsigned kNoRec = 0xFFFFFFFFu;
-
 // Append the overflowed lanes of a wave to the fix-up list (one atomic per wave).
-// With `rec`, an entry whose position has a record slot (below the record
-// capacity in the list's header) is flagged and its position returned, for
-// the caller to write the record there; kNoRec otherwise.
-__device__ __forceinline__ unsigned fixup_append(const StepArgs& a, int ovf, unsigned point,
-                                                 bool rec = false)
+__device__ __forceinline__ void fixup_append(const StepArgs& a, int ovf, unsigned point)
 {
     const unsigned long long m = __ballot(ovf);
-    if (m == 0ull) return kNoRec;
+    if (m == 0ull) return;
     const int lane = threadIdx.x & 63;
     const int leader = __ffsll((long long)m) - 1;
     unsigned base = 0;
     if (lane == leader) base = atomicAdd(a.fix_count, (unsigned)__popcll(m));
     base = __shfl(base, leader);
-    const unsigned pos = base + (unsigned)__popcll(m & ((1ull << lane) - 1ull));
-    const unsigned cap = rec ? a.fix_list[-4] : 0u;
-    const bool has = ovf && pos < cap;
-    if (ovf) a.fix_list[pos] = point | (has ? kRecFlag : 0u);
-    return has ? pos : kNoRec;
-}
-
-// Record of an overflowed point for the fix-up: its 7 x K (id, phi) entries
-// from the LDS ring, in scan order, at record pos (structure of arrays, so the
-// wave's stores and the fix-up's loads are coalesced over consecutive entries).
-template <int K, int NPT = kNPT, int HX = kHX>
-__device__ __forceinline__ void rec_store(const StepArgs& a, const int* iD, const int* iC,
-                                          const int* iU, const float* fD, const float* fC,
-                                          const float* fU, int pt, unsigned pos)
-{
-    const RecView r = rec_view<K>(a);
-    // one row at a time: only 2K values in flight, not 14K registers' worth
-#pragma unroll 1
-    for (int s = 0; s < 7; ++s) {
-        const int o = s == 1 ? pt - HX : s == 2 ? pt - 1 : s == 4 ? pt + 1 : s == 5 ? pt + HX : pt;
-        const int* ib = s == 0 ? iD : (s == 6 ? iU : iC);
-        const float* fb = s == 0 ? fD : (s == 6 ? fU : fC);
-#pragma unroll
-        for (int p = 0; p < K; ++p) {
-            r.id[(s * K + p) * r.cap + (int)pos] = ib[p * NPT + o];
-            r.ph[(s * K + p) * r.cap + (int)pos] = fb[p * NPT + o];
-        }
-    }
+    if (ovf) a.fix_list[base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = point;
 }
 
 // One z plane of a tile.  On entry the ring holds planes k-1, k, k+1.
@@ -1195,8 +1041,8 @@ __device__ __forceinline__ void rec_store(const StepArgs& a, const int* iD, cons
 // order, so the arithmetic only waits for the point's reads, never for the
 // prefetch, and staging only for the prefetch, never for the stores; every
 // path into an iteration has the same operations in flight.
-// REC: hand overflowed points to the fix-up with a record of their entries
-// (the step kernel variant used while neighbourhoods overflow).
+// REC: with the keep test (the step kernel variant used while neighbourhoods
+// overflow).
 template <int K, bool G27, bool REC = true>
 __device__ __forceinline__ void tile_plane(const StepArgs& a, PlaneLoader<K>& ld, int (*rid)[K * kNPT],
                                            float (*rph)[K * kNPT], const float* zs, int i, int j,
@@ -1265,11 +1111,8 @@ __device__ __forceinline__ void tile_plane(const StepArgs& a, PlaneLoader<K>& ld
     // A point that gathered an id may leave non-empty slots (an overflowed one
     // will, through the fix-up): mark the destination tile plane.
     if (ovf || g.n > 0) a.act_dst[k * a.ntiles + tile] = a.ep_new;
-    // Overflowed lanes are redone after the step by the per-point fix-up, from
-    // a record of their entries where one fits (7-point gather).
-    const unsigned pos = fixup_append(a, ovf, (unsigned)C, !G27 && REC);
-    if (!G27 && REC && pos != kNoRec)
-        rec_store<K>(a, rid[sD], rid[sC], rid[sU], rph[sD], rph[sC], rph[sU], pt, pos);
+    // Overflowed lanes are redone after the step by the fix-up.
+    fixup_append(a, ovf, (unsigned)C);
     if (stage_next) {
         __syncthreads();
         loader_store(ld, rid[sD], rph[sD]);
@@ -1550,16 +1393,16 @@ __device__ __forceinline__ bool edge_strip_is_column(const StepArgs& a)
 // and 6 planes, every slot's id and phi, straight from global memory into
 // the step's LDS ring with global_load_lds (K x 1188 points, exactly the
 // ring's size), then each lane runs the tile lane's gather, keep test,
-// records and slot arithmetic with row stride 3 and plane stride 198.  A
+// and slot arithmetic with row stride 3 and plane stride 198.  A
 // lane processes its point under edge_point's activity rule (the others
 // neither store nor mark nor hand over), and a pass none of whose lanes
 // does stages nothing.  Against the direct path (neighbours through L1/L2,
 // one dependent round trip per neighbour) the staging is one round trip per
-// pass, and overflowed points get the keep test and records (the direct path
-// hands every one to the fix-up without a record).  Used by the batched step
+// pass, and overflowed points get the keep test (the direct path hands every
+// one to the fix-up).  Used by the batched step
 // and by the single step's edge kernel of overflow steps (apt_edge).  Returns
-// the overflowed points the keep test settled.  REC false: neither keep test
-// nor records (every overflowed point goes to the fix-up whole).
+// the overflowed points the keep test settled.  REC false: no keep test
+// (every overflowed point goes to the fix-up).
 template <int K, bool REC = true>
 __device__ __forceinline__ unsigned edge_tile(const StepArgs& a, int seg, int k0, int k1,
                                               float a_s, float epsv)
@@ -1665,8 +1508,7 @@ __device__ __forceinline__ unsigned edge_tile(const StepArgs& a, int seg, int k0
             *pp = oph[q];
         }
         if (need && (ovf || g.n > 0)) a.act_dst[kc * a.ntiles + tile] = a.ep_new;
-        const unsigned pos = fixup_append(a, ovf, (unsigned)C, REC);
-        if (REC && pos != kNoRec) rec_store<K, ENPT, EW>(a, iD, iC, iU, fD, fC, fU, pt, pos);
+        fixup_append(a, ovf, (unsigned)C);
     }
     return nres;
 }

@@ -20,21 +20,10 @@ constexpr double kKill = -0.9999;
 constexpr float kLSf = -0.995f;
 constexpr float kKillf = -0.9999f;
 
-// Fix-up list entry flag: the point's entries are in the record buffer at the
-// entry's position (point indices stay below 2^31 since K*L does).
-constexpr unsigned kRecFlag = 0x80000000u;
-
-// The fix-up list is allocated with kFixHeader words in front of entry 0.
-// Words -4 .. -1 describe the record buffer: record capacity, 0, and the
-// buffer's address (low, high word).  The step kernel reads them from memory
-// only in waves that hand a point to the fix-up, so they cost it no uniform
-// registers (it is at its scalar register limit).
-constexpr int kFixHeader = 64;
-
 // Fix-up list length from which a step counts as overflowing for the host's
 // choice of step kernel variant: below it the plain variant's fix-up (every
 // overflowed point, gathered again through L1/L2) costs less than the
-// overflow variant's records, keep test and edge kernel.
+// overflow variant's keep test and edge kernel.
 constexpr unsigned kOvfHeavy = 32768u;
 
 // Leftover columns at the +x end narrower than this take the direct path;
@@ -55,9 +44,7 @@ struct StepArgs {
     const float* R12;      // orientation rows, 12 floats per grain (9 used)
     const float* psi_mac;  // type-4 thermal field
     unsigned long long* overflow;  // count of points with > K distinct ids
-    unsigned* fix_list;    // interior points left to the fix-up pass (capacity: interior points);
-                           // kRecFlag set: the entries of the point are in record (list position);
-                           // preceded by the record header (kFixHeader)
+    unsigned* fix_list;    // interior points left to the fix-up pass (capacity: interior points)
     // Counters of this step: fix_count[0] entries in fix_list; wl_count (below)
     // points into the same 4-word set.  Steps take three sets in turn;
     // cnt_next is the next step's, cleared by this step's plan kernel (its
@@ -115,7 +102,7 @@ struct StepArgs {
     int Nx, Ny, Nz;
     float X0_mac, Y0_mac, Z0_mac, Dx_mac;
     // The host's step kernel variant (not read by the kernels): nonzero for
-    // the one with fix-up records, keep test and the edge kernel, used while
+    // the one with keep test and edge kernel, used while
     // neighbourhoods overflow.  The fix-up reports for that choice: it writes
     // launch_index to seen[0] and, when its list holds kOvfHeavy points or
     // more, to seen[1] (pinned host memory; null: no report).
@@ -197,8 +184,8 @@ struct BatchArgs {
     int wl_cap;            // list capacity: light chunks are listed down from wl_cap - 1
     int step_blocks;
     int fix_blocks;        // workgroups (one wave each) of the batched fix-up kernel
-    // The host's batch_step variant: nonzero for the one with fix-up records
-    // and keep test (7-point gather).  The batched fix-up reports for that
+    // The host's batch_step variant: nonzero for the one with the keep test
+    // (7-point gather).  The batched fix-up reports for that
     // choice (pinned host memory; null: no report): it counts its launches in
     // cnt[9] and writes the count to seen[0] and, when the lists of all
     // members hold kOvfHeavy points or more, to seen[1].

@@ -49,10 +49,7 @@ struct pf_ctx {
     float* phi = nullptr;           // collect target
     int* alpha = nullptr;           // collect target / initial alpha (alpha_m)
     unsigned long long* counters = nullptr;  // [0] overflow points, [1] nucleation events
-    unsigned* fix_buf = nullptr;    // record header (kFixHeader words), then the fix-up list
     unsigned* fix_list = nullptr;   // overflow fix-up list, one entry per interior point
-    int* rec = nullptr;             // fix-up records: 7 x K ids, then 7 x K phis (structure of arrays)
-    unsigned rec_cap = 0;           // records: min(interior points / 8, 2^20), none for 27-point
     unsigned* fix_count = nullptr;  // three 4-word counter sets, used by steps in turn
     int* sink = nullptr;            // 128 words written by lanes that must not store
     long long* sums = nullptr;
@@ -167,8 +164,8 @@ int ctx_check(pf_ctx* c)
 int buf_index(pf_ctx* c, int which) { return which == 0 ? c->cur : 1 - c->cur; }
 
 // Launches without a reported heavy overflow (a fix-up list of kOvfHeavy
-// points or more) after which the step kernel without fix-up records and keep
-// test, its edge items inside it, is used (7-point gather).  The report lags
+// points or more) after which the step kernel without the keep test, its
+// edge items inside it, is used (7-point gather).  The report lags
 // the launches by the queue's depth (at most kLeadEvery * kLeadSlots); either
 // variant gives the same bits.  The lag and the quiet period are kept short:
 // the overflow variant's edge kernel costs 15-35 us per launch once little
@@ -383,8 +380,8 @@ void free_ctx(pf_ctx* c)
     void* bufs[] = {c->ph[0], c->ph[1], c->arg[0], c->arg[1], c->x, c->y, c->z, c->zbuf,
                     c->R12, c->psi_mac, c->T3d, c->phi0, c->phi, c->alpha, c->counters,
                     c->sums, c->alpha_full, c->loss, c->nstatus, c->ball,
-                    c->fix_buf, c->fix_count, c->sink, c->act[0], c->act[1],
-                    c->wl_item, c->wl_need, c->wl_act, c->rec};
+                    c->fix_list, c->fix_count, c->sink, c->act[0], c->act[1],
+                    c->wl_item, c->wl_need, c->wl_act};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (c->seen) (void)hipHostFree(c->seen);
@@ -510,7 +507,7 @@ int batch_upload(pf_batch* b, const std::vector<int>& first_step, int use_iuc, B
     return PF_OK;
 }
 
-// The step kernel variant of the next batched step (1: fix-up records and
+// The step kernel variant of the next batched step (1: with the
 // keep test), from the fix-up's reports as for a single context.
 int batch_variant(pf_batch* b)
 {
@@ -706,7 +703,7 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
         (rc = dalloc(&c->zbuf, p.fnz)) || (rc = dalloc(&c->phi0, (size_t)L)) ||
         (rc = dalloc(&c->phi, (size_t)L)) || (rc = dalloc(&c->alpha, (size_t)L)) ||
         (rc = dalloc(&c->counters, 2)) || (rc = dalloc(&c->sums, p.fnz)) ||
-        (rc = dalloc(&c->fix_buf, kFixHeader + (size_t)(c->fix_alloc = (long long)(p.fnx - 2) * (p.fny - 2) * (p.fnz - 2)))) ||
+        (rc = dalloc(&c->fix_list, (size_t)(c->fix_alloc = (long long)(p.fnx - 2) * (p.fny - 2) * (p.fnz - 2)))) ||
         (rc = dalloc(&c->fix_count, 12)) || (rc = dalloc(&c->sink, 128)) ||
         (rc = dalloc(&c->act[0], (size_t)c->ntiles * p.fnz)) ||
         (rc = dalloc(&c->act[1], (size_t)c->ntiles * p.fnz)) ||
@@ -714,17 +711,6 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
         (rc = dalloc(&c->wl_need, (size_t)c->nzchunk * c->items_chunk + 1)) ||
         (rc = dalloc(&c->wl_act, (size_t)c->nzchunk * c->items_chunk + 1)))
         return bail(rc);
-    if (!p.gather27) {
-        // records of the overflowed points the tile hands to the fix-up (the
-        // first positions of the list; later ones are gathered from the state)
-        const long long interior = (long long)(p.fnx - 2) * (p.fny - 2) * (p.fnz - 2);
-        c->rec_cap = (unsigned)std::max(1LL, std::min(interior / 8, 1LL << 20));
-        if ((rc = dalloc(&c->rec, (size_t)c->rec_cap * 7 * p.K * 2))) return bail(rc);
-    }
-    c->fix_list = c->fix_buf + kFixHeader;
-    unsigned hdr[4] = {c->rec_cap, 0u, 0u, 0u};
-    std::memcpy(&hdr[2], &c->rec, sizeof(int*));
-    static_assert(sizeof(int*) == 8, "record header holds a 64-bit address");
     c->h_sums.resize(p.fnz);
     for (int b = 0; b < 2; ++b) {
         if (hipMemsetD32Async((hipDeviceptr_t)c->ph[b], 0xBF800000u, nst, c->stream) != hipSuccess ||
@@ -733,7 +719,6 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
     }
     if (hipMemsetAsync(c->counters, 0, 2 * sizeof(unsigned long long), c->stream) != hipSuccess ||
         hipMemsetAsync(c->fix_count, 0, 12 * sizeof(unsigned), c->stream) != hipSuccess ||
-        hipMemcpyAsync(c->fix_list - 4, hdr, sizeof(hdr), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
         hipMemsetAsync(c->alpha, 0, L * sizeof(int), c->stream) != hipSuccess ||
         hipMemsetAsync(c->act[0], 0, (size_t)c->ntiles * p.fnz * sizeof(unsigned), c->stream) != hipSuccess ||
         hipMemsetAsync(c->act[1], 0, (size_t)c->ntiles * p.fnz * sizeof(unsigned), c->stream) != hipSuccess ||

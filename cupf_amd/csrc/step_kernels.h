@@ -17,7 +17,7 @@ namespace {
 // chunks.  Every workgroup leaves once the items are exhausted; nothing waits
 // on another workgroup.
 // OVF: the variant for steps whose neighbourhoods overflow K (in-tile keep
-// test, fix-up records; 7-point gather only); the host picks it per launch
+// test; 7-point gather only); the host picks it per launch
 // (StepArgs::ovf_variant).  Its edge items are apt_edge's, on a second stream.
 template <int K, bool G27, bool OVF>
 __global__ __launch_bounds__(kBlock) void apt_step_tiled(StepArgs a)
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kBlock) void apt_step_tiled(StepArgs a)
 
 // The edge items (the +x strip outside the tiles) of an overflow step (7-point
 // gather): one workgroup per item; a one-column strip as edge tiles (keep
-// test and records), other strips on the direct path.  Out of the step kernel
+// test), other strips on the direct path.  Out of the step kernel
 // so its tile march keeps registers (206 against 240 VGPRs, fewer scalar
 // spills), and on a second stream that forks after the plan kernel and joins
 // before the fix-up, so its workgroups run beside the step kernel's.  The two
@@ -98,22 +98,8 @@ __global__ __launch_bounds__(kBlock) void apt_edge(StepArgs a)
 // lives in this step's counter set, which the next-but-one plan kernel
 // clears, so nothing here has to wait for the other workgroups.
 template <int K, bool G27>
-__device__ __forceinline__ void fixup_run(const StepArgs& a_arg, int blk, int nblk)
+__device__ __forceinline__ void fixup_run(const StepArgs& a, int blk, int nblk)
 {
-    // The arguments are read from an LDS copy: with them in scalar registers
-    // the compiler keeps 229 VGPRs live (2 waves/SIMD); from LDS it needs 92
-    // for K=8 (5 waves/SIMD; 120 and 4 with the neighbour entries loaded one
-    // neighbour ahead), and each entry is a long chain of dependent loads that
-    // only more waves in flight can overlap (more workgroups per CU made the
-    // start-up transient of the 256x256x512 run 14 % faster than 2).
-    __shared__ StepArgs s_a;
-    constexpr int kWords = (int)(sizeof(StepArgs) / 4);
-    static_assert(sizeof(StepArgs) % 4 == 0 && kWords <= kFixLanes, "StepArgs staging");
-    if ((int)threadIdx.x < kWords)
-        reinterpret_cast<unsigned*>(&s_a)[threadIdx.x] =
-            reinterpret_cast<const unsigned*>(&a_arg)[threadIdx.x];
-    __syncthreads();
-    const StepArgs& a = s_a;
     const unsigned n = __atomic_load_n(a.fix_count, __ATOMIC_RELAXED);
     if (blk == 0 && threadIdx.x == 0 && a.seen) {  // for the host's variant choice
         if (n >= kOvfHeavy) a.seen[1] = a.launch_index;
@@ -123,13 +109,17 @@ __device__ __forceinline__ void fixup_run(const StepArgs& a_arg, int blk, int nb
     if (blk == 0 && threadIdx.x == 0) atomicAdd(a.overflow, (unsigned long long)n);
     const float a_s = 1.0f + 3.0f * a.kin_delta;
     const float epsv = -4.0f * a.kin_delta / a_s;
+    using F = FixGroup<G27>;
+    __shared__ unsigned s_fix[(kFixLanes / F::kLanes) * kFixStride];
+    const int l = threadIdx.x & (F::kLanes - 1), grp = threadIdx.x / F::kLanes;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // wave units of kPoints entries, the first of every workgroup before the
+    // second of any, so a short list is spread over the CUs
 #pragma unroll 1
-    for (unsigned q = blk * kFixLanes + threadIdx.x; q < n; q += nblk * kFixLanes) {
-        int i, j, k;
-        bool rec;
-        fixup_point(a, q, i, j, k, rec);
-        if (!G27 && rec) apt_point_overflow_rec<K>(a, i, j, k, (int)q, a_s, epsv);
-        else apt_point_overflow<K, G27>(a, i, j, k, a_s, epsv);
+    for (unsigned u = (unsigned)(w * nblk + blk); u * F::kPoints < n; u += (unsigned)(nblk * (kFixLanes / 64))) {
+        const unsigned e = u * F::kPoints + (unsigned)(grp & (F::kPoints - 1));
+        const bool on = e < n;
+        fixup_group<K, G27>(a, a.fix_list[on ? e : u * F::kPoints], on, l, s_fix + grp * kFixStride, a_s, epsv);
     }
 }
 
@@ -234,41 +224,53 @@ __global__ __launch_bounds__(kBlock) void batch_step(BatchArgs b)
 template <int K, bool G27>
 __global__ __launch_bounds__(kFixLanes) void batch_fixup(BatchArgs b)
 {
-    __shared__ unsigned s_pre[kMaxBatch + 1];
+    using F = FixGroup<G27>;
+    __shared__ unsigned s_fix[(kFixLanes / F::kLanes) * kFixStride];
+    __shared__ unsigned s_pre[kMaxBatch + 1];  // wave units of the simulations before each
+    __shared__ unsigned s_total;
     for (int t = threadIdx.x; t < b.n; t += kFixLanes)
         s_pre[t + 1] = __atomic_load_n(b.sims[t].a.fix_count, __ATOMIC_RELAXED);
     __syncthreads();
     if (threadIdx.x == 0) {
         s_pre[0] = 0u;
+        unsigned total = 0u;
         for (int t = 0; t < b.n; ++t) {
             const unsigned c = s_pre[t + 1];
             if (blockIdx.x == 0 && c) atomicAdd(b.sims[t].a.overflow, (unsigned long long)c);
-            s_pre[t + 1] = s_pre[t] + c;
+            s_pre[t + 1] = s_pre[t] + (c + F::kPoints - 1) / F::kPoints;
+            total += c;
         }
+        s_total = total;
     }
     __syncthreads();
-    const unsigned total = s_pre[b.n];
+    const unsigned total = s_total, units = s_pre[b.n];
     if (blockIdx.x == 0 && threadIdx.x == 0 && b.seen) {  // for the host's variant choice
         const unsigned long long idx = ++b.cnt[9];
         if (total >= kOvfHeavy) b.seen[1] = idx;
         b.seen[0] = idx;
     }
-    for (unsigned g = blockIdx.x * kFixLanes + threadIdx.x; g < total; g += gridDim.x * kFixLanes) {
-        int lo = 0, hi = b.n - 1;  // last simulation whose range starts at or before g
+    const int l = threadIdx.x & (F::kLanes - 1), grp = threadIdx.x / F::kLanes;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    typedef const __attribute__((address_space(4))) BatchSim CSim;
+    const CSim* sims = (const CSim*)b.sims;
+#pragma unroll 1
+    for (unsigned u = (unsigned)(w * (int)gridDim.x + (int)blockIdx.x); u < units;
+         u += (unsigned)((int)gridDim.x * (kFixLanes / 64))) {
+        int lo = 0, hi = b.n - 1;  // last simulation whose units start at or before u
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
-            if (s_pre[mid] <= g) lo = mid;
+            if (s_pre[mid] <= u) lo = mid;
             else hi = mid - 1;
         }
-        const StepArgs& a = b.sims[lo].a;
-        const unsigned q = g - s_pre[lo];
-        int i, j, k;
-        bool rec;
-        fixup_point(a, q, i, j, k, rec);
+        lo = __builtin_amdgcn_readfirstlane(lo);
+        const StepArgs& a = *(const StepArgs*)&sims[lo].a;
+        const unsigned n = __atomic_load_n(a.fix_count, __ATOMIC_RELAXED);
+        const unsigned e0 = (u - s_pre[lo]) * F::kPoints;
+        const unsigned e = e0 + (unsigned)(grp & (F::kPoints - 1));
         const float a_s = 1.0f + 3.0f * a.kin_delta;
         const float epsv = -4.0f * a.kin_delta / a_s;
-        if (!G27 && rec) apt_point_overflow_rec<K>(a, i, j, k, (int)q, a_s, epsv);
-        else apt_point_overflow<K, G27>(a, i, j, k, a_s, epsv);
+        const bool on = e < n;
+        fixup_group<K, G27>(a, a.fix_list[on ? e : e0], on, l, s_fix + grp * kFixStride, a_s, epsv);
     }
 }
 
