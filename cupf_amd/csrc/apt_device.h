@@ -160,158 +160,6 @@ __device__ __forceinline__ bool thermal_T(const StepArgs& a, int i, int j, int k
     return thermal_Tv(a, nx ? a.x[i] : 0.0f, ny ? a.y[j] : 0.0f, a.z[k], T);
 }
 
-// Gather state of one point.  la: slot ids in first-appearance order (no
-// holes, n filled).  pm[s]: 4-bit nibble q holds the neighbour slot p whose id
-// landed in slot q at stencil row s (D,B,L,C,R,T,U), 15 = none; the last
-// matching p wins, as the reference's overwrite does.
-template <int K>
-struct Gather {
-    int la[K];
-    uint32_t pm[7];
-    int n;
-    bool ovf;
-};
-
-template <int K>
-__device__ __forceinline__ void gather_init(Gather<K>& g)
-{
-#pragma unroll
-    for (int q = 0; q < K; ++q) g.la[q] = -1;
-#pragma unroll
-    for (int s = 0; s < 7; ++s) g.pm[s] = 0xffffffffu;
-    g.n = 0;
-    g.ovf = false;
-}
-
-// Pass A for one neighbour point (3DgrainMPI/APTPhaseField.cu:215-232): load
-// its K ids and probe-insert them.  la has no holes, so the probe returns the
-// matching slot or slot n.  S is the stencil row (-1: 27-point extra point).
-template <int K, int S>
-__device__ __forceinline__ void scan_point(const int* __restrict__ arg, int base, int L,
-                                           Gather<K>& g)
-{
-    // the K loads go out together: a load inside the probe loop would sit
-    // behind the previous probe's branches and wait out the memory latency
-    // once per slot
-    int ids[K];
-#pragma unroll
-    for (int p = 0; p < K; ++p) ids[p] = arg[base + p * L];
-#pragma unroll
-    for (int p = 0; p < K; ++p) {
-        const int id = ids[p];
-        if (id == -1) continue;
-        int pos = g.n;
-#pragma unroll
-        for (int q = 0; q < K; ++q) pos = (g.la[q] == id) ? q : pos;
-        if (pos >= K) {
-            g.ovf = true;
-            continue;
-        }
-        if (pos == g.n) {  // a new id takes the next free slot
-#pragma unroll
-            for (int q = 0; q < K; ++q) g.la[q] = (q == pos) ? id : g.la[q];
-            ++g.n;
-        }
-        if (S >= 0) {
-            const uint32_t sh = 4u * (uint32_t)pos;
-            g.pm[S] = (g.pm[S] & ~(15u << sh)) | ((uint32_t)p << sh);
-        }
-    }
-    // one neighbour point's loads in flight per lane; occupancy supplies the
-    // rest of the memory parallelism
-    __builtin_amdgcn_sched_barrier(0);
-}
-
-// Neighbour bases of an interior point through the per-axis halo maps.
-struct Nbr {
-    int xs[3], ys[3], zs[3];  // (minus, centre, plus) per axis, already mapped
-};
-
-__device__ __forceinline__ Nbr make_nbr(const StepArgs& a, int i, int j, int k)
-{
-    Nbr n;
-    n.xs[0] = bc_map(i - 1, a.fnx, a.bcx); n.xs[1] = i; n.xs[2] = bc_map(i + 1, a.fnx, a.bcx);
-    n.ys[0] = bc_map(j - 1, a.fny, a.bcy); n.ys[1] = j; n.ys[2] = bc_map(j + 1, a.fny, a.bcy);
-    n.zs[0] = bc_map(k - 1, a.fnz, a.bcz); n.zs[1] = k; n.zs[2] = bc_map(k + 1, a.fnz, a.bcz);
-    return n;
-}
-
-__device__ __forceinline__ int nbase(const StepArgs& a, const Nbr& nb, int xi, int yi, int zi)
-{
-    return nb.xs[xi] + nb.ys[yi] * a.fnx + nb.zs[zi] * a.fnx * a.fny;
-}
-
-// Base of z-major neighbour position q = xi + 3*yi + 9*zi (0..26) chosen at
-// run time, mapped from the centre point (nb.xs[1], nb.ys[1], nb.zs[1]).
-// Arithmetic only: a run-time pick among the Nbr fields compiles to an
-// indexed load from a private copy of the struct (scratch memory).
-__device__ __forceinline__ int nbase_q(const StepArgs& a, const Nbr& nb, int q)
-{
-    const int xi = q % 3, yi = (q / 3) % 3, zi = q / 9;
-    const int x = bc_map(nb.xs[1] + xi - 1, a.fnx, a.bcx);
-    const int y = bc_map(nb.ys[1] + yi - 1, a.fny, a.bcy);
-    const int z = bc_map(nb.zs[1] + zi - 1, a.fnz, a.bcz);
-    return x + y * a.fnx + z * a.fnx * a.fny;
-}
-
-// Rolled runs of z-major positions [from, to) that carry ids only (direct path).
-template <int K>
-__device__ __forceinline__ void scan_point_run(const StepArgs& a, const Nbr& nb, int from, int to,
-                                               Gather<K>& g);
-
-// Stencil row bases D,B,L,C,R,T,U (stencil = -3..3, 3DgrainMPI/APTPhaseField.cu:211-214).
-__device__ __forceinline__ void stencil_bases(const StepArgs& a, const Nbr& nb, int (&b)[7])
-{
-    b[0] = nbase(a, nb, 1, 1, 0);
-    b[1] = nbase(a, nb, 1, 0, 1);
-    b[2] = nbase(a, nb, 0, 1, 1);
-    b[3] = nbase(a, nb, 1, 1, 1);
-    b[4] = nbase(a, nb, 2, 1, 1);
-    b[5] = nbase(a, nb, 1, 2, 1);
-    b[6] = nbase(a, nb, 1, 1, 2);
-}
-
-template <int K>
-__device__ __forceinline__ void scan_point_run(const StepArgs& a, const Nbr& nb, int from, int to,
-                                               Gather<K>& g)
-{
-#pragma unroll 1
-    for (int q = from; q < to; ++q) scan_point<K, -1>(a.arg, nbase_q(a, nb, q), a.L, g);
-}
-
-// Pass A over the whole neighbourhood in the reference's scan order.
-template <int K, bool G27>
-__device__ __forceinline__ void scan_all(const StepArgs& a, const Nbr& nb, Gather<K>& g)
-{
-    if (!G27) {
-        scan_point<K, 0>(a.arg, nbase(a, nb, 1, 1, 0), a.L, g);
-        scan_point<K, 1>(a.arg, nbase(a, nb, 1, 0, 1), a.L, g);
-        scan_point<K, 2>(a.arg, nbase(a, nb, 0, 1, 1), a.L, g);
-        scan_point<K, 3>(a.arg, nbase(a, nb, 1, 1, 1), a.L, g);
-        scan_point<K, 4>(a.arg, nbase(a, nb, 2, 1, 1), a.L, g);
-        scan_point<K, 5>(a.arg, nbase(a, nb, 1, 2, 1), a.L, g);
-        scan_point<K, 6>(a.arg, nbase(a, nb, 1, 1, 2), a.L, g);
-    } else {
-        // z-major 27-point order (3Dgrain/APTPhaseField.cu:241-268), position
-        // q = xi + 3*yi + 9*zi.  The stencil rows keep phi: D=4 B=10 L=12 C=13
-        // R=14 T=16 U=22; the other 20 positions only contribute ids and run as
-        // rolled loops (same order) to keep the code size down.
-        scan_point_run<K>(a, nb, 0, 4, g);
-        scan_point<K, 0>(a.arg, nbase_q(a, nb, 4), a.L, g);
-        scan_point_run<K>(a, nb, 5, 10, g);
-        scan_point<K, 1>(a.arg, nbase_q(a, nb, 10), a.L, g);
-        scan_point_run<K>(a, nb, 11, 12, g);
-        scan_point<K, 2>(a.arg, nbase_q(a, nb, 12), a.L, g);
-        scan_point<K, 3>(a.arg, nbase_q(a, nb, 13), a.L, g);
-        scan_point<K, 4>(a.arg, nbase_q(a, nb, 14), a.L, g);
-        scan_point_run<K>(a, nb, 15, 16, g);
-        scan_point<K, 5>(a.arg, nbase_q(a, nb, 16), a.L, g);
-        scan_point_run<K>(a, nb, 17, 22, g);
-        scan_point<K, 6>(a.arg, nbase_q(a, nb, 22), a.L, g);
-        scan_point_run<K>(a, nb, 23, 27, g);
-    }
-}
-
 // Orientation rows of a slot: the grain's rotation where its centre phi
 // exceeds LS (double compare), the identity elsewhere
 // (3DgrainMPI/APTPhaseField.cu:258-273).
@@ -360,161 +208,6 @@ __device__ __forceinline__ float slot_update(const StepArgs& a, int gid, float p
 {
     return slot_update_r(a, slot_rot(a, gid, phC), phD, phB, phL, phC, phR, phT, phU, repul, Up,
                          a_s, epsv);
-}
-
-// Pass B: right-hand side and explicit Euler update of every slot of one point
-// (3DgrainMPI/APTPhaseField.cu:238-351).  phi_at(S, p) returns the phi of
-// neighbour slot p at stencil row S; only the filled slots' values are read.
-template <int K, class PhiAt>
-__device__ __forceinline__ void rhs_point(const StepArgs& a, int i, int j, int k, int C,
-                                          const Gather<K>& g, float a_s, float epsv, PhiAt&& phi_at)
-{
-    float* __restrict__ phn = a.ph_new;
-    int* __restrict__ agn = a.arg_new;
-    const int L = a.L;
-    if (g.n == 0) {
-#pragma unroll
-        for (int q = 0; q < K; ++q) {
-            agn[C + q * L] = -1;
-            phn[C + q * L] = -1.0f;
-        }
-        return;
-    }
-    float T;
-    const bool skip = thermal_T(a, i, j, k, T);
-    const float Up = T / a.L_cp;
-    // centre phi of every slot first: the repulsion sums over the other slots.
-    // Reads are unconditional (an absent slot reads slot 0 and is replaced by
-    // -1 afterwards) so each group of them goes out together instead of one
-    // memory latency per read.
-    float pc[K];
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        const uint32_t p = (g.pm[3] >> (4 * q)) & 15u;
-        const float x = phi_at(3, p < (uint32_t)K ? p : 0u);
-        pc[q] = (q < g.n && p != 15u) ? x : -1.0f;
-    }
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        const int o = C + q * L;
-        if (q >= g.n) {
-            agn[o] = -1;
-            phn[o] = -1.0f;
-            continue;
-        }
-        if (skip) continue;
-        float v[7];
-#pragma unroll
-        for (int s = 0; s < 7; ++s) {
-            if (s == 3) {
-                v[s] = pc[q];
-            } else {
-                const uint32_t p = (g.pm[s] >> (4 * q)) & 15u;
-                const float x = phi_at(s, p < (uint32_t)K ? p : 0u);
-                v[s] = (p != 15u) ? x : -1.0f;
-            }
-        }
-        const int gid = g.la[q];
-        float repul = 0.0f;
-#pragma unroll
-        for (int p = 0; p < K; ++p) {
-            if (p != q && p < g.n) {
-                const float w = pc[p] + 1.0f;
-                repul += 0.25f * w * w;
-            }
-        }
-        const float nv = slot_update(a, gid, v[0], v[1], v[2], v[3], v[4], v[5], v[6], repul, Up,
-                                     a_s, epsv);
-        phn[o] = nv;
-        agn[o] = (nv < kKillf) ? -1 : gid;
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
-// Pass B into registers, in two phases so that the memory reads of a point
-// (orientation rows, the paraboloid field) can be issued before the next
-// plane's prefetch: slot_prep evaluates the thermal field, the centre phi of
-// every slot and the rows; slot_finish computes the new slot values into
-// out_id/out_ph.  wr is false only for slots the reference leaves untouched
-// (the thermal `continue`).  The caller then issues one straight-line block
-// of stores.
-template <int K>
-struct SlotPrep {
-    float pc[K];
-    float Up;
-    bool skip;
-};
-
-template <int K, class PhiAt>
-__device__ __forceinline__ void slot_prep(const StepArgs& a, const Gather<K>& g, float xi, float yj,
-                                          float zk, PhiAt&& phi_at, SlotPrep<K>& sp)
-{
-    float T;
-    sp.skip = thermal_Tv(a, xi, yj, zk, T);
-    sp.Up = T / a.L_cp;
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        const uint32_t p = (g.pm[3] >> (4 * q)) & 15u;
-        sp.pc[q] = (q < g.n && p != 15u) ? phi_at(3, p) : -1.0f;
-
-    }
-}
-
-template <int K, class PhiAt>
-__device__ __forceinline__ void slot_finish(const StepArgs& a, const Gather<K>& g,
-                                            const SlotPrep<K>& sp, float a_s, float epsv,
-                                            PhiAt&& phi_at, int (&out_id)[K], float (&out_ph)[K],
-                                            bool& wr)
-{
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        out_id[q] = -1;
-        out_ph[q] = -1.0f;
-    }
-    wr = true;
-    if (g.n == 0) return;
-    wr = !sp.skip;
-    if (sp.skip) return;
-    // 0.25*(phiC_p+1)^2 of every filled slot, once per point
-    float rw[K];
-#pragma unroll
-    for (int p = 0; p < K; ++p) {
-        const float w = sp.pc[p] + 1.0f;
-        rw[p] = 0.25f * w * w;
-    }
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        if (q >= g.n) continue;
-        float v[7];
-#pragma unroll
-        for (int s = 0; s < 7; ++s) {
-            if (s == 3) {
-                v[s] = sp.pc[q];
-            } else {
-                const uint32_t p = (g.pm[s] >> (4 * q)) & 15u;
-                v[s] = (p != 15u) ? phi_at(s, p) : -1.0f;
-            }
-        }
-        const int gid = g.la[q];
-        float repul = 0.0f;
-#pragma unroll
-        for (int p = 0; p < K; ++p)
-            if (p != q && p < g.n) repul += rw[p];
-        const float nv = slot_update_r(a, slot_rot(a, gid, sp.pc[q]), v[0], v[1], v[2], v[3], v[4], v[5], v[6], repul,
-                                       sp.Up, a_s, epsv);
-        out_ph[q] = nv;
-        out_id[q] = (nv < kKillf) ? -1 : gid;
-    }
-}
-
-// Direct-path pass B: phi straight from global memory.
-template <int K>
-__device__ __forceinline__ void rhs_point(const StepArgs& a, int i, int j, int k,
-                                          const int (&b)[7], const Gather<K>& g, float a_s,
-                                          float epsv)
-{
-    rhs_point<K>(a, i, j, k, b[3], g, a_s, epsv,
-                 [&](int s, uint32_t p) { return a.ph[b[s] + (int)p * a.L]; });
 }
 
 // Overflow policy for a point whose neighbourhood holds more than K distinct
@@ -724,300 +417,18 @@ __device__ __forceinline__ void fixup_group(const StepArgs& a, unsigned C, bool 
     }
 }
 
-// One interior point: pass A, then pass B.  Returns 0 if no neighbour holds a
-// grain id (every slot was written as the empty pair), 1 if slots were
-// computed, 2 if the neighbourhood overflows K slots: the point is then left
-// untouched here and the fix-up kernel redoes it under the overflow policy.
-template <int K, bool G27>
-__device__ __forceinline__ int apt_point(const StepArgs& a, int i, int j, int k, float a_s,
-                                         float epsv)
-{
-    const Nbr nb = make_nbr(a, i, j, k);
-    Gather<K> g;
-    gather_init(g);
-    scan_all<K, G27>(a, nb, g);
-    if (g.ovf) return 2;
-    int b[7];
-    stencil_bases(a, nb, b);
-    rhs_point<K>(a, i, j, k, b, g, a_s, epsv);
-    return g.n > 0 ? 1 : 0;
-}
-
-// ---------------------------------------------------------------- tiled ---
-// LDS-tiled z-march.  A workgroup owns a TX x TY tile of interior columns
-// and a chunk of z planes.  The ids and phi of the tile plus a one-point halo
-// (boundary maps applied while loading) live in a 3-plane LDS ring; the next
-// plane is prefetched into registers while the current plane is computed, so
-// HBM latency overlaps the gather arithmetic.
-//
+// Column tiles of the activity map and the work list: 64 x 4 interior points.
 // Planes are skipped with the activity map.  If every tile plane that the
 // stencil of plane k can reach (the 3 x 3 neighbouring tiles at k-1, k, k+1,
 // through the boundary maps) holds only empty pairs in the source, every
 // point of plane k gathers no id and its result is K empty pairs; if the
 // destination tile plane is also all empty, writing them changes nothing.
-// Such planes are neither loaded nor written, and a source plane known to be
-// all empty is staged as empty pairs without reading memory.  The results are
-// the same bits as processing everything.
-constexpr int kTX = 64, kTY = 4, kHX = kTX + 2, kHY = kTY + 2, kNPT = kHX * kHY;
+// Such planes are neither read nor written.  The results are the same bits as
+// processing everything.
+constexpr int kTX = 64, kTY = 4;
 
 __device__ __forceinline__ int act_tile_x(int i) { return (i - 1) / kTX; }
 __device__ __forceinline__ int act_tile_y(int j) { return (j - 1) / kTY; }
-
-template <int K>
-struct PlaneLoader {
-    static constexpr int NE = K * kNPT;                   // slots per staged plane
-    static constexpr int PER = (NE + kBlock - 1) / kBlock;
-    int off[PER];                                         // global offset minus the plane term
-    int vid[PER];
-    float vph[PER];
-    bool live;                                            // staged plane holds non-empty slots
-};
-
-// Staging offsets of a tile.  A partial tile (at the +x or +y end) clamps the
-// positions past the halo to the halo column/row; only its inactive lanes
-// read those entries.
-template <int K>
-__device__ __forceinline__ void loader_init(PlaneLoader<K>& ld, const StepArgs& a, int i0, int j0)
-{
-#pragma unroll
-    for (int q = 0; q < PlaneLoader<K>::PER; ++q) {
-        const int e = threadIdx.x + q * kBlock;
-        const int s = e / kNPT;
-        const int pt = e - s * kNPT;
-        const int ly = pt / kHX;
-        const int lx = pt - ly * kHX;
-        ld.off[q] = (e < PlaneLoader<K>::NE)
-                        ? bc_map(min(i0 - 1 + lx, a.fnx - 1), a.fnx, a.bcx)
-                              + bc_map(min(j0 - 1 + ly, a.fny - 1), a.fny, a.bcy) * a.fnx + s * a.L
-                        : -1;
-    }
-}
-
-// Elements 0..PER-2 of every lane are always inside the plane; only the last
-// one can fall past NE, and its offset is clamped so the load stays in bounds
-// (the value is then simply not stored).  The loads are issued whatever the
-// plane: `fetch` false (nothing will be staged) and `active` false (all empty
-// pairs in the source, staged as (-1, -1.0f)) read element 0 instead, so the
-// number of vector-memory operations in flight is the same on every path.
-template <int K>
-__device__ __forceinline__ void loader_fetch(PlaneLoader<K>& ld, const StepArgs& a, int plane,
-                                             bool active, bool fetch = true)
-{
-    const bool real = active && fetch;
-    ld.live = active;
-#pragma unroll
-    for (int q = 0; q < PlaneLoader<K>::PER; ++q) {
-        const int o = (!real || (q == PlaneLoader<K>::PER - 1 && ld.off[q] < 0)) ? 0 : ld.off[q] + plane;
-        ld.vid[q] = a.arg[o];
-        ld.vph[q] = a.ph[o];
-    }
-}
-
-template <int K>
-__device__ __forceinline__ void loader_store(const PlaneLoader<K>& ld, int* ids, float* phs)
-{
-#pragma unroll
-    for (int q = 0; q < PlaneLoader<K>::PER; ++q) {
-        if (q < PlaneLoader<K>::PER - 1 || ld.off[q] >= 0) {
-            ids[threadIdx.x + q * kBlock] = ld.live ? ld.vid[q] : -1;
-            phs[threadIdx.x + q * kBlock] = ld.live ? ld.vph[q] : -1.0f;
-        }
-    }
-}
-
-// Stage a plane straight from global memory into an LDS ring slot (no
-// registers in between), for the start of a run when every slot of the ring
-// is free.  Element q * kBlock + threadIdx.x goes to the same LDS word as in
-// loader_store: the LDS address of a global_load_lds is the wave-uniform base
-// plus 4 * lane.  The caller waits for the loads (vmcnt) and then for the
-// other waves (barrier) before reading the slot.
-template <int K>
-__device__ __forceinline__ void loader_direct(const PlaneLoader<K>& ld, const StepArgs& a, int plane,
-                                              bool active, int* ids, float* phs)
-{
-    const int wbase = threadIdx.x & ~63;
-    if (active) {
-#pragma unroll
-        for (int q = 0; q < PlaneLoader<K>::PER; ++q) {
-            if (q < PlaneLoader<K>::PER - 1 || ld.off[q] >= 0) {
-                const int o = ld.off[q] + plane;
-                __builtin_amdgcn_global_load_lds(
-                    (const __attribute__((address_space(1))) void*)(a.arg + o),
-                    (__attribute__((address_space(3))) void*)(ids + q * kBlock + wbase), 4, 0, 0);
-                __builtin_amdgcn_global_load_lds(
-                    (const __attribute__((address_space(1))) void*)(a.ph + o),
-                    (__attribute__((address_space(3))) void*)(phs + q * kBlock + wbase), 4, 0, 0);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < PlaneLoader<K>::PER; ++q) {
-            if (q < PlaneLoader<K>::PER - 1 || ld.off[q] >= 0) {
-                ids[threadIdx.x + q * kBlock] = -1;
-                phs[threadIdx.x + q * kBlock] = -1.0f;
-            }
-        }
-    }
-}
-
-// Pass A from LDS for one neighbour point (same probe as scan_point), in two
-// parts: the K id reads, then the probes.  Reads issued ahead of the probes
-// keep the LDS latency off the probe chain (a read inside the probe loop sits
-// behind the previous probe's branches and waits once per slot).
-// NPT: points per slot in the LDS layout (slot stride); HX (below): row stride.
-template <int K, int NPT = kNPT>
-__device__ __forceinline__ void lds_ids(const int* __restrict__ plane, int pt, int (&ids)[K])
-{
-#pragma unroll
-    for (int p = 0; p < K; ++p) ids[p] = plane[p * NPT + pt];
-}
-
-template <int K, int S>
-__device__ __forceinline__ void probe_ids(const int (&ids)[K], Gather<K>& g)
-{
-#pragma unroll
-    for (int p = 0; p < K; ++p) {
-        const int id = ids[p];
-        if (id == -1) continue;
-        int pos = g.n;
-#pragma unroll
-        for (int q = 0; q < K; ++q) pos = (g.la[q] == id) ? q : pos;
-        if (pos >= K) {
-            g.ovf = true;
-            continue;
-        }
-        if (pos == g.n) {  // a new id takes the next free slot
-#pragma unroll
-            for (int q = 0; q < K; ++q) g.la[q] = (q == pos) ? id : g.la[q];
-            ++g.n;
-        }
-        if (S >= 0) {
-            const uint32_t sh = 4u * (uint32_t)pos;
-            g.pm[S] = (g.pm[S] & ~(15u << sh)) | ((uint32_t)p << sh);
-        }
-    }
-}
-
-template <int K, int S, int NPT = kNPT>
-__device__ __forceinline__ void scan_lds(const int* __restrict__ plane, int pt, Gather<K>& g)
-{
-    int ids[K];
-    lds_ids<K, NPT>(plane, pt, ids);
-    probe_ids<K, S>(ids, g);
-    __builtin_amdgcn_sched_barrier(0);
-}
-
-// Rolled runs of z-major positions [from, to) of one plane (ids only).
-template <int K, int NPT = kNPT, int HX = kHX>
-__device__ __forceinline__ void scan_lds_run(const int* pl, int pt, int from, int to, Gather<K>& g)
-{
-#pragma unroll 1
-    for (int q = from; q < to; ++q)
-        scan_lds<K, -1, NPT>(pl, pt + ((q / 3) % 3 - 1) * HX + (q % 3 - 1), g);
-}
-
-template <int K, bool G27, int NPT = kNPT, int HX = kHX>
-__device__ __forceinline__ void scan_all_lds(const int* pD, const int* pC, const int* pU, int pt,
-                                             Gather<K>& g)
-{
-    if (!G27) {
-        // two id buffers: the next neighbour's reads are in flight while the
-        // current one is probed
-        int b0[K], b1[K];
-        lds_ids<K, NPT>(pD, pt, b0);
-        lds_ids<K, NPT>(pC, pt - HX, b1);
-        __builtin_amdgcn_sched_barrier(0);
-        probe_ids<K, 0>(b0, g);
-        lds_ids<K, NPT>(pC, pt - 1, b0);
-        __builtin_amdgcn_sched_barrier(0);
-        probe_ids<K, 1>(b1, g);
-        lds_ids<K, NPT>(pC, pt, b1);
-        __builtin_amdgcn_sched_barrier(0);
-        probe_ids<K, 2>(b0, g);
-        lds_ids<K, NPT>(pC, pt + 1, b0);
-        __builtin_amdgcn_sched_barrier(0);
-        probe_ids<K, 3>(b1, g);
-        lds_ids<K, NPT>(pC, pt + HX, b1);
-        __builtin_amdgcn_sched_barrier(0);
-        probe_ids<K, 4>(b0, g);
-        lds_ids<K, NPT>(pU, pt, b0);
-        __builtin_amdgcn_sched_barrier(0);
-        probe_ids<K, 5>(b1, g);
-        probe_ids<K, 6>(b0, g);
-        __builtin_amdgcn_sched_barrier(0);
-    } else {
-        // z-major 27-point order as in scan_all; non-stencil positions rolled,
-        // each run within one plane (a run-time pick among the plane pointers
-        // compiles to an indexed load from a private copy of them)
-        scan_lds_run<K, NPT, HX>(pD, pt, 0, 4, g);
-        scan_lds<K, 0, NPT>(pD, pt, g);
-        scan_lds_run<K, NPT, HX>(pD, pt, 5, 9, g);
-        scan_lds_run<K, NPT, HX>(pC, pt, 9, 10, g);
-        scan_lds<K, 1, NPT>(pC, pt - HX, g);
-        scan_lds_run<K, NPT, HX>(pC, pt, 11, 12, g);
-        scan_lds<K, 2, NPT>(pC, pt - 1, g);
-        scan_lds<K, 3, NPT>(pC, pt, g);
-        scan_lds<K, 4, NPT>(pC, pt + 1, g);
-        scan_lds_run<K, NPT, HX>(pC, pt, 15, 16, g);
-        scan_lds<K, 5, NPT>(pC, pt + HX, g);
-        scan_lds_run<K, NPT, HX>(pC, pt, 17, 18, g);
-        scan_lds_run<K, NPT, HX>(pU, pt, 18, 22, g);
-        scan_lds<K, 6, NPT>(pU, pt, g);
-        scan_lds_run<K, NPT, HX>(pU, pt, 23, 27, g);
-    }
-}
-
-// Overflow policy (above) for a 7-point point inside the tile, from the LDS
-// ring, given the normal gather g of the point (g.n == K, g.ovf set): its slot
-// list holds the first K distinct ids in first-appearance order.  If every
-// entry outside that list has a smaller phi than the smallest of the list
-// ids' largest phi, every other id ranks below all K list ids, so the list is
-// the kept set, in the policy's (first-appearance) order, and g stands as it
-// is.  A list id's largest phi is taken over the entries its row nibbles name;
-// an entry a nibble does not name (another id, or a second entry of a list id
-// in one row) counts as outside, which can only make the test fail, never pass
-// wrongly.  Returns false when the test fails: the fix-up kernel then applies
-// the policy in full.  (At the 256x256x512 start-up, 83-96 % of the overflowed
-// points pass.)
-template <int K, int NPT = kNPT, int HX = kHX>
-__device__ __forceinline__ bool overflow_keeps_list(const int* iD, const int* iC, const int* iU,
-                                                    const float* fD, const float* fC,
-                                                    const float* fU, int pt, const Gather<K>& g)
-{
-    auto off = [&](int s) {
-        return s == 1 ? pt - HX : s == 2 ? pt - 1 : s == 4 ? pt + 1 : s == 5 ? pt + HX : pt;
-    };
-    float best[K];
-#pragma unroll
-    for (int q = 0; q < K; ++q) best[q] = -__builtin_huge_valf();
-    float outside = -__builtin_huge_valf();
-#pragma unroll
-    for (int s = 0; s < 7; ++s) {
-        const int* ib = s == 0 ? iD : (s == 6 ? iU : iC);
-        const float* fb = s == 0 ? fD : (s == 6 ? fU : fC);
-        const int o = off(s);
-        uint32_t named = 0u;  // neighbour slots a nibble of this row names
-#pragma unroll
-        for (int q = 0; q < K; ++q) {
-            const uint32_t p = (g.pm[s] >> (4 * q)) & 15u;
-            if (p == 15u) continue;
-            named |= 1u << p;
-            const float v = fb[(int)p * NPT + o];
-            best[q] = v > best[q] ? v : best[q];
-        }
-#pragma unroll
-        for (int p = 0; p < K; ++p) {
-            if ((named >> p) & 1u) continue;
-            if (ib[p * NPT + o] == -1) continue;
-            const float v = fb[p * NPT + o];
-            outside = v > outside ? v : outside;
-        }
-    }
-    float low = __builtin_huge_valf();
-#pragma unroll
-    for (int q = 0; q < K; ++q) low = best[q] < low ? best[q] : low;
-    return outside < low;
-}
 
 // Append the overflowed lanes of a wave to the fix-up list (one atomic per wave).
 __device__ __forceinline__ void fixup_append(const StepArgs& a, int ovf, unsigned point)
@@ -1032,110 +443,6 @@ __device__ __forceinline__ void fixup_append(const StepArgs& a, int ovf, unsigne
     if (ovf) a.fix_list[base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = point;
 }
 
-// One z plane of a tile.  On entry the ring holds planes k-1, k, k+1.
-// Order of the vector-memory work: gather from LDS, then the point's own
-// reads (orientation rows, paraboloid field), then the prefetch of plane k+2
-// (when plane k+1 is processed next), then the slot arithmetic, then one
-// straight-line block of 2K stores, then plane k+2 is staged into the ring
-// slot plane k-1 leaves free.  Vector-memory operations retire in issue
-// order, so the arithmetic only waits for the point's reads, never for the
-// prefetch, and staging only for the prefetch, never for the stores; every
-// path into an iteration has the same operations in flight.
-// REC: with the keep test (the step kernel variant used while neighbourhoods
-// overflow).
-template <int K, bool G27, bool REC = true>
-__device__ __forceinline__ void tile_plane(const StepArgs& a, PlaneLoader<K>& ld, int (*rid)[K * kNPT],
-                                           float (*rph)[K * kNPT], const float* zs, int i, int j,
-                                           int k, int k0, int tile, int pt, bool lane_on, float xi,
-                                           float yj, float a_s, float epsv, bool stage_next,
-                                           bool act_next2, unsigned& nres)
-{
-    const int A = a.fnx * a.fny;
-    __syncthreads();
-    const int sD = (k + 2) % 3, sC = k % 3, sU = (k + 1) % 3;
-    Gather<K> g;
-    gather_init(g);
-    scan_all_lds<K, G27>(rid[sD], rid[sC], rid[sU], pt, g);
-    if (!lane_on) {  // lane past the end of a partial tile: nothing to compute or store
-        g.n = 0;
-        g.ovf = false;
-    }
-    // 7-point overflow settled here from the ring when the gather's list is
-    // the kept set (the wave skips this when no lane overflowed); the rest go
-    // to the fix-up kernel.  nres counts the wave's settled points for the
-    // overflow diagnostic.
-    if (!G27 && REC) {
-        const bool was = g.ovf;
-        if (__ballot(was) != 0ull) {
-            if (was && overflow_keeps_list<K>(rid[sD], rid[sC], rid[sU], rph[sD], rph[sC], rph[sU], pt, g))
-                g.ovf = false;
-            nres += (unsigned)__popcll(__ballot(was && !g.ovf));
-        }
-    }
-    const int ovf = g.ovf ? 1 : 0;
-    const int C = i + j * a.fnx + k * A;
-    const float* pD = rph[sD];
-    const float* pC = rph[sC];
-    const float* pU = rph[sU];
-    auto phi_at = [&](int s, uint32_t p) {
-        const int o = (int)p * kNPT;
-        switch (s) {
-        case 0: return pD[o + pt];
-        case 1: return pC[o + pt - kHX];
-        case 2: return pC[o + pt - 1];
-        case 3: return pC[o + pt];
-        case 4: return pC[o + pt + 1];
-        case 5: return pC[o + pt + kHX];
-        default: return pU[o + pt];
-        }
-    };
-    SlotPrep<K> sp;
-    if (ovf) g.n = 0;  // an overflowed point computes nothing here (fix-up kernel)
-    slot_prep<K>(a, g, xi, yj, zs[k - k0], phi_at, sp);
-    loader_fetch(ld, a, bc_map(k + 2, a.fnz, a.bcz) * A, act_next2, stage_next);
-    int oid[K];
-    float oph[K];
-    bool wr;
-    slot_finish<K>(a, g, sp, a_s, epsv, phi_at, oid, oph, wr);
-    // Overflowed points are written by the fix-up kernel; skipped slots keep the
-    // destination's old value.  Both send their stores to the per-lane sink.
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        const bool w = lane_on && !ovf && (wr || q >= g.n);
-        int* pa = w ? a.arg_new + C + q * a.L : a.sink_i + lane;
-        float* pp = w ? a.ph_new + C + q * a.L : a.sink_f + lane;
-        *pa = oid[q];
-        *pp = oph[q];
-    }
-    // A point that gathered an id may leave non-empty slots (an overflowed one
-    // will, through the fix-up): mark the destination tile plane.
-    if (ovf || g.n > 0) a.act_dst[k * a.ntiles + tile] = a.ep_new;
-    // Overflowed lanes are redone after the step by the fix-up.
-    fixup_append(a, ovf, (unsigned)C);
-    if (stage_next) {
-        __syncthreads();
-        loader_store(ld, rid[sD], rph[sD]);
-    }
-}
-
-// The LDS ring of a step workgroup: 3 planes of a 66x6 tile region (tile plus
-// halo), every slot's id and phi.  One allocation per K, shared by the tile
-// march and the edge strip (edge_tile), which never run at the same time in a
-// workgroup.
-template <int K>
-struct LdsRing {
-    int id[3][K * kNPT];
-    float ph[3][K * kNPT];
-};
-
-template <int K>
-__device__ __forceinline__ LdsRing<K>& lds_ring()
-{
-    __shared__ LdsRing<K> r;
-    return r;
-}
-
 // The plan kernels' unit of work: wave gw of a simulation covers z-chunk
 // group cg = gw / (waves per group) and plan_tiles consecutive full tiles.
 // Lane l reads the activity of tile slot l / plan_rows at plane kb - 1 +
@@ -1144,13 +451,12 @@ __device__ __forceinline__ LdsRing<K>& lds_ring()
 // and lane l = c * plan_tiles + slot assembles the masks of chunk c of the
 // group for that tile slot, chunk = [k0, k1): need bit m for plane k0+m to
 // process (some source word of the 3 x 3 tiles around the tile is active at a
-// plane within one of it, through the z map, or its own destination word is),
-// act bit r for the source activity of plane k0-1+r.  Items leave a wave
-// chunk-major, so the list runs through z-chunk groups in order and the items
-// in flight together lie in few planes.  put: the chunk has planes to
+// plane within one of it, through the z map, or its own destination word is).
+// Items leave a wave chunk-major, so the list runs through z-chunk groups in
+// order and the items in flight together lie in few planes.  put: the chunk has planes to
 // process; item = its work-list code.
 __device__ __forceinline__ void plan_wave(const StepArgs& a, int gw, int lane, bool& put, int& item,
-                                          uint64_t& need, uint64_t& act)
+                                          uint64_t& need)
 {
     const int R = plan_rows(a.kchunk);
     const int TW = plan_tiles(a.kchunk);
@@ -1192,18 +498,15 @@ __device__ __forceinline__ void plan_wave(const StepArgs& a, int gw, int lane, b
     put = false;
     item = 0;
     need = 0ull;
-    act = 0ull;
     if (c < C && zc < a.nzchunk && t < a.items_chunk) {
         const int k0 = 1 + zc * a.kchunk;
         const int n = min(k0 + a.kchunk, a.fnz - 1) - k0;
         const uint64_t full = (1ull << n) - 1ull;  // n <= 61
         if (!a.use_act) {
             need = full;
-            act = ~0ull;
         } else {
             const int sh = slot * R + c * a.kchunk;  // lane of plane k0 - 1 for this tile
             const uint64_t ac = (A >> sh) & ((1ull << (n + 2)) - 1ull);
-            act = ac;
             need = ((ac | (ac >> 1) | (ac >> 2)) | ((D >> (sh + 1)) & full)) & full;
         }
         put = need != 0ull;
@@ -1211,45 +514,28 @@ __device__ __forceinline__ void plan_wave(const StepArgs& a, int gw, int lane, b
     }
 }
 
-// List position of this lane's chunk if `put`: a heavy chunk (more than half
-// of its planes to process) from the front of the list, a light one from the
-// back (cap - 1 downward).  Every thread of the workgroup (kPlanWaves waves)
-// calls it; waves take consecutive runs of positions in wave order.
+// List position of this lane's chunk if `put`.  Every thread of the workgroup
+// (kPlanWaves waves) calls it; waves take consecutive runs of positions in
+// wave order, reserved with one atomic per workgroup.
 template <int kPlanWaves>
-__device__ __forceinline__ unsigned plan_slot(bool put, bool heavy, unsigned* front, unsigned* back,
-                                              unsigned cap, unsigned* s_cnt)
+__device__ __forceinline__ unsigned plan_slot(bool put, unsigned* count, unsigned* s_cnt)
 {
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
-    const unsigned long long mh = __ballot(put && heavy);
-    const unsigned long long ml = __ballot(put && !heavy);
-    if (lane == 0) {
-        s_cnt[w] = (unsigned)__popcll(mh);
-        s_cnt[kPlanWaves + 1 + w] = (unsigned)__popcll(ml);
-    }
+    const unsigned long long m = __ballot(put);
+    if (lane == 0) s_cnt[w] = (unsigned)__popcll(m);
     __syncthreads();
     if (threadIdx.x == 0) {
-        unsigned th = 0u, tl = 0u;
+        unsigned t = 0u;
         for (int u = 0; u < kPlanWaves; ++u) {
-            const unsigned ch = s_cnt[u], cl = s_cnt[kPlanWaves + 1 + u];
-            s_cnt[u] = th;
-            s_cnt[kPlanWaves + 1 + u] = tl;
-            th += ch;
-            tl += cl;
+            const unsigned c = s_cnt[u];
+            s_cnt[u] = t;
+            t += c;
         }
-        s_cnt[kPlanWaves] = th ? atomicAdd(front, th) : 0u;
-        s_cnt[2 * kPlanWaves + 1] = tl ? atomicAdd(back, tl) : 0u;
+        s_cnt[kPlanWaves] = t ? atomicAdd(count, t) : 0u;
     }
     __syncthreads();
-    const unsigned long long below = (1ull << lane) - 1ull;
-    if (heavy) return s_cnt[kPlanWaves] + s_cnt[w] + (unsigned)__popcll(mh & below);
-    return cap - 1u - (s_cnt[2 * kPlanWaves + 1] + s_cnt[kPlanWaves + 1 + w] +
-                       (unsigned)__popcll(ml & below));
-}
-
-__device__ __forceinline__ bool plan_heavy(uint64_t need, int kchunk)
-{
-    return 2 * __popcll(need) > kchunk;
+    return s_cnt[kPlanWaves] + s_cnt[w] + (unsigned)__popcll(m & ((1ull << lane) - 1ull));
 }
 
 // One workgroup of a step's plan (apt_plan, and the plan half of
@@ -1258,7 +544,7 @@ __device__ __forceinline__ bool plan_heavy(uint64_t need, int kchunk)
 __device__ __forceinline__ void plan_block(const StepArgs& a, int pb)
 {
     constexpr int kPlanWaves = kBlock / 64;
-    __shared__ unsigned s_cnt[2 * kPlanWaves + 2];
+    __shared__ unsigned s_cnt[kPlanWaves + 1];
     const int g = pb * kBlock + (int)threadIdx.x;
     // the counter set of the step after this one (last used two steps
     // before, whose fix-up has finished) starts from zero
@@ -1267,250 +553,13 @@ __device__ __forceinline__ void plan_block(const StepArgs& a, int pb)
     const int lane = threadIdx.x & 63;
     bool put = false;
     int item = 0;
-    uint64_t need = 0ull, act = 0ull;
-    if (gw < plan_waves(a.kchunk, a.nzchunk, a.items_chunk))
-        plan_wave(a, gw, lane, put, item, need, act);
-    const unsigned q = plan_slot<kPlanWaves>(put, plan_heavy(need, a.kchunk), a.wl_count, a.wl_light,
-                                             (unsigned)(a.nzchunk * a.items_chunk), s_cnt);
+    uint64_t need = 0ull;
+    if (gw < plan_waves(a.kchunk, a.nzchunk, a.items_chunk)) plan_wave(a, gw, lane, put, item, need);
+    const unsigned q = plan_slot<kPlanWaves>(put, a.wl_count, s_cnt);
     if (put) {
         a.wl_item[q] = item;
         a.wl_need[q] = need;
-        a.wl_act[q] = act;
     }
-}
-
-// nres (wave-uniform) accumulates the overflowed points the tile resolved.
-template <int K, bool G27, bool REC = true>
-__device__ __forceinline__ void tile_march(const StepArgs& a, int tx, int ty, int k0, int k1,
-                                           uint64_t need, uint64_t act, float a_s, float epsv,
-                                           unsigned& nres)
-{
-    int (*rid)[K * kNPT] = lds_ring<K>().id;
-    float (*rph)[K * kNPT] = lds_ring<K>().ph;
-    __shared__ float zs[64];  // z of the chunk's planes (a chunk has at most 61)
-    const int i0 = 1 + tx * kTX, j0 = 1 + ty * kTY;
-    const int lx = threadIdx.x & (kTX - 1);
-    const int ly = threadIdx.x / kTX;
-    const int i = i0 + lx, j = j0 + ly;
-    const int pt = (ly + 1) * kHX + (lx + 1);
-    const int A = a.fnx * a.fny;
-    const int tile = tx + ty * a.ntx;
-    auto act_at = [&](int kk) { return kk <= k1 && ((act >> (kk - k0 + 1)) & 1ull) != 0ull; };
-    auto need_at = [&](int kk) { return kk < k1 && ((need >> (kk - k0)) & 1ull) != 0ull; };
-    // coordinates for the thermal field: per lane once, z through LDS (made
-    // visible by the barrier that opens every run)
-    const bool lane_on = i <= a.fnx - 2 && j <= a.fny - 2;
-    const float xi = a.x[min(i, a.fnx - 2)], yj = a.y[min(j, a.fny - 2)];
-    if ((int)threadIdx.x < k1 - k0) zs[threadIdx.x] = a.z[k0 + threadIdx.x];
-    PlaneLoader<K> ld;
-    loader_init(ld, a, i0, j0);
-    int k = k0;
-    while (k < k1) {
-        if (!need_at(k)) {
-            ++k;
-            continue;
-        }
-        // start of a run of processed planes: k-1, k, k+1 into the ring once
-        // every wave is done with the ring
-        __syncthreads();
-        loader_direct(ld, a, bc_map(k - 1, a.fnz, a.bcz) * A, act_at(k - 1), rid[(k + 2) % 3],
-                      rph[(k + 2) % 3]);
-        loader_direct(ld, a, k * A, act_at(k), rid[k % 3], rph[k % 3]);
-        loader_direct(ld, a, bc_map(k + 1, a.fnz, a.bcz) * A, act_at(k + 1), rid[(k + 1) % 3],
-                      rph[(k + 1) % 3]);
-        __builtin_amdgcn_s_waitcnt(0);  // the three planes are in LDS (barrier in tile_plane)
-        do {
-            tile_plane<K, G27, REC>(a, ld, rid, rph, zs, i, j, k, k0, tile, pt, lane_on, xi, yj, a_s,
-                               epsv, need_at(k + 1), act_at(k + 2), nres);
-            ++k;
-        } while (need_at(k));
-    }
-}
-
-// A narrow strip of columns left at the +x end (fewer than kPartialMin; wider
-// leftovers, and every leftover in y, are partial LDS tiles) takes the direct
-// path, one point per lane: point p of z chunk [k0, k1) is strip column
-// p % edge_cols (row-major over the strip) at plane k0 + p / edge_cols.  A
-// point is skipped under the same rule as a tile plane: all of its stencil's
-// tile planes empty in the source and its own tile plane empty in the
-// destination.
-// Whether interior point (i, j, k) of the +x strip must be processed: some
-// tile plane of its 3x3x3 tile neighbourhood is active in the source, or its
-// own tile plane is in the destination (the tile plane rule of the activity
-// map, per point).
-__device__ __forceinline__ bool edge_need(const StepArgs& a, int i, int j, int k, int tile)
-{
-    if (!a.use_act) return true;
-    const int xl = act_tile_x(bc_map(i - 1, a.fnx, a.bcx)), xc = act_tile_x(i);
-    const int xr = act_tile_x(bc_map(i + 1, a.fnx, a.bcx));
-    const int rl = act_tile_y(bc_map(j - 1, a.fny, a.bcy)) * a.ntx, rc = act_tile_y(j) * a.ntx;
-    const int rr = act_tile_y(bc_map(j + 1, a.fny, a.bcy)) * a.ntx;
-    const unsigned e = a.ep_src;
-    // bitwise ors: all 28 reads go out together (a short-circuit chain
-    // would issue them one memory latency apart)
-    bool any = a.act_dst[k * a.ntiles + tile] >= a.ep_dst;
-#pragma unroll
-    for (int dz = -1; dz <= 1; ++dz) {
-        const unsigned* w = a.act_src + bc_map(k + dz, a.fnz, a.bcz) * a.ntiles;
-        any = any | (w[xl + rl] >= e) | (w[xc + rl] >= e) | (w[xr + rl] >= e) |
-              (w[xl + rc] >= e) | (w[xc + rc] >= e) | (w[xr + rc] >= e) |
-              (w[xl + rr] >= e) | (w[xc + rr] >= e) | (w[xr + rr] >= e);
-    }
-    return any;
-}
-
-template <int K, bool G27>
-__device__ __forceinline__ void edge_point(const StepArgs& a, int p, int k0, int k1, float a_s,
-                                           float epsv)
-{
-    const int r = p / a.edge_cols;
-    const int c = p - r * a.edge_cols;
-    const int k = k0 + r;
-    const int ex = (a.fnx - 2) - a.tiles_x * kTX;  // strip width, > 0 whenever edge items exist
-    const int j = 1 + c / ex;
-    const int i = 1 + a.tiles_x * kTX + (c - (j - 1) * ex);
-    const bool live = k < k1;
-    const int tile = act_tile_x(i) + act_tile_y(j) * a.ntx;
-    const bool need = live && edge_need(a, i, j, k, tile);
-    int res = 0;
-    if (need) {
-        res = apt_point<K, G27>(a, i, j, k, a_s, epsv);
-        if (res != 0) a.act_dst[k * a.ntiles + tile] = a.ep_new;
-    }
-    fixup_append(a, res == 2, (unsigned)(i + j * a.fnx + k * a.fnx * a.fny));
-}
-
-// The strip is one column wide (the reference sizes its grids as 64 m + 1
-// points, e.g. 257 = 4 x 64 + 1): it runs as edge tiles (7-point gather).
-__device__ __forceinline__ bool edge_strip_is_column(const StepArgs& a)
-{
-    return a.edge_cols == a.fny - 2;
-}
-
-// One edge tile: rows 1 + 64 seg .. 64 seg + 64 of the one-column strip
-// i = fnx - 2 over planes [k0, k1).  Lanes are (row, plane), 4 planes per
-// pass.  A pass stages the columns i-1, i, i+1 of its 66 rows (halo included)
-// and 6 planes, every slot's id and phi, straight from global memory into
-// the step's LDS ring with global_load_lds (K x 1188 points, exactly the
-// ring's size), then each lane runs the tile lane's gather, keep test,
-// and slot arithmetic with row stride 3 and plane stride 198.  A
-// lane processes its point under edge_point's activity rule (the others
-// neither store nor mark nor hand over), and a pass none of whose lanes
-// does stages nothing.  Against the direct path (neighbours through L1/L2,
-// one dependent round trip per neighbour) the staging is one round trip per
-// pass, and overflowed points get the keep test (the direct path hands every
-// one to the fix-up).  Used by the batched step
-// and by the single step's edge kernel of overflow steps (apt_edge).  Returns
-// the overflowed points the keep test settled.  REC false: no keep test
-// (every overflowed point goes to the fix-up).
-template <int K, bool REC = true>
-__device__ __forceinline__ unsigned edge_tile(const StepArgs& a, int seg, int k0, int k1,
-                                              float a_s, float epsv)
-{
-    unsigned nres = 0u;
-    constexpr int EW = 3, EH = kEdgeRows + 2, EPL = EW * EH, ENPT = EPL * 6;
-    static_assert(ENPT == 3 * kNPT, "an edge tile fills the step's LDS ring exactly");
-    constexpr int NE = K * ENPT;  // staged entries per pass
-    constexpr int PER = (NE + kBlock - 1) / kBlock;
-    int* eid = &lds_ring<K>().id[0][0];
-    float* eph = &lds_ring<K>().ph[0][0];
-    const int A = a.fnx * a.fny;
-    const int i = a.fnx - 2;  // the strip column
-    const int lane = threadIdx.x & 63;
-    const int ly = (int)threadIdx.x % kEdgeRows, lz = (int)threadIdx.x / kEdgeRows;
-    const int j = 1 + seg * kEdgeRows + ly;
-    const bool row_on = j <= a.fny - 2;
-    const int jc = min(j, a.fny - 2);
-    const float xi = a.x[i], yj = a.y[jc];
-    const int tile = act_tile_x(i) + act_tile_y(jc) * a.ntx;
-    const int pt = lz * EPL + (ly + 1) * EW + 1;  // in plane lz + 1 through iC / fC
-    const int* iD = eid;
-    const int* iC = eid + EPL;
-    const int* iU = eid + 2 * EPL;
-    const float* fD = eph;
-    const float* fC = eph + EPL;
-    const float* fU = eph + 2 * EPL;
-    const int wbase = threadIdx.x & ~63;
-#pragma unroll 1
-    for (int kb = k0; kb < k1; kb += kBlock / kEdgeRows) {
-        const int k = kb + lz;
-        const int kc = min(k, a.fnz - 2);
-        const bool need = row_on && k < k1 && edge_need(a, i, jc, kc, tile);
-        // the barrier also orders the previous pass's LDS reads before this
-        // pass's staging
-        if (!__syncthreads_or(need ? 1 : 0)) continue;
-#pragma unroll 1
-        for (int q = 0; q < PER; ++q) {
-            const int e = q * kBlock + (int)threadIdx.x;
-            if (e < NE) {
-                const int p = e / ENPT;
-                const int r = e - p * ENPT;
-                const int z = r / EPL;
-                const int r2 = r - z * EPL;
-                const int y = r2 / EW;
-                const int x = r2 - y * EW;
-                const int gx = bc_map(i - 1 + x, a.fnx, a.bcx);
-                const int gy = bc_map(min(seg * kEdgeRows + y, a.fny - 1), a.fny, a.bcy);
-                const int gz = bc_map(min(kb - 1 + z, a.fnz - 1), a.fnz, a.bcz);
-                const int o = gx + gy * a.fnx + gz * A + p * a.L;
-                __builtin_amdgcn_global_load_lds(
-                    (const __attribute__((address_space(1))) void*)(a.arg + o),
-                    (__attribute__((address_space(3))) void*)(eid + q * kBlock + wbase), 4, 0, 0);
-                __builtin_amdgcn_global_load_lds(
-                    (const __attribute__((address_space(1))) void*)(a.ph + o),
-                    (__attribute__((address_space(3))) void*)(eph + q * kBlock + wbase), 4, 0, 0);
-            }
-        }
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        Gather<K> g;
-        gather_init(g);
-        scan_all_lds<K, false, ENPT, EW>(iD, iC, iU, pt, g);
-        if (!need) {
-            g.n = 0;
-            g.ovf = false;
-        }
-        if (REC) {  // the keep test of tile_plane
-            const bool was = g.ovf;
-            if (__ballot(was) != 0ull) {
-                if (was && overflow_keeps_list<K, ENPT, EW>(iD, iC, iU, fD, fC, fU, pt, g))
-                    g.ovf = false;
-                nres += (unsigned)__popcll(__ballot(was && !g.ovf));
-            }
-        }
-        const int ovf = g.ovf ? 1 : 0;
-        const int C = i + jc * a.fnx + kc * A;
-        auto phi_at = [&](int s, uint32_t p) {
-            const int o = (int)p * ENPT;
-            switch (s) {
-            case 0: return fD[o + pt];
-            case 1: return fC[o + pt - EW];
-            case 2: return fC[o + pt - 1];
-            case 3: return fC[o + pt];
-            case 4: return fC[o + pt + 1];
-            case 5: return fC[o + pt + EW];
-            default: return fU[o + pt];
-            }
-        };
-        SlotPrep<K> sp;
-        if (ovf) g.n = 0;
-        slot_prep<K>(a, g, xi, yj, a.z[kc], phi_at, sp);
-        int oid[K];
-        float oph[K];
-        bool wr;
-        slot_finish<K>(a, g, sp, a_s, epsv, phi_at, oid, oph, wr);
-#pragma unroll
-        for (int q = 0; q < K; ++q) {
-            const bool w = need && !ovf && (wr || q >= g.n);
-            int* pa = w ? a.arg_new + C + q * a.L : a.sink_i + lane;
-            float* pp = w ? a.ph_new + C + q * a.L : a.sink_f + lane;
-            *pa = oid[q];
-            *pp = oph[q];
-        }
-        if (need && (ovf || g.n > 0)) a.act_dst[kc * a.ntiles + tile] = a.ep_new;
-        fixup_append(a, ovf, (unsigned)C);
-    }
-    return nres;
 }
 
 __host__ __device__ inline int cdiv(long long a, long long b) { return (int)((a + b - 1) / b); }

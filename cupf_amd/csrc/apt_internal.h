@@ -20,15 +20,9 @@ constexpr double kKill = -0.9999;
 constexpr float kLSf = -0.995f;
 constexpr float kKillf = -0.9999f;
 
-// Fix-up list length from which a step counts as overflowing for the host's
-// choice of step kernel variant: below it the plain variant's fix-up (every
-// overflowed point, gathered again through L1/L2) costs less than the
-// overflow variant's keep test and edge kernel.
-constexpr unsigned kOvfHeavy = 32768u;
-
-// Leftover columns at the +x end narrower than this take the direct path;
-// wider ones form a partial LDS tile (its idle lanes cost less than the direct
-// path's per-point neighbour loads).
+// Leftover columns at the +x end narrower than this form a strip, whose rows
+// share waves (64 / width rows each); wider ones form a partial tile, one row
+// per wave.
 constexpr int kPartialMin = 16;
 
 // Everything one APT step launch reads.  Passed by value (kernel argument
@@ -52,8 +46,6 @@ struct StepArgs {
     // run beside the next step's plan, keeps its own).
     unsigned* fix_count;
     unsigned* cnt_next;
-    int* sink_i;           // 64-lane write sinks for lanes that must not store
-    float* sink_f;
     // Activity map: one word per (column tile, z plane) and buffer.  A tile
     // plane of a buffer may hold a slot other than the empty pair (-1, -1.0f)
     // only if its word is >= that buffer's epoch.  Epochs come from one
@@ -65,32 +57,26 @@ struct StepArgs {
     unsigned ep_new;       // epoch the destination buffer gets from this step
     int use_act;           // 0: process every plane (the map is still maintained)
     int ntx, nty, ntiles;  // activity tiles (64x4, partial ones included)
-    // Work of one step: nzchunk * edge_items edge items (the leftover columns:
-    // kEdgePoints points or one edge tile each; the first work indices, or a
-    // kernel of their own in a single overflow step), and the tile chunks
-    // listed by the plan kernel:
-    // wl_item = z chunk * items_chunk + full tile, with the chunk's plane masks.
-    // Chunks with more than half their planes to process are listed from the
-    // front (wl_count[0] of them), the others from the back of the list
-    // (wl_light[0] of them, down from nzchunk * items_chunk - 1), so the long
-    // items are taken first and the short ones fill the end.  wl_count[1] is
-    // the next work index to take (words 2 and 3 of this step's counter set).
+    // Row map: one word per (row of a column tile, z plane) and buffer, epoch
+    // << 4 | bound.  A row of a buffer may hold anything but empty pairs only
+    // if its word's epoch is >= the buffer's, and then only in slots below
+    // the bound.  Index (k * fny + j) * ntx + column tile.
+    const unsigned* row_src;
+    unsigned* row_dst;
+    // Work of one step: the strip's units (see apt_step), then the tile chunks
+    // listed by the plan kernel: wl_item = z chunk * items_chunk + tile, with
+    // the chunk's plane mask, wl_count[0] of them (word 2 of the counter set).
     int* wl_item;
     unsigned long long* wl_need;
-    unsigned long long* wl_act;
     unsigned* wl_count;
-    unsigned* wl_light;    // chunks listed from the end of the list (word 1 of the counter set)
-    int items_chunk;       // full tiles per z chunk
-    int edge_cols;         // interior columns outside the full tiles
-    int edge_items;        // edge items per z chunk (edge_items_per_chunk)
-    int step_blocks;       // persistent workgroups of the step kernel
-    int fix_blocks;        // workgroups (one wave each) of the overflow fix-up kernel
+    int items_chunk;       // tiles per z chunk
+    int step_blocks;       // one-wave workgroups of the step kernel
+    int fix_blocks;        // workgroups of the overflow fix-up kernel
     int fnx, fny, fnz;
     int L;                 // slot stride fnx*fny*fnz
-    int ncolx, ncols;      // interior columns: (fnx-2), (fnx-2)*(fny-2)
     int nzchunk, kchunk;   // z-chunks per column, planes per chunk
-    int tiles_x, tiles_y;  // 64x4 column tiles of the LDS path (partial ones at the +x/+y
-                           // end included; see kPartialMin)
+    int tiles_x, tiles_y;  // 64x4 column tiles (partial ones at the +x/+y end included;
+                           // see kPartialMin)
     int bcx, bcy, bcz;
     int num_theta;
     int thermal_type;
@@ -101,14 +87,6 @@ struct StepArgs {
     float tan_angle, cos_angle;
     int Nx, Ny, Nz;
     float X0_mac, Y0_mac, Z0_mac, Dx_mac;
-    // The host's step kernel variant (not read by the kernels): nonzero for
-    // the one with keep test and edge kernel, used while
-    // neighbourhoods overflow.  The fix-up reports for that choice: it writes
-    // launch_index to seen[0] and, when its list holds kOvfHeavy points or
-    // more, to seen[1] (pinned host memory; null: no report).
-    unsigned long long* seen;
-    unsigned long long launch_index;
-    int ovf_variant;
 };
 
 // One simulation of a batch, in device memory.  `a` holds the arguments of
@@ -120,15 +98,16 @@ struct BatchSim {
     float* ph[2];
     int* arg[2];
     unsigned* act[2];
+    unsigned* row[2];
     unsigned ep[2];        // epochs of the two buffers
     unsigned ep_ctr;       // epoch counter of the simulation
     int cur;               // source buffer of the next step
     int step;              // index s of the next step (t = (float)s*dt*tau0)
     int parity;            // counter set of the next step (0..2, in turn)
-    unsigned* cnt;         // the simulation's two 4-word counter sets
+    unsigned* cnt;         // the simulation's three 4-word counter sets
     float tau0;
     int plan_base;         // first plan wave of this simulation
-    int edge_base;         // first edge work index of this simulation
+    int strip_base;        // first strip unit of this simulation
 };
 
 // Plan waves: a wave's 64 lanes cover plan_tiles tiles, plan_rows lanes (z
@@ -144,23 +123,12 @@ __host__ __device__ inline int plan_waves(int kchunk, int nzchunk, int items_chu
     return ((nzchunk + g - 1) / g) * ((items_chunk + tw - 1) / tw);
 }
 
-// Points of one edge item: kEdgePerLane per lane of a 256-lane workgroup
-// (4 per lane was measured 8 % slower on the 256x256x512 step: edge items are
-// taken first, and fewer, longer ones hold workgroups the tile items need).
-constexpr int kEdgePerLane = 1;
-constexpr int kEdgePoints = 256 * kEdgePerLane;
-// Rows of one edge tile (a one-column strip, 7-point gather): 64 rows x 4
-// planes per pass of a 256-lane workgroup.
-constexpr int kEdgeRows = 64;
-
-// Edge items per z chunk for a strip of edge_cols = width x (fny - 2) points:
-// kEdgePoints points each, or (tiles: batched or overflow steps, 7-point
-// gather, one-column strip) edge tiles of kEdgeRows rows.
-inline int edge_items_per_chunk(int edge_cols, int fny, int kchunk, bool gather27, bool tiles)
+// Waves of the +x strip per z chunk: ex columns of fny - 2 rows (ex <= 0: no
+// strip), 64 / ex rows to a wave.
+__host__ __device__ inline int strip_width(int fnx, int tiles_x) { return (fnx - 2) - 64 * tiles_x; }
+__host__ __device__ inline int strip_waves(int ex, int fny)
 {
-    if (edge_cols == 0) return 0;
-    if (tiles && !gather27 && edge_cols == fny - 2) return (fny - 2 + kEdgeRows - 1) / kEdgeRows;
-    return (int)(((long long)kchunk * edge_cols + kEdgePoints - 1) / kEdgePoints);
+    return ex > 0 ? (fny - 2 + 64 / ex - 1) / (64 / ex) : 0;
 }
 
 // Most simulations one batch may hold.
@@ -168,29 +136,19 @@ constexpr int kMaxBatch = 1024;
 
 // A batched step over n simulations sharing K and the gather variant.  The
 // work list holds tile chunks of every simulation; cnt holds two 4-word
-// counter sets ([0] chunks listed from the front, [1] next work index, [2]
-// chunks listed from the back) used by alternate steps, selected by cnt[8];
-// cnt[9] counts the batched fix-up's launches.
+// counter sets ([0] chunks listed) used by alternate steps, selected by
+// cnt[8].
 struct BatchArgs {
     BatchSim* sims;
     int n;
     int plan_total;        // waves of the plan kernel (all simulations)
-    int edge_total;        // edge work items of all simulations
+    int strip_total;       // strip units of all simulations
     int* wl_sim;
     int* wl_item;
     unsigned long long* wl_need;
-    unsigned long long* wl_act;
     unsigned* cnt;
-    int wl_cap;            // list capacity: light chunks are listed down from wl_cap - 1
     int step_blocks;
-    int fix_blocks;        // workgroups (one wave each) of the batched fix-up kernel
-    // The host's batch_step variant: nonzero for the one with the keep test
-    // (7-point gather).  The batched fix-up reports for that
-    // choice (pinned host memory; null: no report): it counts its launches in
-    // cnt[9] and writes the count to seen[0] and, when the lists of all
-    // members hold kOvfHeavy points or more, to seen[1].
-    unsigned long long* seen;
-    int ovf_variant;
+    int fix_blocks;        // workgroups of the batched fix-up kernel
 };
 
 // Nucleation launch block (3DgrainMPI/APTPhaseField.cu:459-536).
@@ -204,7 +162,8 @@ struct NuclArgs {
     const float* T3d;
     const float* ball;     // (2p+1)^3 tanh template
     unsigned long long* events;
-    unsigned* act;         // activity map of the buffer nucleated into, and its epoch
+    unsigned* act;         // activity and row maps of the buffer nucleated into, and its epoch
+    unsigned* row;
     unsigned ep;
     int ntx, ntiles;
     int fnx, fny, fnz, L, K;
@@ -227,34 +186,26 @@ int batch_kernel_slots(int K, int gather27, int device);
 int fixup_kernel_slots(int K, int gather27, int device, bool batch);
 // Batched step: plan, persistent step, fix-up and advance kernels.
 hipError_t launch_batch_step(const BatchArgs& b, int K, int gather27, hipStream_t stream);
-// The second stream of an overflow step's edge kernel and the events that
-// order it: `ready` (recorded on the step's stream after the plan kernel),
-// `done` (on the edge stream after the edge kernel; the fix-up waits for it).
-struct EdgeLaunch {
-    hipStream_t stream;
-    hipEvent_t ready, done;
-};
-
 // Pieces shared by the per-K launchers.
 hipError_t launch_plan(const StepArgs& a, hipStream_t stream);
 hipError_t launch_batch_plan(const BatchArgs& b, hipStream_t stream);
 hipError_t launch_batch_advance(const BatchArgs& b, hipStream_t stream);
-hipError_t launch_step_k5_g7(const StepArgs& a, hipStream_t stream, const EdgeLaunch* edge,
+hipError_t launch_step_k5_g7(const StepArgs& a, hipStream_t stream,
                              hipEvent_t e0, hipEvent_t e1, hipEvent_t e2, hipEvent_t e3,
                              bool planned, const StepArgs* next);
 hipError_t launch_batch_k5_g7(const BatchArgs& b, hipStream_t stream);
 int step_slots_k5_g7(int device, int which);
-hipError_t launch_step_k5_g27(const StepArgs& a, hipStream_t stream, const EdgeLaunch* edge,
+hipError_t launch_step_k5_g27(const StepArgs& a, hipStream_t stream,
                              hipEvent_t e0, hipEvent_t e1, hipEvent_t e2, hipEvent_t e3,
                              bool planned, const StepArgs* next);
 hipError_t launch_batch_k5_g27(const BatchArgs& b, hipStream_t stream);
 int step_slots_k5_g27(int device, int which);
-hipError_t launch_step_k8_g7(const StepArgs& a, hipStream_t stream, const EdgeLaunch* edge,
+hipError_t launch_step_k8_g7(const StepArgs& a, hipStream_t stream,
                              hipEvent_t e0, hipEvent_t e1, hipEvent_t e2, hipEvent_t e3,
                              bool planned, const StepArgs* next);
 hipError_t launch_batch_k8_g7(const BatchArgs& b, hipStream_t stream);
 int step_slots_k8_g7(int device, int which);
-hipError_t launch_step_k8_g27(const StepArgs& a, hipStream_t stream, const EdgeLaunch* edge,
+hipError_t launch_step_k8_g27(const StepArgs& a, hipStream_t stream,
                              hipEvent_t e0, hipEvent_t e1, hipEvent_t e2, hipEvent_t e3,
                              bool planned, const StepArgs* next);
 hipError_t launch_batch_k8_g27(const BatchArgs& b, hipStream_t stream);
@@ -265,7 +216,7 @@ int step_slots_k8_g27(int device, int which);
 // Optional events are recorded before the plan, after it, after the main
 // kernel and after the fix-up.
 hipError_t launch_step(const StepArgs& a, int K, int gather27, hipStream_t stream,
-                       const EdgeLaunch* edge, hipEvent_t ev_begin = nullptr,
+                       hipEvent_t ev_begin = nullptr,
                        hipEvent_t ev_planned = nullptr, hipEvent_t ev_mid = nullptr,
                        hipEvent_t ev_end = nullptr, bool planned = false,
                        const StepArgs* next = nullptr);
@@ -298,9 +249,9 @@ hipError_t launch_move_frame(float* ph_old, int* arg_old, float* ph_new, int* ar
 hipError_t launch_nucl_status(const float* phi0, int* status, int cnx, int cny, int cnz, int p,
                               int fnx, int fny, hipStream_t stream);
 hipError_t launch_nucl(const NuclArgs& a, hipStream_t stream);
-// Activity map of one buffer from its contents: every tile plane holding a
-// non-empty slot gets `ep`.
-hipError_t launch_act_rebuild(const float* ph, const int* arg, unsigned* act, unsigned ep, int fnx,
+// Activity and row maps of one buffer from its contents: every tile plane and
+// row holding a non-empty slot gets `ep` (the row with its bound).
+hipError_t launch_act_rebuild(const float* ph, const int* arg, unsigned* act, unsigned* row, unsigned ep, int fnx,
                               int fny, int fnz, int K, int ntx, int ntiles, hipStream_t stream);
 hipError_t launch_copy(const void* src, void* dst, size_t bytes, hipStream_t stream);
 

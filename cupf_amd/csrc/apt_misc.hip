@@ -12,11 +12,10 @@ namespace {
 // 16 for a batch, whose plan has many more waves.
 constexpr int kBatchPlanBlock = 1024;
 
-// Work list of one step (runs before apt_step_tiled): waves over (z-chunk
-// group, tiles), see plan_wave.  A tile chunk is listed only if some plane of
-// it needs processing, with its plane masks.  Edge items are not listed: the
-// first nzchunk * edge_items work indices are edge items, always taken (their
-// points decide one by one), or the edge kernel's in overflow steps.
+// Work list of one step (runs before apt_step): waves over (z-chunk group,
+// tiles), see plan_wave.  A tile chunk is listed only if some plane of it needs
+// processing, with its plane mask.  The strip's units are not listed: the step
+// takes them all, and their waves decide plane by plane.
 __global__ __launch_bounds__(kBlock) void apt_plan(StepArgs a)
 {
     plan_block(a, (int)blockIdx.x);
@@ -27,7 +26,7 @@ __global__ __launch_bounds__(kBlock) void apt_plan(StepArgs a)
 __global__ __launch_bounds__(kBatchPlanBlock) void batch_plan(BatchArgs b)
 {
     constexpr int kPlanWaves = kBatchPlanBlock / 64;
-    __shared__ unsigned s_cnt[2 * kPlanWaves + 2];
+    __shared__ unsigned s_cnt[kPlanWaves + 1];
     // wave-uniform index and member records read through the constant address
     // space (batch_advance rewrites them only after this kernel): the search
     // and the step-argument fields are scalar loads
@@ -36,9 +35,9 @@ __global__ __launch_bounds__(kBatchPlanBlock) void batch_plan(BatchArgs b)
     const CSim* sims = (const CSim*)b.sims;
     unsigned* cnt = b.cnt + 4 * __atomic_load_n(b.cnt + 8, __ATOMIC_RELAXED);
     const int lane = threadIdx.x & 63;
-    bool put = false, heavy = false;
+    bool put = false;
     int item = 0, sim = 0;
-    uint64_t need = 0ull, act = 0ull;
+    uint64_t need = 0ull;
     if (gw < b.plan_total) {
         int lo = 0, hi = b.n - 1;
         while (lo < hi) {
@@ -48,15 +47,13 @@ __global__ __launch_bounds__(kBatchPlanBlock) void batch_plan(BatchArgs b)
         }
         sim = lo;
         const StepArgs& a = *(const StepArgs*)&sims[sim].a;
-        plan_wave(a, gw - sims[sim].plan_base, lane, put, item, need, act);
-        heavy = plan_heavy(need, a.kchunk);
+        plan_wave(a, gw - sims[sim].plan_base, lane, put, item, need);
     }
-    const unsigned q = plan_slot<kPlanWaves>(put, heavy, cnt, cnt + 2, (unsigned)b.wl_cap, s_cnt);
+    const unsigned q = plan_slot<kPlanWaves>(put, cnt, s_cnt);
     if (put) {
         b.wl_sim[q] = sim;
         b.wl_item[q] = item;
         b.wl_need[q] = need;
-        b.wl_act[q] = act;
     }
 }
 
@@ -71,8 +68,6 @@ __global__ __launch_bounds__(64) void batch_advance(BatchArgs b)
     if (s == 0) {
         const unsigned p = b.cnt[8];
         b.cnt[4 * (1 - p)] = 0u;
-        b.cnt[4 * (1 - p) + 1] = 0u;
-        b.cnt[4 * (1 - p) + 2] = 0u;
         b.cnt[8] = 1u - p;
     }
     if (s >= b.n) return;
@@ -83,9 +78,7 @@ __global__ __launch_bounds__(64) void batch_advance(BatchArgs b)
     m.parity = (m.parity + 1) % 3;
     unsigned* next = m.cnt + 4 * m.parity;
     next[0] = 0u;
-    next[1] = 0u;
     next[2] = 0u;
-    next[3] = 0u;
     StepArgs& a = m.a;
     a.ph = m.ph[m.cur];
     a.arg = m.arg[m.cur];
@@ -93,6 +86,8 @@ __global__ __launch_bounds__(64) void batch_advance(BatchArgs b)
     a.arg_new = m.arg[1 - m.cur];
     a.act_src = m.act[m.cur];
     a.act_dst = m.act[1 - m.cur];
+    a.row_src = m.row[m.cur];
+    a.row_dst = m.row[1 - m.cur];
     a.ep_src = m.ep[m.cur];
     a.ep_dst = m.ep[1 - m.cur];
     m.ep_ctr += 1u;
@@ -100,7 +95,6 @@ __global__ __launch_bounds__(64) void batch_advance(BatchArgs b)
     a.fix_count = next;
     a.cnt_next = m.cnt + 4 * ((m.parity + 1) % 3);
     a.wl_count = next + 2;
-    a.wl_light = next + 1;
     // t_cur_step = (2*kt+1)*dt*tau0 in float (3DgrainMPI/APTPhaseField.cu:863,919)
     a.t = (float)m.step * a.dt * m.tau0;
 }
@@ -360,17 +354,19 @@ __global__ __launch_bounds__(kBlock) void nucl_kernel(NuclArgs a)
                     if (v > -0.9999f) a.arg[o] = id;
                     a.act[(gk + lk) * a.ntiles + act_tile_x(gi + li) + act_tile_y(gj + lj) * a.ntx] =
                         a.ep;
+                    atomicMax(a.row + ((gk + lk) * a.fny + gj + lj) * a.ntx + act_tile_x(gi + li), a.ep << 4 | 1u);
                 }
         a.status[C] = 1;
         atomicAdd(a.events, 1ull);
     }
 }
 
-// Activity map from a buffer's contents (after it was written other than by
-// a step): one lane per interior point, K slots each.
+// Activity and row maps from a buffer's contents (after it was written other
+// than by a step): one lane per interior point, K slots each.
 __global__ __launch_bounds__(kBlock) void act_rebuild_kernel(const float* __restrict__ ph,
                                                              const int* __restrict__ arg,
-                                                             unsigned* act, unsigned ep, int fnx,
+                                                             unsigned* act, unsigned* row,
+                                                             unsigned ep, int fnx,
                                                              int fny, int fnz, int K, int ntx,
                                                              int ntiles)
 {
@@ -383,9 +379,12 @@ __global__ __launch_bounds__(kBlock) void act_rebuild_kernel(const float* __rest
     const int i = 1 + r - (j - 1) * nx;
     const int L = fnx * fny * fnz;
     const int C = i + j * fnx + k * fnx * fny;
-    bool on = false;
-    for (int s = 0; s < K; ++s) on = on || arg[C + s * L] != -1 || ph[C + s * L] != -1.0f;
-    if (on) act[k * ntiles + act_tile_x(i) + act_tile_y(j) * ntx] = ep;
+    unsigned bound = 0u;
+    for (int s = 0; s < K; ++s) bound = arg[C + s * L] != -1 || ph[C + s * L] != -1.0f ? s + 1u : bound;
+    if (bound) {
+        act[k * ntiles + act_tile_x(i) + act_tile_y(j) * ntx] = ep;
+        atomicMax(row + (k * fny + j) * ntx + act_tile_x(i), ep << 4 | bound);
+    }
 }
 
 // Plain streaming copy (16 B per lane per iteration), the reference point for
@@ -422,15 +421,15 @@ hipError_t launch_batch_advance(const BatchArgs& b, hipStream_t stream)
 }
 
 hipError_t launch_step(const StepArgs& a, int K, int gather27, hipStream_t stream,
-                       const EdgeLaunch* edge, hipEvent_t ev_begin, hipEvent_t ev_planned,
-                       hipEvent_t ev_mid, hipEvent_t ev_end, bool planned, const StepArgs* next)
+                       hipEvent_t ev_begin, hipEvent_t ev_planned, hipEvent_t ev_mid, hipEvent_t ev_end,
+                       bool planned, const StepArgs* next)
 {
     if (K == 5)
-        return gather27 ? launch_step_k5_g27(a, stream, edge, ev_begin, ev_planned, ev_mid, ev_end, planned, next)
-                        : launch_step_k5_g7(a, stream, edge, ev_begin, ev_planned, ev_mid, ev_end, planned, next);
+        return gather27 ? launch_step_k5_g27(a, stream, ev_begin, ev_planned, ev_mid, ev_end, planned, next)
+                        : launch_step_k5_g7(a, stream, ev_begin, ev_planned, ev_mid, ev_end, planned, next);
     if (K == 8)
-        return gather27 ? launch_step_k8_g27(a, stream, edge, ev_begin, ev_planned, ev_mid, ev_end, planned, next)
-                        : launch_step_k8_g7(a, stream, edge, ev_begin, ev_planned, ev_mid, ev_end, planned, next);
+        return gather27 ? launch_step_k8_g27(a, stream, ev_begin, ev_planned, ev_mid, ev_end, planned, next)
+                        : launch_step_k8_g7(a, stream, ev_begin, ev_planned, ev_mid, ev_end, planned, next);
     return hipErrorInvalidValue;
 }
 
@@ -457,12 +456,12 @@ int fixup_kernel_slots(int K, int gather27, int device, bool batch)
     return slots(K, gather27, device, batch ? 3 : 2);
 }
 
-hipError_t launch_act_rebuild(const float* ph, const int* arg, unsigned* act, unsigned ep, int fnx,
-                              int fny, int fnz, int K, int ntx, int ntiles, hipStream_t stream)
+hipError_t launch_act_rebuild(const float* ph, const int* arg, unsigned* act, unsigned* row, unsigned ep,
+                              int fnx, int fny, int fnz, int K, int ntx, int ntiles, hipStream_t stream)
 {
     const long long n = (long long)(fnx - 2) * (fny - 2) * (fnz - 2);
     hipLaunchKernelGGL(act_rebuild_kernel, dim3(cdiv(n, kBlock)), dim3(kBlock), 0, stream, ph, arg,
-                       act, ep, fnx, fny, fnz, K, ntx, ntiles);
+                       act, row, ep, fnx, fny, fnz, K, ntx, ntiles);
     return hipGetLastError();
 }
 

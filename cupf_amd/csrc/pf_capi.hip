@@ -28,15 +28,6 @@ struct pf_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    // the stream of the overflow steps' edge kernel and the events that fork
-    // it off `stream` and join it back before the fix-up
-    EdgeLaunch edge = {nullptr, nullptr, nullptr};
-    // Marks every kLeadEvery launches (kLeadSlots of them in turn): before a
-    // slot is reused, the host waits for the launch it marked, so it runs at
-    // most kLeadEvery * kLeadSlots launches ahead of the device and the fix-up's
-    // overflow report it chooses the step variant by is at most that old.
-    static constexpr int kLeadEvery = 8, kLeadSlots = 4;
-    hipEvent_t lead[kLeadSlots] = {};
     int L = 0;
     int cur = 0;                    // index of the current buffer
     float* ph[2] = {nullptr, nullptr};
@@ -51,7 +42,6 @@ struct pf_ctx {
     unsigned long long* counters = nullptr;  // [0] overflow points, [1] nucleation events
     unsigned* fix_list = nullptr;   // overflow fix-up list, one entry per interior point
     unsigned* fix_count = nullptr;  // three 4-word counter sets, used by steps in turn
-    int* sink = nullptr;            // 128 words written by lanes that must not store
     long long* sums = nullptr;
     std::vector<long long> h_sums;
     int* alpha_full = nullptr;
@@ -63,30 +53,24 @@ struct pf_ctx {
     unsigned long long ncall = 0;
     long long wl_alloc = 0;         // entries allocated for wl_item / wl_need / wl_act
     long long fix_alloc = 0;        // entries allocated for fix_list
-    int kchunk = 4;                 // z planes per work item
-    // Activity map per buffer (one word per 64x4 column tile and z plane) and
-    // the epoch each buffer was last written at; see StepArgs.
+    int kchunk = 1;                 // z planes per work item
+    // Activity map per buffer (one word per 64x4 column tile and z plane), row
+    // map (one per row of a tile) and the epoch each buffer was last written
+    // at; see StepArgs.
     unsigned* act[2] = {nullptr, nullptr};
+    unsigned* row[2] = {nullptr, nullptr};
     unsigned ep[2] = {1u, 1u};
     unsigned ep_ctr = 1u;
     int use_act = 1;
     int ntx = 0, nty = 0, ntiles = 0;
-    // Work list of the step (filled by the plan kernel, cleared by the fix-up).
+    // Work list of the step (filled by the plan kernel).
     int* wl_item = nullptr;
     unsigned long long* wl_need = nullptr;
-    unsigned long long* wl_act = nullptr;
     unsigned long long nlaunch = 0;  // step launches so far (selects the counter set)
-    // Step kernel variant: the fix-up's report (pinned host memory: launch of
-    // the last fix-up, launch of the last one with a non-empty list), and the
-    // launch up to which the overflow variant is used regardless (a new state).
-    unsigned long long* seen = nullptr;
-    unsigned long long ovf_until = 0;
-    int variant_force = -1;         // CUPF_STEP_VARIANT: 0 / 1 fixes the variant (tests, timing)
-    int nzchunk = 0, edge_cols = 0, edge_items = 0, items_chunk = 0;
-    int tiles_x = 0, tiles_y = 0;   // LDS tiles (partial ones included)
-    int step_blocks = 0;            // persistent step workgroups (occupancy x CUs)
+    int nzchunk = 0, items_chunk = 0;
+    int tiles_x = 0, tiles_y = 0;   // column tiles (partial ones included)
+    int step_blocks = 0;            // persistent step waves (occupancy x CUs, at most one per unit)
     int fix_blocks = 0;             // fix-up workgroups (occupancy x CUs)
-    // overflow on the LDS path by tile plane (see StepArgs)
     bool have_coords = false, have_orient = false, have_state = false;
 };
 
@@ -163,41 +147,6 @@ int ctx_check(pf_ctx* c)
 
 int buf_index(pf_ctx* c, int which) { return which == 0 ? c->cur : 1 - c->cur; }
 
-// Launches without a reported heavy overflow (a fix-up list of kOvfHeavy
-// points or more) after which the step kernel without the keep test, its
-// edge items inside it, is used (7-point gather).  The report lags
-// the launches by the queue's depth (at most kLeadEvery * kLeadSlots); either
-// variant gives the same bits.  The lag and the quiet period are kept short:
-// the overflow variant's edge kernel costs 15-35 us per launch once little
-// overflows.
-constexpr unsigned long long kOvfQuiet = 16;
-// Launches after a new state that take the overflow variant whatever the
-// reports say (those in flight are still the old state's).
-constexpr unsigned long long kOvfNew =
-    (unsigned long long)(pf_ctx::kLeadEvery * pf_ctx::kLeadSlots) + kOvfQuiet;
-
-// Before launch c->nlaunch: every kLeadEvery launches, wait for the launch
-// marked kLeadEvery * kLeadSlots launches ago, then mark this one.
-hipError_t bound_lead(pf_ctx* c)
-{
-    if (c->nlaunch % pf_ctx::kLeadEvery != 0) return hipSuccess;
-    hipEvent_t& e = c->lead[(c->nlaunch / pf_ctx::kLeadEvery) % pf_ctx::kLeadSlots];
-    hipError_t r = hipEventSynchronize(e);  // an event never recorded completes at once
-    if (r != hipSuccess) return r;
-    return hipEventRecord(e, c->stream);
-}
-
-int ovf_variant(const pf_ctx* c)
-{
-    if (c->p.gather27) return 0;
-    if (c->variant_force >= 0) return c->variant_force;
-    if (c->nlaunch < c->ovf_until || !c->seen) return 1;
-    const volatile unsigned long long* r = c->seen;
-    const unsigned long long last = r[1], now = r[0];
-    if (now == 0) return 1;  // nothing reported yet
-    return now < last + kOvfQuiet ? 1 : 0;
-}
-
 StepArgs make_step_args(pf_ctx* c, int src, float t, int use_iuc)
 {
     const pf_params& p = c->p;
@@ -222,22 +171,19 @@ StepArgs make_step_args(pf_ctx* c, int src, float t, int use_iuc)
         a.fix_count = c->fix_count + 4 * set;
         a.cnt_next = c->fix_count + 4 * ((set + 1) % 3);
         a.wl_count = a.fix_count + 2;
-        a.wl_light = a.fix_count + 1;
     }
-    a.sink_i = c->sink;
-    a.sink_f = reinterpret_cast<float*>(c->sink + 64);
     a.fnx = p.fnx;
     a.fny = p.fny;
     a.fnz = p.fnz;
     a.L = c->L;
-    a.ncolx = p.fnx - 2;
-    a.ncols = (p.fnx - 2) * (p.fny - 2);
     a.kchunk = c->kchunk;
     a.nzchunk = c->nzchunk;
     a.tiles_x = c->tiles_x;
     a.tiles_y = c->tiles_y;
     a.act_src = c->act[src];
     a.act_dst = c->act[1 - src];
+    a.row_src = c->row[src];
+    a.row_dst = c->row[1 - src];
     a.ep_src = c->ep[src];
     a.ep_dst = c->ep[1 - src];
     a.ep_new = ++c->ep_ctr;
@@ -245,18 +191,11 @@ StepArgs make_step_args(pf_ctx* c, int src, float t, int use_iuc)
     a.ntx = c->ntx;
     a.nty = c->nty;
     a.ntiles = c->ntiles;
-    a.edge_cols = c->edge_cols;
-    a.ovf_variant = ovf_variant(c);
-    a.seen = c->seen;
-    a.launch_index = c->nlaunch + 1;
-    a.edge_items = edge_items_per_chunk(c->edge_cols, p.fny, c->kchunk, p.gather27 != 0,
-                                        a.ovf_variant != 0);
     a.items_chunk = c->items_chunk;
     a.step_blocks = c->step_blocks;
     a.fix_blocks = c->fix_blocks;
     a.wl_item = c->wl_item;
     a.wl_need = c->wl_need;
-    a.wl_act = c->wl_act;
 
     a.bcx = p.bcx;
     a.bcy = p.bcy;
@@ -310,6 +249,7 @@ int nucl_launch(pf_ctx* c, float t, float dt_nuc, int use_iuc)
     a.ball = c->ball;
     a.events = c->counters + 1;
     a.act = c->act[c->cur];
+    a.row = c->row[c->cur];
     a.ep = c->ep[c->cur];
     a.ntx = c->ntx;
     a.ntiles = c->ntiles;
@@ -349,24 +289,32 @@ int nucl_launch(pf_ctx* c, float t, float dt_nuc, int use_iuc)
     return PF_OK;
 }
 
-// Activity map of buffer b from its contents, under a fresh epoch.
+// Activity and row maps of buffer b from their contents, under a fresh epoch.
 hipError_t act_rebuild(pf_ctx* c, int b)
 {
     const pf_params& p = c->p;
     c->ep[b] = ++c->ep_ctr;
-    return launch_act_rebuild(c->ph[b], c->arg[b], c->act[b], c->ep[b], p.fnx, p.fny, p.fnz, p.K,
+    return launch_act_rebuild(c->ph[b], c->arg[b], c->act[b], c->row[b], c->ep[b], p.fnx, p.fny, p.fnz, p.K,
                               c->ntx, c->ntiles, c->stream);
 }
 
-// Before the epoch counter could wrap within the next `ahead` steps: clear
-// both maps and rebuild them.
+// The epoch counter's limit: row words hold an epoch and 4 bits of bound.
+constexpr unsigned kEpochMax = 0x07ffffffu;
+
+size_t row_words(const pf_params& p) { return (size_t)((p.fnx - 2 + 63) / 64) * p.fny * p.fnz; }
+
+// Before the epoch counter could pass its limit within the next `ahead`
+// steps: clear the maps and rebuild them.
 hipError_t act_renew_if_needed(pf_ctx* c, unsigned ahead = 1u)
 {
-    if (c->ep_ctr < 0x7fffffffu - ahead) return hipSuccess;
+    if (c->ep_ctr < kEpochMax - ahead) return hipSuccess;
     const size_t n = (size_t)c->ntiles * c->p.fnz;
     hipError_t e;
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < 2; ++b) {
         if ((e = hipMemsetAsync(c->act[b], 0, n * sizeof(unsigned), c->stream)) != hipSuccess) return e;
+        if ((e = hipMemsetAsync(c->row[b], 0, row_words(c->p) * sizeof(unsigned), c->stream)) != hipSuccess)
+            return e;
+    }
     c->ep_ctr = 1u;
     if ((e = act_rebuild(c, 0)) != hipSuccess) return e;
     return act_rebuild(c, 1);
@@ -375,23 +323,15 @@ hipError_t act_renew_if_needed(pf_ctx* c, unsigned ahead = 1u)
 void free_ctx(pf_ctx* c)
 {
     (void)hipSetDevice(c->device);
-    // a step that failed between its fork and join leaves the edge stream unjoined
-    if (c->edge.stream) (void)hipStreamSynchronize(c->edge.stream);
     void* bufs[] = {c->ph[0], c->ph[1], c->arg[0], c->arg[1], c->x, c->y, c->z, c->zbuf,
                     c->R12, c->psi_mac, c->T3d, c->phi0, c->phi, c->alpha, c->counters,
                     c->sums, c->alpha_full, c->loss, c->nstatus, c->ball,
-                    c->fix_list, c->fix_count, c->sink, c->act[0], c->act[1],
-                    c->wl_item, c->wl_need, c->wl_act};
+                    c->fix_list, c->fix_count, c->act[0], c->act[1],
+                    c->row[0], c->row[1], c->wl_item, c->wl_need};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
-    if (c->seen) (void)hipHostFree(c->seen);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
-    for (hipEvent_t e : c->lead)
-        if (e) (void)hipEventDestroy(e);
-    if (c->edge.ready) (void)hipEventDestroy(c->edge.ready);
-    if (c->edge.done) (void)hipEventDestroy(c->edge.done);
-    if (c->edge.stream) (void)hipStreamDestroy(c->edge.stream);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -410,28 +350,14 @@ struct pf_batch {
     int* wl_sim = nullptr;
     int* wl_item = nullptr;
     unsigned long long* wl_need = nullptr;
-    unsigned long long* wl_act = nullptr;
-    unsigned* cnt = nullptr;        // 2 x 4 list counters, parity word, fix-up count
+    unsigned* cnt = nullptr;        // 2 x 4 list counters, parity word
     size_t wl_cap = 0;
-    // hipGraphs of kGraphSteps batched steps, one per step kernel variant,
-    // each captured for one kchunk
-    hipGraph_t graph[2] = {nullptr, nullptr};
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
-    int graph_kchunk[2] = {0, 0};
+    // hipGraph of kGraphSteps batched steps, captured for one kchunk
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t gexec = nullptr;
+    int graph_kchunk = 0;
     static constexpr int kGraphSteps = 8;
     static constexpr int kMinChunk = 2;
-    // Step kernel variant choice, as for a single context: batch_fixup
-    // reports (pinned) the index within the current run of its step and of
-    // the last step whose lists held kOvfHeavy points or more in all.
-    unsigned long long* seen = nullptr;
-    unsigned long long nstep = 0;     // batched steps enqueued over the batch's life
-    unsigned long long seen_base = 0; // nstep when the current run began
-    unsigned long long heavy_at = 0;  // last step known to overflow heavily (1-based)
-    int variant_force = -1;           // CUPF_STEP_VARIANT
-    // lead bound: a mark every kGraphSteps steps, kLeadSlots of them in turn
-    static constexpr int kLeadSlots = 4;
-    hipEvent_t lead[kLeadSlots] = {};
-    unsigned long long lead_n = 0, next_mark = 0;
 };
 
 namespace {
@@ -439,16 +365,11 @@ namespace {
 void batch_free(pf_batch* b)
 {
     (void)hipSetDevice(b->device);
-    for (int v = 0; v < 2; ++v) {
-        if (b->gexec[v]) (void)hipGraphExecDestroy(b->gexec[v]);
-        if (b->graph[v]) (void)hipGraphDestroy(b->graph[v]);
-    }
-    void* bufs[] = {b->sims, b->wl_sim, b->wl_item, b->wl_need, b->wl_act, b->cnt};
+    if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
+    if (b->graph) (void)hipGraphDestroy(b->graph);
+    void* bufs[] = {b->sims, b->wl_sim, b->wl_item, b->wl_need, b->cnt};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
-    if (b->seen) (void)hipHostFree(b->seen);
-    for (hipEvent_t e : b->lead)
-        if (e) (void)hipEventDestroy(e);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }
@@ -459,7 +380,7 @@ int batch_upload(pf_batch* b, const std::vector<int>& first_step, int use_iuc, B
 {
     const int n = (int)b->ctxs.size();
     std::vector<BatchSim> h(n);
-    int plan_total = 0, edge_total = 0;
+    int plan_total = 0, strip_total = 0;
     for (int i = 0; i < n; ++i) {
         pf_ctx* c = b->ctxs[i];
         const pf_params& p = c->p;
@@ -468,13 +389,13 @@ int batch_upload(pf_batch* b, const std::vector<int>& first_step, int use_iuc, B
         m.a = make_step_args(c, c->cur, t, use_iuc);  // takes this step's epoch from the context
         m.a.kchunk = b->kchunk;
         m.a.nzchunk = (p.fnz - 2 + b->kchunk - 1) / b->kchunk;
-        m.a.edge_items = edge_items_per_chunk(c->edge_cols, p.fny, b->kchunk, p.gather27 != 0, true);
         m.a.step_blocks = b->step_blocks;
         m.a.fix_blocks = b->fix_blocks;
         for (int q = 0; q < 2; ++q) {
             m.ph[q] = c->ph[q];
             m.arg[q] = c->arg[q];
             m.act[q] = c->act[q];
+            m.row[q] = c->row[q];
             m.ep[q] = c->ep[q];
         }
         m.ep_ctr = c->ep_ctr;
@@ -484,53 +405,23 @@ int batch_upload(pf_batch* b, const std::vector<int>& first_step, int use_iuc, B
         m.cnt = c->fix_count;
         m.tau0 = p.tau0;
         m.plan_base = plan_total;
-        m.edge_base = edge_total;
+        m.strip_base = strip_total;
         plan_total += plan_waves(b->kchunk, m.a.nzchunk, m.a.items_chunk);
-        edge_total += m.a.nzchunk * m.a.edge_items;
+        strip_total += m.a.nzchunk * strip_waves(strip_width(p.fnx, c->tiles_x), p.fny);
     }
     HIPCHK(hipMemcpyAsync(b->sims, h.data(), sizeof(BatchSim) * n, hipMemcpyHostToDevice, b->stream));
-    HIPCHK(hipMemsetAsync(b->cnt, 0, 10 * sizeof(unsigned), b->stream));
+    HIPCHK(hipMemsetAsync(b->cnt, 0, 9 * sizeof(unsigned), b->stream));
     ba.sims = b->sims;
     ba.n = n;
     ba.plan_total = plan_total;
-    ba.edge_total = edge_total;
+    ba.strip_total = strip_total;
     ba.wl_sim = b->wl_sim;
     ba.wl_item = b->wl_item;
     ba.wl_need = b->wl_need;
-    ba.wl_act = b->wl_act;
-    ba.wl_cap = (int)b->wl_cap;
     ba.cnt = b->cnt;
     ba.step_blocks = b->step_blocks;
     ba.fix_blocks = b->fix_blocks;
-    ba.seen = b->seen;
-    ba.ovf_variant = 0;
     return PF_OK;
-}
-
-// The step kernel variant of the next batched step (1: with the
-// keep test), from the fix-up's reports as for a single context.
-int batch_variant(pf_batch* b)
-{
-    if (b->g27) return 0;
-    if (b->variant_force >= 0) return b->variant_force;
-    const volatile unsigned long long* r = b->seen;
-    const unsigned long long now = r[0], last = r[1];
-    if (last) b->heavy_at = std::max(b->heavy_at, b->seen_base + last);
-    return b->seen_base + now < b->heavy_at + kOvfQuiet ? 1 : 0;
-}
-
-// Before the steps from b->nstep on: every kGraphSteps steps, wait for the
-// mark set kLeadSlots marks before, then mark the stream, so the host runs at
-// most ~kLeadSlots * kGraphSteps steps ahead of the reports it chooses by.
-hipError_t batch_bound_lead(pf_batch* b)
-{
-    if (b->nstep < b->next_mark) return hipSuccess;
-    hipEvent_t& e = b->lead[b->lead_n % pf_batch::kLeadSlots];
-    hipError_t r = hipEventSynchronize(e);  // an event never recorded completes at once
-    if (r != hipSuccess) return r;
-    ++b->lead_n;
-    b->next_mark = b->nstep + pf_batch::kGraphSteps;
-    return hipEventRecord(e, b->stream);
 }
 
 // The host side of nsteps batched steps (what step_impl does per launch),
@@ -559,22 +450,14 @@ int batch_run(pf_batch* b, int nsteps, std::vector<int>& first_step, int use_iuc
     BatchArgs ba;
     int rc = batch_upload(b, first_step, use_iuc, ba);
     if (rc) return rc;
-    // the previous run ended with a synchronisation: fold its last reports in,
-    // then count this run's steps from 1 (batch_upload cleared the device count)
-    (void)batch_variant(b);
-    b->seen[0] = b->seen[1] = 0ull;
-    b->seen_base = b->nstep;
     int left = nsteps;
     while (left > 0) {
-        HIPCHK(batch_bound_lead(b));
-        const int v = batch_variant(b);
-        ba.ovf_variant = v;
         if (use_graph && left >= pf_batch::kGraphSteps) {
-            if (!b->gexec[v] || b->graph_kchunk[v] != b->kchunk) {
-                if (b->gexec[v]) (void)hipGraphExecDestroy(b->gexec[v]);
-                if (b->graph[v]) (void)hipGraphDestroy(b->graph[v]);
-                b->gexec[v] = nullptr;
-                b->graph[v] = nullptr;
+            if (!b->gexec || b->graph_kchunk != b->kchunk) {
+                if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
+                if (b->graph) (void)hipGraphDestroy(b->graph);
+                b->gexec = nullptr;
+                b->graph = nullptr;
                 HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
                 hipError_t e = hipSuccess;
                 for (int q = 0; q < pf_batch::kGraphSteps && e == hipSuccess; ++q)
@@ -586,17 +469,15 @@ int batch_run(pf_batch* b, int nsteps, std::vector<int>& first_step, int use_iuc
                     return fail(PF_E_HIP, std::string("graph capture: ") +
                                               hipGetErrorString(e != hipSuccess ? e : e2));
                 }
-                b->graph[v] = g;
-                HIPCHK(hipGraphInstantiate(&b->gexec[v], b->graph[v], nullptr, nullptr, 0));
-                b->graph_kchunk[v] = b->kchunk;
+                b->graph = g;
+                HIPCHK(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
+                b->graph_kchunk = b->kchunk;
             }
-            HIPCHK(hipGraphLaunch(b->gexec[v], b->stream));
+            HIPCHK(hipGraphLaunch(b->gexec, b->stream));
             left -= pf_batch::kGraphSteps;
-            b->nstep += pf_batch::kGraphSteps;
         } else {
             HIPCHK(launch_batch_step(ba, b->K, b->g27, b->stream));
             --left;
-            ++b->nstep;
         }
     }
     HIPCHK(hipStreamSynchronize(b->stream));
@@ -643,29 +524,33 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
         if (v >= 1 && v <= 61) c->kchunk = v;  // plane masks of a chunk fit 64 bits
     }
     if (const char* na = getenv("CUPF_NO_ACTIVITY")) c->use_act = atoi(na) ? 0 : 1;
-    if (const char* sv = getenv("CUPF_STEP_VARIANT")) c->variant_force = atoi(sv) ? 1 : 0;
     c->ntx = (p.fnx - 2 + 63) / 64;
     c->nty = (p.fny - 2 + 3) / 4;
     c->ntiles = c->ntx * c->nty;
     {
-        // 64x4 tiles take the LDS path, a partial tile where the +x leftover is
-        // at least kPartialMin wide and always in y; a narrower +x strip goes to
-        // edge items of 256 points each
+        // 64x4 column tiles, a partial one where the +x leftover is at least
+        // kPartialMin wide and always in y; a narrower +x leftover is the strip
         int tiles_x = (p.fnx - 2) / 64;
-        int ex = (p.fnx - 2) - tiles_x * 64;
-        if (ex >= kPartialMin) {
-            ++tiles_x;
-            ex = 0;
-        }
+        const int ex = (p.fnx - 2) - tiles_x * 64;
+        if (ex >= kPartialMin) ++tiles_x;
         c->tiles_x = tiles_x;
         c->tiles_y = (p.fny - 2 + 3) / 4;
-        c->edge_cols = ex * (p.fny - 2);
-        c->edge_items = edge_items_per_chunk(c->edge_cols, p.fny, c->kchunk, p.gather27 != 0, false);
         c->items_chunk = c->tiles_x * c->tiles_y;
         c->nzchunk = (p.fnz - 2 + c->kchunk - 1) / c->kchunk;
     }
-    c->step_blocks = step_kernel_slots(p.K, p.gather27, device);
-    c->fix_blocks = fixup_kernel_slots(p.K, p.gather27, device, false);
+    {
+        // one wave per unit is enough: a small grid does not dispatch idle waves
+        const long long units = c->nzchunk * (4LL * c->items_chunk + strip_waves(strip_width(p.fnx, c->tiles_x), p.fny));
+        c->step_blocks = (int)std::min<long long>(step_kernel_slots(p.K, p.gather27, device), units);
+    }
+    {
+        // at most the workgroups that could have an overflowed point (4 waves
+        // of 8 or, 27-point gather, 4 points)
+        const long long interior = (long long)(p.fnx - 2) * (p.fny - 2) * (p.fnz - 2);
+        const int per = p.gather27 ? 16 : 32;
+        c->fix_blocks = (int)std::min<long long>(fixup_kernel_slots(p.K, p.gather27, device, false),
+                                                 (interior + per - 1) / per);
+    }
     if (c->step_blocks < 1 || c->fix_blocks < 1) {
         delete c;
         return fail(PF_E_HIP, "occupancy query for the step or fix-up kernel failed");
@@ -687,14 +572,6 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
         return bail(fail(PF_E_HIP, "hipStreamCreate failed"));
     if (hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess)
         return bail(fail(PF_E_HIP, "hipEventCreate failed"));
-    for (hipEvent_t& e : c->lead)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
-            return bail(fail(PF_E_HIP, "hipEventCreate failed"));
-    if (c->edge_items > 0 && !p.gather27 &&
-        (hipStreamCreateWithFlags(&c->edge.stream, hipStreamNonBlocking) != hipSuccess ||
-         hipEventCreateWithFlags(&c->edge.ready, hipEventDisableTiming) != hipSuccess ||
-         hipEventCreateWithFlags(&c->edge.done, hipEventDisableTiming) != hipSuccess))
-        return bail(fail(PF_E_HIP, "edge stream or event creation failed"));
     const size_t nst = (size_t)L * p.K;
     for (int b = 0; b < 2; ++b) {
         if ((rc = dalloc(&c->ph[b], nst)) || (rc = dalloc(&c->arg[b], nst))) return bail(rc);
@@ -704,12 +581,12 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
         (rc = dalloc(&c->phi, (size_t)L)) || (rc = dalloc(&c->alpha, (size_t)L)) ||
         (rc = dalloc(&c->counters, 2)) || (rc = dalloc(&c->sums, p.fnz)) ||
         (rc = dalloc(&c->fix_list, (size_t)(c->fix_alloc = (long long)(p.fnx - 2) * (p.fny - 2) * (p.fnz - 2)))) ||
-        (rc = dalloc(&c->fix_count, 12)) || (rc = dalloc(&c->sink, 128)) ||
+        (rc = dalloc(&c->fix_count, 12)) ||
         (rc = dalloc(&c->act[0], (size_t)c->ntiles * p.fnz)) ||
         (rc = dalloc(&c->act[1], (size_t)c->ntiles * p.fnz)) ||
+        (rc = dalloc(&c->row[0], row_words(p))) || (rc = dalloc(&c->row[1], row_words(p))) ||
         (rc = dalloc(&c->wl_item, (size_t)(c->wl_alloc = (long long)c->nzchunk * c->items_chunk + 1))) ||
-        (rc = dalloc(&c->wl_need, (size_t)c->nzchunk * c->items_chunk + 1)) ||
-        (rc = dalloc(&c->wl_act, (size_t)c->nzchunk * c->items_chunk + 1)))
+        (rc = dalloc(&c->wl_need, (size_t)c->nzchunk * c->items_chunk + 1)))
         return bail(rc);
     c->h_sums.resize(p.fnz);
     for (int b = 0; b < 2; ++b) {
@@ -722,14 +599,10 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
         hipMemsetAsync(c->alpha, 0, L * sizeof(int), c->stream) != hipSuccess ||
         hipMemsetAsync(c->act[0], 0, (size_t)c->ntiles * p.fnz * sizeof(unsigned), c->stream) != hipSuccess ||
         hipMemsetAsync(c->act[1], 0, (size_t)c->ntiles * p.fnz * sizeof(unsigned), c->stream) != hipSuccess ||
+        hipMemsetAsync(c->row[0], 0, row_words(p) * sizeof(unsigned), c->stream) != hipSuccess ||
+        hipMemsetAsync(c->row[1], 0, row_words(p) * sizeof(unsigned), c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
         return bail(fail(PF_E_HIP, "initial fill failed"));
-    if (hipHostMalloc(&c->seen, 2 * sizeof(unsigned long long)) != hipSuccess) {
-        c->seen = nullptr;
-        return bail(fail(PF_E_NOMEM, "hipHostMalloc of the step variant report failed"));
-    }
-    c->seen[0] = c->seen[1] = 0ull;
-    c->ovf_until = kOvfNew;
     *out = c;
     return PF_OK;
 }
@@ -840,7 +713,6 @@ int pf_init_from_phi_alpha(pf_ctx* c, const float* phi0, const int* alpha0)
     HIPCHK(act_rebuild(c, 1));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->have_state = true;
-    c->ovf_until = c->nlaunch + kOvfNew;  // a new state may overflow
     return PF_OK;
 }
 
@@ -855,7 +727,6 @@ int pf_reinit_from_collect(pf_ctx* c)
     HIPCHK(act_rebuild(c, 0));
     HIPCHK(act_rebuild(c, 1));
     HIPCHK(hipStreamSynchronize(c->stream));
-    c->ovf_until = c->nlaunch + kOvfNew;  // a new state may overflow
     return PF_OK;
 }
 
@@ -871,7 +742,6 @@ int pf_upload_state(pf_ctx* c, int which, const float* ph, const int* arg)
     HIPCHK(act_rebuild(c, b));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->have_state = true;
-    c->ovf_until = c->nlaunch + kOvfNew;  // a new state may overflow
     return PF_OK;
 }
 
@@ -937,7 +807,6 @@ static int step_impl(pf_ctx* c, int nsteps, int first_step, int flags)
         const float t = s * p.dt * p.tau0;
         if (!have) {
             HIPCHK(act_renew_if_needed(c));
-            HIPCHK(bound_lead(c));
             a = make_step_args(c, c->cur, t, use_iuc);
             planned = false;
         }
@@ -947,13 +816,12 @@ static int step_impl(pf_ctx* c, int nsteps, int first_step, int flags)
         c->cur = 1 - c->cur;
         // an activity-map renewal (epoch counter near its end) must come
         // between this step and the next plan: no fused launch then
-        have = !nucl && s + 1 < end && c->ep_ctr < 0x7fffffffu - 1u;
+        have = !nucl && s + 1 < end && c->ep_ctr < kEpochMax - 1u;
         if (have) {
-            HIPCHK(bound_lead(c));
             a = make_step_args(c, c->cur, (s + 1) * p.dt * p.tau0, use_iuc);
         }
-        HIPCHK(launch_step(cur, p.K, p.gather27, c->stream, &c->edge, nullptr, nullptr, nullptr,
-                           nullptr, planned, have ? &a : nullptr));
+        HIPCHK(launch_step(cur, p.K, p.gather27, c->stream, nullptr, nullptr, nullptr, nullptr, planned,
+                           have ? &a : nullptr));
         planned = have;
         if (nucl && (s & 1)) {
             int rc = nucl_launch(c, t, 2.0f * p.dt * p.tau0, use_iuc);
@@ -1002,10 +870,9 @@ int pf_step_profiled(pf_ctx* c, int nsteps, int first_step, int flags, float* ms
         const int s = first_step + q;
         const float t = s * p.dt * p.tau0;
         err = act_renew_if_needed(c);
-        if (err == hipSuccess) err = bound_lead(c);
         if (err != hipSuccess) break;
         StepArgs a = make_step_args(c, c->cur, t, use_iuc);
-        err = launch_step(a, p.K, p.gather27, c->stream, &c->edge, ev[4 * q], ev[4 * q + 1],
+        err = launch_step(a, p.K, p.gather27, c->stream, ev[4 * q], ev[4 * q + 1],
                           ev[4 * q + 2], ev[4 * q + 3]);
         if (err != hipSuccess) break;
         ++c->nlaunch;
@@ -1481,17 +1348,8 @@ int pf_batch_create(pf_ctx* const* ctxs, int n, pf_batch** out)
     int rc;
     if ((rc = dalloc(&b->sims, (size_t)n)) || (rc = dalloc(&b->wl_sim, b->wl_cap + 1)) ||
         (rc = dalloc(&b->wl_item, b->wl_cap + 1)) || (rc = dalloc(&b->wl_need, b->wl_cap + 1)) ||
-        (rc = dalloc(&b->wl_act, b->wl_cap + 1)) || (rc = dalloc(&b->cnt, 10)))
+        (rc = dalloc(&b->cnt, 9)))
         return bail(rc);
-    for (hipEvent_t& e : b->lead)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
-            return bail(fail(PF_E_HIP, "hipEventCreate failed"));
-    if (hipHostMalloc(&b->seen, 2 * sizeof(unsigned long long)) != hipSuccess) {
-        b->seen = nullptr;
-        return bail(fail(PF_E_NOMEM, "hipHostMalloc of the step variant report failed"));
-    }
-    b->seen[0] = b->seen[1] = 0ull;
-    if (const char* sv = getenv("CUPF_STEP_VARIANT")) b->variant_force = atoi(sv) ? 1 : 0;
     *out = b;
     return PF_OK;
 }

@@ -3,11 +3,11 @@
 
 namespace cupf {
 
-hipError_t launch_step_k5_g7(const StepArgs& a, hipStream_t stream, const EdgeLaunch* edge,
+hipError_t launch_step_k5_g7(const StepArgs& a, hipStream_t stream,
                              hipEvent_t e0, hipEvent_t e1, hipEvent_t e2, hipEvent_t e3,
                              bool planned, const StepArgs* next)
 {
-    return launch_step_t<5, false>(a, stream, edge, e0, e1, e2, e3, planned, next);
+    return launch_step_t<5, false>(a, stream, e0, e1, e2, e3, planned, next);
 }
 
 hipError_t launch_batch_k5_g7(const BatchArgs& b, hipStream_t stream)
