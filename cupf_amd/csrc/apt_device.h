@@ -430,17 +430,69 @@ constexpr int kTX = 64, kTY = 4;
 __device__ __forceinline__ int act_tile_x(int i) { return (i - 1) / kTX; }
 __device__ __forceinline__ int act_tile_y(int j) { return (j - 1) / kTY; }
 
-// Append the overflowed lanes of a wave to the fix-up list (one atomic per wave).
-__device__ __forceinline__ void fixup_append(const StepArgs& a, int ovf, unsigned point)
+// Append the overflowed lanes of a wave to its row plane's segment of the
+// fix-up list (one atomic per wave); row: its index (capacity.h),
+// wave-uniform.
+__device__ __forceinline__ void fixup_append(const StepArgs& a, int ovf, unsigned point, int row)
 {
     const unsigned long long m = __ballot(ovf);
     if (m == 0ull) return;
     const int lane = threadIdx.x & 63;
     const int leader = __ffsll((long long)m) - 1;
+    const int seg = row & (a.fix_segs - 1);
     unsigned base = 0;
-    if (lane == leader) base = atomicAdd(a.fix_count, (unsigned)__popcll(m));
+    if (lane == leader) base = atomicAdd(a.fix_count + kLineWords * seg, (unsigned)__popcll(m));
     base = __shfl(base, leader);
-    if (ovf) a.fix_list[base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = point;
+    if (ovf) a.fix_list[(unsigned)(seg * a.fix_cap) + base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = point;
+}
+
+// Counts of m fix-up segments (count(q), m <= kMaxBatch) into s_cnt and the
+// exclusive prefix of the wave units they make (POINTS entries each) into
+// s_pre[0 .. m]; every thread of a kFixLanes workgroup calls it.  Returns the
+// number of units.
+template <int POINTS, class Count>
+__device__ __forceinline__ unsigned fixup_units(int m, Count&& count, unsigned* s_pre, unsigned* s_cnt,
+                                                unsigned* s_wave)
+{
+    const int per = (m + kFixLanes - 1) / kFixLanes;
+    const int q0 = min((int)threadIdx.x * per, m), q1 = min(q0 + per, m);
+    unsigned own = 0u;
+    for (int q = q0; q < q1; ++q) {
+        const unsigned c = count(q);
+        s_cnt[q] = c;
+        own += (c + POINTS - 1) / POINTS;
+    }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    unsigned x = own;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const unsigned v = __shfl_up(x, d);
+        x += lane >= d ? v : 0u;
+    }
+    if (lane == 63) s_wave[w] = x;
+    __syncthreads();
+    unsigned run = x - own;
+#pragma unroll
+    for (int u = 0; u < kFixLanes / 64; ++u) run += u < w ? s_wave[u] : 0u;
+    for (int q = q0; q < q1; ++q) {
+        s_pre[q] = run;
+        run += (s_cnt[q] + POINTS - 1) / POINTS;
+    }
+    if (threadIdx.x == kFixLanes - 1) s_pre[m] = run;
+    __syncthreads();
+    return s_pre[m];
+}
+
+// Last segment whose units start at or before u (wave-uniform).
+__device__ __forceinline__ int fixup_find(const unsigned* s_pre, int m, unsigned u)
+{
+    int lo = 0, hi = m - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (s_pre[mid] <= u) lo = mid;
+        else hi = mid - 1;
+    }
+    return __builtin_amdgcn_readfirstlane(lo);
 }
 
 // The plan kernels' unit of work: wave gw of a simulation covers z-chunk
@@ -548,7 +600,7 @@ __device__ __forceinline__ void plan_block(const StepArgs& a, int pb)
     const int g = pb * kBlock + (int)threadIdx.x;
     // the counter set of the step after this one (last used two steps
     // before, whose fix-up has finished) starts from zero
-    if (g < 4) a.cnt_next[g] = 0u;
+    if (g <= kSpread) a.cnt_next[kLineWords * g] = 0u;  // the list segments' and the work list's
     const int gw = g >> 6;  // wave-uniform
     const int lane = threadIdx.x & 63;
     bool put = false;

@@ -25,6 +25,20 @@ constexpr float kKillf = -0.9999f;
 // per wave.
 constexpr int kPartialMin = 16;
 
+// Atomics of a whole grid on one address go through one at a time, ~17 ns each
+// (the start-up of a 256x256x512 simulation hands over points from ~25,000 row
+// planes of a 400 us step), so the fix-up list and the overflow count are
+// spread over kSpread counters on cache lines of their own: by row for the
+// list, whose segments hold every point of their rows.  (One counter each
+// before; step kernel at step 6: 400 -> 266 us; 64^3 at step 10 45 -> 34; the
+// 27-point gather at 96x96x128 115 -> 80.)
+constexpr int kSpread = 64;
+constexpr int kLineWords = 32;             // 128 bytes
+constexpr int kWlWord = kSpread * kLineWords;           // a set's work-list counter
+constexpr int kSetWords = (kSpread + 1) * kLineWords;   // a step's counter set
+// Counters over all members of a batch (kMaxBatch at most).
+constexpr int kBatchSpread = 256;
+
 // Everything one APT step launch reads.  Passed by value (kernel argument
 // segment -> SGPRs), so no constant-memory upload per step.
 struct StepArgs {
@@ -37,10 +51,15 @@ struct StepArgs {
     const float* z;
     const float* R12;      // orientation rows, 12 floats per grain (9 used)
     const float* psi_mac;  // type-4 thermal field
-    unsigned long long* overflow;  // count of points with > K distinct ids
-    unsigned* fix_list;    // interior points left to the fix-up pass (capacity: interior points)
-    // Counters of this step: fix_count[0] entries in fix_list; wl_count (below)
-    // points into the same 4-word set.  Steps take three sets in turn;
+    unsigned long long* overflow;  // points with > K distinct ids: the sum of kSpread counts,
+                                   // kLineWords / 2 apart
+    // Interior points left to the fix-up pass: fix_segs segments (a power of
+    // two) of fix_cap entries; a row plane's points go to the segment of its
+    // index (capacity.h).
+    unsigned* fix_list;
+    int fix_segs, fix_cap;
+    // Counters of this step: fix_count[kLineWords * s] entries in segment s;
+    // wl_count (below) points into the same set (kSetWords).  Steps take three sets in turn;
     // cnt_next is the next step's, cleared by this step's plan kernel (its
     // last user, two steps back, has finished; this step's fix-up, which may
     // run beside the next step's plan, keeps its own).
@@ -65,7 +84,7 @@ struct StepArgs {
     unsigned* row_dst;
     // Work of one step: the strip's units (see apt_step), then the tile chunks
     // listed by the plan kernel: wl_item = z chunk * items_chunk + tile, with
-    // the chunk's plane mask, wl_count[0] of them (word 2 of the counter set).
+    // the chunk's plane mask, wl_count[0] of them (word kWlWord of the counter set).
     int* wl_item;
     unsigned long long* wl_need;
     unsigned* wl_count;
@@ -104,7 +123,7 @@ struct BatchSim {
     int cur;               // source buffer of the next step
     int step;              // index s of the next step (t = (float)s*dt*tau0)
     int parity;            // counter set of the next step (0..2, in turn)
-    unsigned* cnt;         // the simulation's three 4-word counter sets
+    unsigned* cnt;         // the simulation's three counter sets
     float tau0;
     int plan_base;         // first plan wave of this simulation
     int strip_base;        // first strip unit of this simulation
@@ -135,9 +154,8 @@ __host__ __device__ inline int strip_waves(int ex, int fny)
 constexpr int kMaxBatch = 1024;
 
 // A batched step over n simulations sharing K and the gather variant.  The
-// work list holds tile chunks of every simulation; cnt holds two 4-word
-// counter sets ([0] chunks listed) used by alternate steps, selected by
-// cnt[8].
+// work list holds tile chunks of every simulation; cnt holds the chunks listed
+// by alternate steps (words 0 and 4), selected by cnt[8].
 struct BatchArgs {
     BatchSim* sims;
     int n;
@@ -147,6 +165,7 @@ struct BatchArgs {
     int* wl_item;
     unsigned long long* wl_need;
     unsigned* cnt;
+    int fix_segs;          // fix-up list segments of each simulation
     int step_blocks;
     int fix_blocks;        // workgroups of the batched fix-up kernel
 };

@@ -61,24 +61,25 @@ __global__ __launch_bounds__(kBatchPlanBlock) void batch_plan(BatchArgs b)
 // host does between single launches (buffers swap, the destination takes the
 // step's epoch, the step index and t advance, the next of the member's three
 // counter sets is cleared for the next step); the batch's own two list
-// counter sets alternate.
+// counters alternate.  One wave per simulation.
 __global__ __launch_bounds__(64) void batch_advance(BatchArgs b)
 {
-    const int s = blockIdx.x * 64 + threadIdx.x;
-    if (s == 0) {
+    BatchSim& m = b.sims[blockIdx.x];
+    const int parity = (m.parity + 1) % 3;
+    unsigned* next = m.cnt + kSetWords * parity;
+    next[kLineWords * threadIdx.x] = 0u;
+    static_assert(kSpread == 64, "one counter per lane");
+    if (threadIdx.x != 0) return;
+    next[kWlWord] = 0u;
+    if (blockIdx.x == 0) {
         const unsigned p = b.cnt[8];
         b.cnt[4 * (1 - p)] = 0u;
         b.cnt[8] = 1u - p;
     }
-    if (s >= b.n) return;
-    BatchSim& m = b.sims[s];
     m.ep[1 - m.cur] = m.a.ep_new;
     m.cur = 1 - m.cur;
     m.step += 1;
-    m.parity = (m.parity + 1) % 3;
-    unsigned* next = m.cnt + 4 * m.parity;
-    next[0] = 0u;
-    next[2] = 0u;
+    m.parity = parity;
     StepArgs& a = m.a;
     a.ph = m.ph[m.cur];
     a.arg = m.arg[m.cur];
@@ -93,8 +94,8 @@ __global__ __launch_bounds__(64) void batch_advance(BatchArgs b)
     m.ep_ctr += 1u;
     a.ep_new = m.ep_ctr;
     a.fix_count = next;
-    a.cnt_next = m.cnt + 4 * ((m.parity + 1) % 3);
-    a.wl_count = next + 2;
+    a.cnt_next = m.cnt + kSetWords * ((parity + 1) % 3);
+    a.wl_count = next + kWlWord;
     // t_cur_step = (2*kt+1)*dt*tau0 in float (3DgrainMPI/APTPhaseField.cu:863,919)
     a.t = (float)m.step * a.dt * m.tau0;
 }
@@ -416,7 +417,7 @@ hipError_t launch_batch_plan(const BatchArgs& b, hipStream_t stream)
 
 hipError_t launch_batch_advance(const BatchArgs& b, hipStream_t stream)
 {
-    hipLaunchKernelGGL(batch_advance, dim3(max(1, cdiv(b.n, 64))), dim3(64), 0, stream, b);
+    hipLaunchKernelGGL(batch_advance, dim3(b.n), dim3(64), 0, stream, b);
     return hipGetLastError();
 }
 

@@ -479,7 +479,13 @@ __device__ __forceinline__ void wide_plane(const StepArgs& a, const RowLane& r, 
         }
     }
     row_mark<K>(a, r, k, tx, nn);
-    fixup_append(a, ovf ? 1 : 0, (unsigned)t.zC + (t.c >> 2));
+    if (__ballot(ovf) != 0ull) {
+        const int j = __builtin_amdgcn_readfirstlane(r.j);  // the row, or a strip wave's first
+        const int ex = strip_width(a.fnx, a.tiles_x);
+        const int row = tx >= 0 ? (k * a.fny + j) * a.tiles_x + tx
+                                : a.fnz * a.fny * a.tiles_x + k * strip_waves(ex, a.fny) + (j - 1) / (64 / max(ex, 1));
+        fixup_append(a, ovf ? 1 : 0, (unsigned)t.zC + (t.c >> 2), row);
+    }
 }
 
 template <int K, bool G27>

@@ -33,4 +33,23 @@ inline long long worst_fix_entries(int fnx, int fny, int fnz)
     return (long long)(fnx - 2) * (fny - 2) * (fnz - 2);
 }
 
+// Waves of the +x strip of one plane (its columns, 64 / width rows to a wave).
+inline int cap_strip_waves(int fnx, int fny, int partial_min)
+{
+    const int ex = (fnx - 2) - 64 * cap_tiles_x(fnx, partial_min);
+    return ex > 0 ? (fny - 2 + 64 / ex - 1) / (64 / ex) : 0;
+}
+
+// Entries of one of `segs` (a power of two up to 64) segments of that list:
+// the points of a row plane (64 at most) go to the segment of its index, the
+// tiles' rows first, (k * fny + j) * tiles + tile, then the strip's waves,
+// k * waves + wave.  A quarter as many segments hold four of the full split's
+// each, so every split fits the full one's list.
+inline long long fix_segment_cap(int fnx, int fny, int fnz, int partial_min, int segs)
+{
+    const long long rows = (long long)cap_tiles_x(fnx, partial_min) * fny * fnz +
+                           (long long)cap_strip_waves(fnx, fny, partial_min) * fnz;
+    return (rows + 63) / 64 * 64 * (64 / segs);
+}
+
 }  // namespace cupf

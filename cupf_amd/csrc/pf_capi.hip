@@ -39,9 +39,9 @@ struct pf_ctx {
     float* phi0 = nullptr;          // initial single field (phi_old of the reference)
     float* phi = nullptr;           // collect target
     int* alpha = nullptr;           // collect target / initial alpha (alpha_m)
-    unsigned long long* counters = nullptr;  // [0] overflow points, [1] nucleation events
+    unsigned long long* counters = nullptr;  // overflow counts (kSpread lines), then nucleation events
     unsigned* fix_list = nullptr;   // overflow fix-up list, one entry per interior point
-    unsigned* fix_count = nullptr;  // three 4-word counter sets, used by steps in turn
+    unsigned* fix_count = nullptr;  // three counter sets (kSetWords each), used by steps in turn
     long long* sums = nullptr;
     std::vector<long long> h_sums;
     int* alpha_full = nullptr;
@@ -145,6 +145,9 @@ int ctx_check(pf_ctx* c)
     return PF_OK;
 }
 
+// Words of the spread overflow counts, ahead of the nucleation events.
+constexpr int kOverflowWords = kSpread * kLineWords / 2;
+
 int buf_index(pf_ctx* c, int which) { return which == 0 ? c->cur : 1 - c->cur; }
 
 StepArgs make_step_args(pf_ctx* c, int src, float t, int use_iuc)
@@ -162,15 +165,17 @@ StepArgs make_step_args(pf_ctx* c, int src, float t, int use_iuc)
     a.psi_mac = c->psi_mac;
     a.overflow = c->counters;
     a.fix_list = c->fix_list;
+    a.fix_segs = kSpread;
+    a.fix_cap = (int)fix_segment_cap(p.fnx, p.fny, p.fnz, kPartialMin, kSpread);
     {
         // three sets in turn (advanced once the launch succeeded): this step's
         // plan clears the next step's set, whose last user (two steps back) has
         // finished; the next step's plan may run beside this step's fix-up
         // (apt_fixplan), so it must not clear this step's set
         const int set = (int)(c->nlaunch % 3ull);
-        a.fix_count = c->fix_count + 4 * set;
-        a.cnt_next = c->fix_count + 4 * ((set + 1) % 3);
-        a.wl_count = a.fix_count + 2;
+        a.fix_count = c->fix_count + kSetWords * set;
+        a.cnt_next = c->fix_count + kSetWords * ((set + 1) % 3);
+        a.wl_count = a.fix_count + kWlWord;
     }
     a.fnx = p.fnx;
     a.fny = p.fny;
@@ -247,7 +252,7 @@ int nucl_launch(pf_ctx* c, float t, float dt_nuc, int use_iuc)
     a.z = c->z;
     a.T3d = c->T3d;
     a.ball = c->ball;
-    a.events = c->counters + 1;
+    a.events = c->counters + kOverflowWords;
     a.act = c->act[c->cur];
     a.row = c->row[c->cur];
     a.ep = c->ep[c->cur];
@@ -350,7 +355,8 @@ struct pf_batch {
     int* wl_sim = nullptr;
     int* wl_item = nullptr;
     unsigned long long* wl_need = nullptr;
-    unsigned* cnt = nullptr;        // 2 x 4 list counters, parity word
+    unsigned* cnt = nullptr;        // two list counters (words 0, 4), parity word 8
+    int fix_segs = 1;               // fix-up list segments of each member
     size_t wl_cap = 0;
     // hipGraph of kGraphSteps batched steps, captured for one kchunk
     hipGraph_t graph = nullptr;
@@ -391,6 +397,8 @@ int batch_upload(pf_batch* b, const std::vector<int>& first_step, int use_iuc, B
         m.a.nzchunk = (p.fnz - 2 + b->kchunk - 1) / b->kchunk;
         m.a.step_blocks = b->step_blocks;
         m.a.fix_blocks = b->fix_blocks;
+        m.a.fix_segs = b->fix_segs;
+        m.a.fix_cap = (int)fix_segment_cap(p.fnx, p.fny, p.fnz, kPartialMin, b->fix_segs);
         for (int q = 0; q < 2; ++q) {
             m.ph[q] = c->ph[q];
             m.arg[q] = c->arg[q];
@@ -419,6 +427,7 @@ int batch_upload(pf_batch* b, const std::vector<int>& first_step, int use_iuc, B
     ba.wl_item = b->wl_item;
     ba.wl_need = b->wl_need;
     ba.cnt = b->cnt;
+    ba.fix_segs = b->fix_segs;
     ba.step_blocks = b->step_blocks;
     ba.fix_blocks = b->fix_blocks;
     return PF_OK;
@@ -579,9 +588,9 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
     if ((rc = dalloc(&c->x, p.fnx)) || (rc = dalloc(&c->y, p.fny)) || (rc = dalloc(&c->z, p.fnz)) ||
         (rc = dalloc(&c->zbuf, p.fnz)) || (rc = dalloc(&c->phi0, (size_t)L)) ||
         (rc = dalloc(&c->phi, (size_t)L)) || (rc = dalloc(&c->alpha, (size_t)L)) ||
-        (rc = dalloc(&c->counters, 2)) || (rc = dalloc(&c->sums, p.fnz)) ||
-        (rc = dalloc(&c->fix_list, (size_t)(c->fix_alloc = (long long)(p.fnx - 2) * (p.fny - 2) * (p.fnz - 2)))) ||
-        (rc = dalloc(&c->fix_count, 12)) ||
+        (rc = dalloc(&c->counters, kOverflowWords + 1)) || (rc = dalloc(&c->sums, p.fnz)) ||
+        (rc = dalloc(&c->fix_list, (size_t)(c->fix_alloc = kSpread * fix_segment_cap(p.fnx, p.fny, p.fnz, kPartialMin, kSpread)))) ||
+        (rc = dalloc(&c->fix_count, 3 * kSetWords)) ||
         (rc = dalloc(&c->act[0], (size_t)c->ntiles * p.fnz)) ||
         (rc = dalloc(&c->act[1], (size_t)c->ntiles * p.fnz)) ||
         (rc = dalloc(&c->row[0], row_words(p))) || (rc = dalloc(&c->row[1], row_words(p))) ||
@@ -594,8 +603,8 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
             hipMemsetAsync(c->arg[b], 0xFF, nst * sizeof(int), c->stream) != hipSuccess)
             return bail(fail(PF_E_HIP, "initial fill failed"));
     }
-    if (hipMemsetAsync(c->counters, 0, 2 * sizeof(unsigned long long), c->stream) != hipSuccess ||
-        hipMemsetAsync(c->fix_count, 0, 12 * sizeof(unsigned), c->stream) != hipSuccess ||
+    if (hipMemsetAsync(c->counters, 0, (kOverflowWords + 1) * sizeof(unsigned long long), c->stream) != hipSuccess ||
+        hipMemsetAsync(c->fix_count, 0, 3 * kSetWords * sizeof(unsigned), c->stream) != hipSuccess ||
         hipMemsetAsync(c->alpha, 0, L * sizeof(int), c->stream) != hipSuccess ||
         hipMemsetAsync(c->act[0], 0, (size_t)c->ntiles * p.fnz * sizeof(unsigned), c->stream) != hipSuccess ||
         hipMemsetAsync(c->act[1], 0, (size_t)c->ntiles * p.fnz * sizeof(unsigned), c->stream) != hipSuccess ||
@@ -777,7 +786,8 @@ static int check_capacity(const pf_ctx* c)
     const pf_params& p = c->p;
     const long long items = worst_list_items(p.fnx, p.fny, p.fnz, c->kchunk, kPartialMin);
     if ((long long)c->nzchunk * c->items_chunk != items || items > c->wl_alloc ||
-        worst_fix_entries(p.fnx, p.fny, p.fnz) > c->fix_alloc)
+        worst_fix_entries(p.fnx, p.fny, p.fnz) > c->fix_alloc ||
+        kSpread * fix_segment_cap(p.fnx, p.fny, p.fnz, kPartialMin, kSpread) > c->fix_alloc)
         return fail(PF_E_STATE, "work list capacity below its worst case (" + std::to_string(items) +
                                     " chunks, " + std::to_string(c->wl_alloc) + " allocated)");
     return PF_OK;
@@ -1225,7 +1235,7 @@ int pf_nucl_events(pf_ctx* c, long long* events)
     int rc = ctx_check(c);
     if (rc) return rc;
     unsigned long long v = 0;
-    HIPCHK(hipMemcpyAsync(&v, c->counters + 1, sizeof(v), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(&v, c->counters + kOverflowWords, sizeof(v), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     if (events) *events = (long long)v;
     return PF_OK;
@@ -1235,9 +1245,10 @@ int pf_overflow_count(pf_ctx* c, long long* count)
 {
     int rc = ctx_check(c);
     if (rc) return rc;
-    unsigned long long v = 0;
-    HIPCHK(hipMemcpyAsync(&v, c->counters, sizeof(v), hipMemcpyDeviceToHost, c->stream));
+    unsigned long long h[kOverflowWords], v = 0;
+    HIPCHK(hipMemcpyAsync(h, c->counters, sizeof(h), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    for (int q = 0; q < kSpread; ++q) v += h[kLineWords / 2 * q];
     if (count) *count = (long long)v;
     return PF_OK;
 }
@@ -1323,6 +1334,7 @@ int pf_batch_create(pf_ctx* const* ctxs, int n, pf_batch** out)
         if (v >= pf_batch::kMinChunk && v <= 61) b->kchunk = v;
     }
     b->step_blocks = batch_kernel_slots(b->K, b->g27, b->device);
+    while (b->fix_segs < kSpread && 2 * b->fix_segs * n <= kBatchSpread) b->fix_segs *= 2;
     // 2 fix-up workgroups per CU (3.60 s for the 64-simulation ensemble, against 3.63-3.65 s
     // with the 4 or 6 per CU that fit)
     {

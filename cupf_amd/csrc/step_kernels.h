@@ -41,9 +41,10 @@ __global__ __launch_bounds__(kRowLanes, 4) void apt_step(StepArgs)
     const unsigned ns = (unsigned)(wseg * a.nzchunk);
     const unsigned n = ns + 4u * __atomic_load_n(a.wl_count, __ATOMIC_RELAXED);
     const unsigned W = gridDim.x;
+    const unsigned place = row_place(W);
     unsigned nres = 0u;  // overflowed points settled here
 #pragma unroll 1
-    for (unsigned u = row_place(W); u < n; u += W) {
+    for (unsigned u = place; u < n; u += W) {
         const StepArgs& b = *args_ref(args);
         RowUnit w;
         if (u < ns) {
@@ -54,7 +55,8 @@ __global__ __launch_bounds__(kRowLanes, 4) void apt_step(StepArgs)
         }
         row_unit<K, G27>(args, w, nres);
     }
-    if (threadIdx.x == 0 && nres) atomicAdd(a.overflow, (unsigned long long)nres);
+    if (threadIdx.x == 0 && nres)
+        atomicAdd(a.overflow + kLineWords / 2 * (place % kSpread), (unsigned long long)nres);
 }
 
 // Fix-up pass for the points of the last apt_step launch whose neighbourhood
@@ -64,22 +66,29 @@ __global__ __launch_bounds__(kRowLanes, 4) void apt_step(StepArgs)
 template <int K, bool G27>
 __device__ __forceinline__ void fixup_run(const StepArgs& a, int blk, int nblk)
 {
-    const unsigned n = __atomic_load_n(a.fix_count, __ATOMIC_RELAXED);
-    if (n == 0u) return;
-    if (blk == 0 && threadIdx.x == 0) atomicAdd(a.overflow, (unsigned long long)n);
-    const float a_s = 1.0f + 3.0f * a.kin_delta;
-    const float epsv = -4.0f * a.kin_delta / a_s;
     using F = FixGroup<G27>;
     __shared__ unsigned s_fix[(kFixLanes / F::kLanes) * kFixStride];
+    __shared__ unsigned s_pre[kSpread + 1], s_cnt[kSpread], s_wave[kFixLanes / 64];
+    const unsigned units = fixup_units<F::kPoints>(
+        kSpread, [&](int q) { return __atomic_load_n(a.fix_count + kLineWords * q, __ATOMIC_RELAXED); }, s_pre,
+        s_cnt, s_wave);
+    if (units == 0u) return;
+    if (blk == 0 && threadIdx.x < kSpread && s_cnt[threadIdx.x])
+        atomicAdd(a.overflow + kLineWords / 2 * threadIdx.x, (unsigned long long)s_cnt[threadIdx.x]);
+    const float a_s = 1.0f + 3.0f * a.kin_delta;
+    const float epsv = -4.0f * a.kin_delta / a_s;
     const int l = threadIdx.x & (F::kLanes - 1), grp = threadIdx.x / F::kLanes;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     // wave units of kPoints entries, the first of every workgroup before the
     // second of any, so a short list is spread over the CUs
 #pragma unroll 1
-    for (unsigned u = (unsigned)(w * nblk + blk); u * F::kPoints < n; u += (unsigned)(nblk * (kFixLanes / 64))) {
-        const unsigned e = u * F::kPoints + (unsigned)(grp & (F::kPoints - 1));
-        const bool on = e < n;
-        fixup_group<K, G27>(a, a.fix_list[on ? e : u * F::kPoints], on, l, s_fix + grp * kFixStride, a_s, epsv);
+    for (unsigned u = (unsigned)(w * nblk + blk); u < units; u += (unsigned)(nblk * (kFixLanes / 64))) {
+        const int seg = fixup_find(s_pre, kSpread, u);
+        const unsigned e0 = (u - s_pre[seg]) * F::kPoints;
+        const unsigned e = e0 + (unsigned)(grp & (F::kPoints - 1));
+        const bool on = e < s_cnt[seg];
+        const unsigned* list = a.fix_list + (unsigned)(seg * a.fix_cap);
+        fixup_group<K, G27>(a, list[on ? e : e0], on, l, s_fix + grp * kFixStride, a_s, epsv);
     }
 }
 
@@ -138,54 +147,47 @@ __global__ __launch_bounds__(kRowLanes, 4) void batch_step(BatchArgs b)
             w = tile_unit(*(const StepArgs*)&sims[sim].a, b.wl_item[e], b.wl_need[e], (int)((u - ns) & 3u));
         }
         row_unit<K, G27>((CArgs*)&sims[sim].a, w, nres);
-        if (threadIdx.x == 0 && nres) atomicAdd(sims[sim].a.overflow, (unsigned long long)nres);
+        if (threadIdx.x == 0 && nres)
+            atomicAdd(sims[sim].a.overflow + kLineWords / 2 * (u % kSpread), (unsigned long long)nres);
     }
 }
 
-// Batched fix-up: the overflow lists of all simulations form one index space
-// (prefix sums of their lengths, in LDS) that the grid strides over, so long
-// and short lists alike are spread over every workgroup.
+// Batched fix-up: the list segments of all simulations (fix_segs each) form
+// one index space of wave units (prefix sums in LDS) that the grid strides
+// over, so long and short lists alike are spread over every workgroup.
 template <int K, bool G27>
 __global__ __launch_bounds__(kFixLanes) void batch_fixup(BatchArgs b)
 {
     using F = FixGroup<G27>;
     __shared__ unsigned s_fix[(kFixLanes / F::kLanes) * kFixStride];
-    __shared__ unsigned s_pre[kMaxBatch + 1];  // wave units of the simulations before each
-    for (int t = threadIdx.x; t < b.n; t += kFixLanes)
-        s_pre[t + 1] = __atomic_load_n(b.sims[t].a.fix_count, __ATOMIC_RELAXED);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        s_pre[0] = 0u;
-        for (int t = 0; t < b.n; ++t) {
-            const unsigned c = s_pre[t + 1];
-            if (blockIdx.x == 0 && c) atomicAdd(b.sims[t].a.overflow, (unsigned long long)c);
-            s_pre[t + 1] = s_pre[t] + (c + F::kPoints - 1) / F::kPoints;
-        }
-    }
-    __syncthreads();
-    const unsigned units = s_pre[b.n];
-    const int l = threadIdx.x & (F::kLanes - 1), grp = threadIdx.x / F::kLanes;
-    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    __shared__ unsigned s_pre[kMaxBatch + 1], s_cnt[kMaxBatch], s_wave[kFixLanes / 64];
     typedef const __attribute__((address_space(4))) BatchSim CSim;
     const CSim* sims = (const CSim*)b.sims;
+    const int segs = b.fix_segs, m = b.n * segs;
+    const unsigned units = fixup_units<F::kPoints>(
+        m,
+        [&](int q) {
+            return __atomic_load_n(b.sims[q / segs].a.fix_count + kLineWords * (q % segs), __ATOMIC_RELAXED);
+        },
+        s_pre, s_cnt, s_wave);
+    if (blockIdx.x == 0)
+        for (int q = threadIdx.x; q < m; q += kFixLanes)
+            if (s_cnt[q])
+                atomicAdd(b.sims[q / segs].a.overflow + kLineWords / 2 * (q % segs), (unsigned long long)s_cnt[q]);
+    const int l = threadIdx.x & (F::kLanes - 1), grp = threadIdx.x / F::kLanes;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 #pragma unroll 1
     for (unsigned u = (unsigned)(w * (int)gridDim.x + (int)blockIdx.x); u < units;
          u += (unsigned)((int)gridDim.x * (kFixLanes / 64))) {
-        int lo = 0, hi = b.n - 1;  // last simulation whose units start at or before u
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (s_pre[mid] <= u) lo = mid;
-            else hi = mid - 1;
-        }
-        lo = __builtin_amdgcn_readfirstlane(lo);
-        const StepArgs& a = *(const StepArgs*)&sims[lo].a;
-        const unsigned n = __atomic_load_n(a.fix_count, __ATOMIC_RELAXED);
-        const unsigned e0 = (u - s_pre[lo]) * F::kPoints;
+        const int q = fixup_find(s_pre, m, u);
+        const StepArgs& a = *(const StepArgs*)&sims[q / segs].a;
+        const unsigned e0 = (u - s_pre[q]) * F::kPoints;
         const unsigned e = e0 + (unsigned)(grp & (F::kPoints - 1));
         const float a_s = 1.0f + 3.0f * a.kin_delta;
         const float epsv = -4.0f * a.kin_delta / a_s;
-        const bool on = e < n;
-        fixup_group<K, G27>(a, a.fix_list[on ? e : e0], on, l, s_fix + grp * kFixStride, a_s, epsv);
+        const bool on = e < s_cnt[q];
+        const unsigned* list = a.fix_list + (unsigned)(q % segs * a.fix_cap);
+        fixup_group<K, G27>(a, list[on ? e : e0], on, l, s_fix + grp * kFixStride, a_s, epsv);
     }
 }
 
