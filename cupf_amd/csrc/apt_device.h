@@ -430,20 +430,19 @@ constexpr int kTX = 64, kTY = 4;
 __device__ __forceinline__ int act_tile_x(int i) { return (i - 1) / kTX; }
 __device__ __forceinline__ int act_tile_y(int j) { return (j - 1) / kTY; }
 
-// Append the overflowed lanes of a wave to its row plane's segment of the
+// Append the lanes of a wave in m (not 0) to its row plane's segment of the
 // fix-up list (one atomic per wave); row: its index (capacity.h),
 // wave-uniform.
-__device__ __forceinline__ void fixup_append(const StepArgs& a, int ovf, unsigned point, int row)
+__device__ __forceinline__ void fixup_append(const StepArgs& a, unsigned long long m, unsigned point, int row)
 {
-    const unsigned long long m = __ballot(ovf);
-    if (m == 0ull) return;
     const int lane = threadIdx.x & 63;
     const int leader = __ffsll((long long)m) - 1;
     const int seg = row & (a.fix_segs - 1);
     unsigned base = 0;
     if (lane == leader) base = atomicAdd(a.fix_count + kLineWords * seg, (unsigned)__popcll(m));
     base = __shfl(base, leader);
-    if (ovf) a.fix_list[(unsigned)(seg * a.fix_cap) + base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = point;
+    if ((m >> lane) & 1ull)
+        a.fix_list[(unsigned)(seg * a.fix_cap) + base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = point;
 }
 
 // Counts of m fix-up segments (count(q), m <= kMaxBatch) into s_cnt and the

@@ -111,22 +111,21 @@ __device__ __forceinline__ int wave_max(int v)
     return m;
 }
 
-// Destination maps of one row plane: nn filled slots per lane (K where the
-// fix-up will fill them).  tx >= 0: the whole wave is one row of column tile
-// tx; otherwise (a strip) each lane marks its own row.
-template <int K>
-__device__ __forceinline__ void row_mark(const StepArgs& a, const RowLane& r, int k, int tx, int nn)
+// Destination maps of one row plane, m filled slots (K where the fix-up will
+// fill them): the row of column tile tx, or (a strip) each lane's own row.
+__device__ __forceinline__ void row_mark_tile(const StepArgs& a, const RowLane& r, int k, int tx, int m)
 {
-    if (tx >= 0) {
-        const int m = wave_max<K>(nn);
-        if (m > 0 && threadIdx.x == 0) {
-            a.act_dst[k * a.ntiles + act_tile_y(r.j) * a.ntx + tx] = a.ep_new;
-            a.row_dst[(k * a.fny + r.j) * a.ntx + tx] = a.ep_new << 4 | (unsigned)m;
-        }
-    } else if (nn > 0) {
+    if (m > 0 && threadIdx.x == 0) {
+        a.act_dst[k * a.ntiles + act_tile_y(r.j) * a.ntx + tx] = a.ep_new;
+        a.row_dst[(k * a.fny + r.j) * a.ntx + tx] = a.ep_new << 4 | (unsigned)m;
+    }
+}
+__device__ __forceinline__ void row_mark_strip(const StepArgs& a, const RowLane& r, int k, int m)
+{
+    if (m > 0) {
         const int x = act_tile_x(r.i);
         a.act_dst[k * a.ntiles + act_tile_y(r.j) * a.ntx + x] = a.ep_new;
-        atomicMax(a.row_dst + (k * a.fny + r.j) * a.ntx + x, a.ep_new << 4 | (unsigned)nn);
+        atomicMax(a.row_dst + (k * a.fny + r.j) * a.ntx + x, a.ep_new << 4 | (unsigned)m);
     }
 }
 
@@ -140,128 +139,24 @@ __device__ __forceinline__ void row_store(const StepArgs& a, const RowStencil& t
     }
 }
 
-// List positions of the narrow path: a row bounded by P <= 4 slots hardly
-// ever gathers a fifth id (0.2 % of the rows of a grown 256x256x512 state).
-constexpr int kNarrowList = 4;
-
-// One plane of a row whose neighbourhood holds nothing above slot P - 1
-// (7-point gather).  False if some lane gathers more than kNarrowList ids:
-// nothing is written then and the wave takes the general path.
-template <int K, int P>
-__device__ __forceinline__ bool narrow_plane(const StepArgs& a, const RowLane& r, int k, int tx, int D,
-                                             float xi, float yj, float a_s, float epsv)
-{
-    constexpr int M = kNarrowList;
-    const RowStencil t = row_stencil(a, r, k);
-    int id[7][P];
-    float ph[7][P];
-#pragma unroll
-    for (int s = 0; s < 7; ++s) {
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const long long b = (long long)p * a.L + t.plane(s);
-            id[s][p] = at_off(a.arg + b, t.off(s));
-            ph[s][p] = at_off(a.ph + b, t.off(s));
-        }
-    }
-    int la[M];
-    float v[7][M];
-#pragma unroll
-    for (int q = 0; q < M; ++q) {
-        la[q] = kNoKey;  // never a grain id
-#pragma unroll
-        for (int s = 0; s < 7; ++s) v[s][q] = -1.0f;
-    }
-    int n = 0;
-    bool more = false;
-#pragma unroll
-    for (int s = 0; s < 7; ++s) {
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const int x = id[s][p];
-            bool hit = x == -1;
-#pragma unroll
-            for (int q = 0; q < M; ++q) {
-                const bool e = la[q] == x;
-                v[s][q] = e ? ph[s][p] : v[s][q];
-                hit = hit | e;
-            }
-            if (__ballot(!hit) != 0ull) {  // some lane meets a new id
-#pragma unroll
-                for (int q = 0; q < M; ++q) {
-                    const bool w = !hit & (n == q);
-                    la[q] = w ? x : la[q];
-                    v[s][q] = w ? ph[s][p] : v[s][q];
-                }
-                more = more | (!hit & (n >= M));
-                n += !hit ? 1 : 0;
-            }
-        }
-    }
-    if (__ballot(more) != 0ull) return false;
-    const int nm = wave_max<M>(n);
-    const int nst = max(nm, D);
-    if (nst == 0) return true;
-    bool skip = false;
-    float Up = 0.0f;
-    float rw[M];
-    if (nm > 0) {
-        float T;
-        skip = thermal_Tv(a, xi, yj, a.z[k], T);
-        Up = T / a.L_cp;
-#pragma unroll
-        for (int q = 0; q < M; ++q) {
-            const float w = v[3][q] + 1.0f;
-            rw[q] = 0.25f * w * w;
-        }
-    }
-    // every slot's orientation rows in one round trip; a lane without a
-    // gradient needs none (its anisotropy is 1 under any rotation)
-    Rot m[M];
-#pragma unroll
-    for (int q = 0; q < M; ++q) {
-        if (q < nm) {
-            const bool flat = v[4][q] == v[2][q] && v[5][q] == v[1][q] && v[6][q] == v[0][q];
-            m[q] = slot_rot(a, q < n ? la[q] : 0, flat ? -1.0f : v[3][q]);
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < M; ++q) {
-        if (q < nst) {
-            int oid = -1;
-            float oph = -1.0f;
-            if (q < nm) {
-                float repul = 0.0f;  // unfilled slots add exactly +0
-#pragma unroll
-                for (int p = 0; p < M; ++p)
-                    if (p != q) repul += rw[p];
-                const bool in = q < n;
-                const float nv = slot_update_r(a, m[q], v[0][q], v[1][q], v[2][q], v[3][q], v[4][q], v[5][q],
-                                               v[6][q], repul, Up, a_s, epsv);
-                oph = in ? nv : -1.0f;
-                oid = in && !(nv < kKillf) ? la[q] : -1;
-            }
-            row_store(a, t, q, r.on && !(skip && q < n), oid, oph);
-        }
-    }
-#pragma unroll 1
-    for (int q = M; q < nst; ++q) row_store(a, t, q, r.on, -1, -1.0f);
-    if (nm > 0) row_mark<M>(a, r, k, tx, r.on ? n : 0);
-    return true;
-}
-
 // Gather of one row: ids in first-appearance order and, by list position and
 // stencil row (D,B,L,C,R,T,U), the phi of the last entry holding the id (-1
 // where the row has none).  Static registers throughout: an entry is compared
 // with every list position and its phi selected into each.
+// Which lanes have position q filled is a wave mask in scalar registers: a new
+// id's lanes then find their free position with scalar ands, and only the
+// positions that some of them take cost vector work (a new id takes 2-3 of the
+// 8 over a wave; with a count per lane every new id went through all 8).
 template <int K>
 struct RowList {
     int la[K];
     float v[7][K];
-    int n;
-    float outside;  // largest phi of an entry whose id found no room
-    bool ovf;
+    unsigned long long filled[K];  // lanes whose list reaches position q
+    unsigned long long ovf;        // lanes with more ids than positions
+    float outside;                 // largest phi of an entry whose id found no room
 };
+
+__device__ __forceinline__ bool in_mask(unsigned long long m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
 template <int K>
 __device__ __forceinline__ void list_init(RowList<K>& g)
@@ -269,12 +164,12 @@ __device__ __forceinline__ void list_init(RowList<K>& g)
 #pragma unroll
     for (int q = 0; q < K; ++q) {
         g.la[q] = kNoKey;  // never a grain id
+        g.filled[q] = 0ull;
 #pragma unroll
         for (int s = 0; s < 7; ++s) g.v[s][q] = -1.0f;
     }
-    g.n = 0;
     g.outside = -__builtin_huge_valf();
-    g.ovf = false;
+    g.ovf = 0ull;
 }
 
 // Entry (x, f) of a neighbour point; S: its stencil row, -1 for none.
@@ -288,18 +183,43 @@ __device__ __forceinline__ void list_entry(int x, float f, RowList<K>& g)
         if (S >= 0) g.v[S < 0 ? 0 : S][q] = e ? f : g.v[S < 0 ? 0 : S][q];
         hit = hit | e;
     }
-    if (__ballot(!hit) != 0ull) {  // some lane meets a new id
+    unsigned long long left = __ballot(!hit);  // lanes that meet a new id
+    if (left != 0ull) {
 #pragma unroll
         for (int q = 0; q < K; ++q) {
-            const bool w = !hit & (g.n == q);
-            g.la[q] = w ? x : g.la[q];
-            if (S >= 0) g.v[S < 0 ? 0 : S][q] = w ? f : g.v[S < 0 ? 0 : S][q];
+            const unsigned long long t = left & ~g.filled[q];
+            if (t != 0ull) {
+                const bool w = in_mask(t);
+                g.la[q] = w ? x : g.la[q];
+                if (S >= 0) g.v[S < 0 ? 0 : S][q] = w ? f : g.v[S < 0 ? 0 : S][q];
+                g.filled[q] |= t;
+                left &= ~t;
+            }
         }
-        const bool full = !hit & (g.n >= K);
-        g.ovf = g.ovf | full;
-        g.outside = full && f > g.outside ? f : g.outside;
-        g.n += !hit && g.n < K ? 1 : 0;
+        if (left != 0ull) {
+            const bool full = in_mask(left);
+            g.ovf |= left;
+            g.outside = full && f > g.outside ? f : g.outside;
+        }
     }
+}
+
+// Positions filled in any lane of the wave, and in this lane.
+template <int K>
+__device__ __forceinline__ int list_max(const RowList<K>& g)
+{
+    int m = 0;
+#pragma unroll
+    for (int q = 0; q < K; ++q) m += g.filled[q] != 0ull ? 1 : 0;
+    return m;
+}
+template <int K>
+__device__ __forceinline__ int list_len(const RowList<K>& g)
+{
+    int n = 0;
+#pragma unroll
+    for (int q = 0; q < K; ++q) n += in_mask(g.filled[q]) ? 1 : 0;
+    return n;
 }
 
 template <int P>
@@ -343,6 +263,84 @@ __device__ __forceinline__ void entries_list_next(const StepArgs& a, int z, unsi
         e.f[p] = at_off(a.ph + b, o);
         __builtin_amdgcn_sched_barrier(0);
     }
+}
+
+// List positions of the narrow path: a row bounded by P <= 4 slots hardly
+// ever gathers a fifth id (0.2 % of the rows of a grown 256x256x512 state).
+constexpr int kNarrowList = 4;
+
+// One plane of a row whose neighbourhood holds nothing above slot P - 1
+// (7-point gather).  False if some lane gathers more than kNarrowList ids:
+// nothing is written then and the wave takes the general path.
+template <int K, int P>
+__device__ __forceinline__ bool narrow_plane(const StepArgs& a, const RowLane& r, int k, int tx, int D,
+                                             float xi, float yj, float a_s, float epsv)
+{
+    constexpr int M = kNarrowList;
+    const RowStencil t = row_stencil(a, r, k);
+    RowEntries<P> e[7];
+#pragma unroll
+    for (int s = 0; s < 7; ++s) entries_load(a, t.plane(s), t.off(s), e[s]);
+    RowList<M> g;
+    list_init(g);
+    entries_list<M, P, 0>(e[0], g);
+    entries_list<M, P, 1>(e[1], g);
+    entries_list<M, P, 2>(e[2], g);
+    entries_list<M, P, 3>(e[3], g);
+    entries_list<M, P, 4>(e[4], g);
+    entries_list<M, P, 5>(e[5], g);
+    entries_list<M, P, 6>(e[6], g);
+    if (g.ovf != 0ull) return false;
+    const int nm = list_max(g);
+    const int nst = max(nm, D);
+    if (nst == 0) return true;
+    bool skip = false;
+    float Up = 0.0f;
+    float rw[M];
+    if (nm > 0) {
+        float T;
+        skip = thermal_Tv(a, xi, yj, a.z[k], T);
+        Up = T / a.L_cp;
+#pragma unroll
+        for (int q = 0; q < M; ++q) {
+            const float w = g.v[3][q] + 1.0f;
+            rw[q] = 0.25f * w * w;
+        }
+    }
+    // every slot's orientation rows in one round trip; a lane without a
+    // gradient needs none (its anisotropy is 1 under any rotation)
+    Rot m[M];
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        if (q < nm) {
+            const bool flat = g.v[4][q] == g.v[2][q] && g.v[5][q] == g.v[1][q] && g.v[6][q] == g.v[0][q];
+            m[q] = slot_rot(a, in_mask(g.filled[q]) ? g.la[q] : 0, flat ? -1.0f : g.v[3][q]);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        if (q < nst) {
+            int oid = -1;
+            float oph = -1.0f;
+            const bool in = in_mask(g.filled[q]);
+            if (q < nm) {
+                float repul = 0.0f;  // unfilled slots add exactly +0
+#pragma unroll
+                for (int p = 0; p < M; ++p)
+                    if (p != q) repul += rw[p];
+                const float nv = slot_update_r(a, m[q], g.v[0][q], g.v[1][q], g.v[2][q], g.v[3][q], g.v[4][q],
+                                               g.v[5][q], g.v[6][q], repul, Up, a_s, epsv);
+                oph = in ? nv : -1.0f;
+                oid = in && !(nv < kKillf) ? g.la[q] : -1;
+            }
+            row_store(a, t, q, r.on && !(skip && in), oid, oph);
+        }
+    }
+#pragma unroll 1
+    for (int q = M; q < nst; ++q) row_store(a, t, q, r.on, -1, -1.0f);
+    if (tx >= 0) row_mark_tile(a, r, k, tx, nm);
+    else row_mark_strip(a, r, k, r.on ? list_len(g) : 0);
+    return true;
 }
 
 template <int K, bool G27, int P>
@@ -413,17 +411,16 @@ __device__ __forceinline__ void wide_plane(const StepArgs& a, const RowLane& r, 
     if (P <= 4) row_gather<K, G27, 4>(a, t, g);
     else if (K > 6 && P <= 6) row_gather<K, G27, 6>(a, t, g);
     else row_gather<K, G27, K>(a, t, g);
-    if (!r.on) {
-        g.n = 0;
-        g.ovf = false;
-    }
+    const unsigned long long on = __ballot(r.on);
+#pragma unroll
+    for (int q = 0; q < K; ++q) g.filled[q] &= on;
+    g.ovf &= on;
     // An overflowed point whose list ids all reach a phi above every entry
     // that found no room keeps its list: the list is the kept set of the
     // overflow policy, in its order.  (A list id's largest phi is taken over
     // the stencil rows' values; rows without the id count as -1, so a list
     // that does not rise above -1 goes to the fix-up.)
-    if (!G27 && __ballot(g.ovf) != 0ull) {
-        const bool was = g.ovf;
+    if (!G27 && g.ovf != 0ull) {
         float low = __builtin_huge_valf();
 #pragma unroll
         for (int q = 0; q < K; ++q) {
@@ -432,15 +429,14 @@ __device__ __forceinline__ void wide_plane(const StepArgs& a, const RowLane& r, 
             for (int s = 0; s < 7; ++s) best = g.v[s][q] > best ? g.v[s][q] : best;
             low = best < low ? best : low;
         }
-        if (low > -1.0f && g.outside < low) g.ovf = false;
-        nres += (unsigned)__popcll(__ballot(was && !g.ovf));
+        const unsigned long long keep = __ballot(low > -1.0f && g.outside < low) & g.ovf;
+        nres += (unsigned)__popcll(keep);
+        g.ovf &= ~keep;
     }
-    const bool ovf = g.ovf;
-    const int nn = ovf ? K : g.n;
-    const int n = ovf ? 0 : g.n;  // an overflowed point computes nothing here (fix-up kernel)
-    const int nm = wave_max<K>(n);
+    // an overflowed point computes nothing here (fix-up kernel)
+    const bool st = in_mask(on & ~g.ovf);
+    const int nm = list_max(g);
     const int nst = max(nm, D);
-    const bool st = r.on && !ovf;
     bool skip = false;
     float Up = 0.0f;
     float rw[K];
@@ -457,34 +453,37 @@ __device__ __forceinline__ void wide_plane(const StepArgs& a, const RowLane& r, 
     // each slot's orientation rows are requested while the slot before it is
     // computed
     Rot m[2];
-    if (nm > 0) m[0] = slot_rot(a, 0 < n ? g.la[0] : 0, g.v[3][0]);
+    if (nm > 0) m[0] = slot_rot(a, in_mask(g.filled[0]) ? g.la[0] : 0, g.v[3][0]);
 #pragma unroll
     for (int q = 0; q < K; ++q) {
         if (q < nst) {
             int oid = -1;
             float oph = -1.0f;
+            const bool in = in_mask(g.filled[q]);
             if (q < nm) {
-                if (q + 1 < K && q + 1 < nm) m[(q + 1) & 1] = slot_rot(a, q + 1 < n ? g.la[(q + 1) % K] : 0, g.v[3][(q + 1) % K]);
+                if (q + 1 < K && q + 1 < nm)
+                    m[(q + 1) & 1] = slot_rot(a, in_mask(g.filled[(q + 1) % K]) ? g.la[(q + 1) % K] : 0,
+                                              g.v[3][(q + 1) % K]);
                 float repul = 0.0f;  // empty slots add exactly +0
 #pragma unroll
                 for (int p = 0; p < K; ++p)
                     if (p != q) repul += rw[p];
                 const float nv = slot_update_r(a, m[q & 1], g.v[0][q], g.v[1][q], g.v[2][q], g.v[3][q], g.v[4][q],
                                                g.v[5][q], g.v[6][q], repul, Up, a_s, epsv);
-                const bool in = q < n;
                 oph = in ? nv : -1.0f;
                 oid = in && !(nv < kKillf) ? g.la[q] : -1;
             }
-            row_store(a, t, q, st && !(skip && q < n), oid, oph);
+            row_store(a, t, q, st && !(skip && in), oid, oph);
         }
     }
-    row_mark<K>(a, r, k, tx, nn);
-    if (__ballot(ovf) != 0ull) {
+    if (tx >= 0) row_mark_tile(a, r, k, tx, g.ovf != 0ull ? K : nm);
+    else row_mark_strip(a, r, k, in_mask(g.ovf) ? K : list_len(g));
+    if (g.ovf != 0ull) {
         const int j = __builtin_amdgcn_readfirstlane(r.j);  // the row, or a strip wave's first
         const int ex = strip_width(a.fnx, a.tiles_x);
         const int row = tx >= 0 ? (k * a.fny + j) * a.tiles_x + tx
                                 : a.fnz * a.fny * a.tiles_x + k * strip_waves(ex, a.fny) + (j - 1) / (64 / max(ex, 1));
-        fixup_append(a, ovf ? 1 : 0, (unsigned)t.zC + (t.c >> 2), row);
+        fixup_append(a, g.ovf, (unsigned)t.zC + (t.c >> 2), row);
     }
 }
 
