@@ -13,9 +13,9 @@
 // instructions per row plane, 16 waves per CU) and by latency and launches in
 // small grids.  Measured against 64x4 tiles with their halo in a three-plane
 // LDS ring (76 KB, 203 registers: 8 waves per CU, every slot staged), step
-// kernel: 256x256x512 at step 6 450 -> 400 us, at 150 259 -> 177, at 450 87 ->
-// 40, at 1500 128 -> 61; 64^3 at step 10 108 -> 45, at 900 56 -> 23; 32^3 K=5
-// 62 -> 24; a 78 % solid 256^3 window 1340 -> 1120.  The general path with its
+// kernel: 256x256x512 at step 6 450 -> 240 us, at 150 259 -> 156, at 450 87 ->
+// 36, at 1500 128 -> 55; 64^3 at step 10 108 -> 32, at 900 56 -> 21; 32^3 K=5
+// 62 -> 16; a 78 % solid 256^3 window 1340 -> 1000.  The general path with its
 // values in LDS (14 KB a wave, 10 waves per CU) took 1530 us for that window.
 #pragma once
 
@@ -172,23 +172,35 @@ __device__ __forceinline__ void list_init(RowList<K>& g)
     g.ovf = 0ull;
 }
 
-// Entry (x, f) of a neighbour point; S: its stencil row, -1 for none.
-template <int K, int S>
-__device__ __forceinline__ void list_entry(int x, float f, RowList<K>& g)
+// Entry (x, f) of a neighbour point, the (before + 1)th of the gather; S: its
+// stencil row, -1 for none; SKIP: leave at once where no lane has an id (pays
+// with the 7 points, whose entries run up to the largest bound around: 1060 ->
+// 1020 us for a 78 % solid 256^3 window; the 27 points lose 5 %).
+// Only positions that entries so far can have filled are looked at.  Positions
+// fill in order, so a pair whose second one is filled in every lane that meets
+// a new id has nothing to take: one branch per pair (256x256x512 at step 150:
+// 162 us with a branch per position or one for all 8, 157 with pairs).
+template <int K, int S, bool SKIP>
+__device__ __forceinline__ void list_entry(int x, float f, int before, RowList<K>& g)
 {
-    bool hit = x == -1;
+    unsigned long long left = __ballot(x != -1);  // lanes that meet a new id
+    if (SKIP && left == 0ull) return;
 #pragma unroll
     for (int q = 0; q < K; ++q) {
+        if (q >= before) break;
         const bool e = g.la[q] == x;
         if (S >= 0) g.v[S < 0 ? 0 : S][q] = e ? f : g.v[S < 0 ? 0 : S][q];
-        hit = hit | e;
+        left &= ~__ballot(e);
     }
-    unsigned long long left = __ballot(!hit);  // lanes that meet a new id
     if (left != 0ull) {
 #pragma unroll
-        for (int q = 0; q < K; ++q) {
-            const unsigned long long t = left & ~g.filled[q];
-            if (t != 0ull) {
+        for (int b = 0; b < K; b += 2) {
+            if (b > before) break;
+            if ((left & ~g.filled[b + 1 < K ? b + 1 : b]) == 0ull) continue;
+#pragma unroll
+            for (int q = b; q < b + 2 && q < K; ++q) {
+                if (q > before) break;
+                const unsigned long long t = left & ~g.filled[q];
                 const bool w = in_mask(t);
                 g.la[q] = w ? x : g.la[q];
                 if (S >= 0) g.v[S < 0 ? 0 : S][q] = w ? f : g.v[S < 0 ? 0 : S][q];
@@ -196,7 +208,7 @@ __device__ __forceinline__ void list_entry(int x, float f, RowList<K>& g)
                 left &= ~t;
             }
         }
-        if (left != 0ull) {
+        if (before >= K && left != 0ull) {
             const bool full = in_mask(left);
             g.ovf |= left;
             g.outside = full && f > g.outside ? f : g.outside;
@@ -239,11 +251,12 @@ __device__ __forceinline__ void entries_load(const StepArgs& a, int z, unsigned 
     }
 }
 
-template <int K, int P, int S>
+// (SKIP comes with the 7-point order, whose S * P + p entries came before.)
+template <int K, int P, int S, bool SKIP = true>
 __device__ __forceinline__ void entries_list(const RowEntries<P>& e, RowList<K>& g)
 {
 #pragma unroll
-    for (int p = 0; p < P; ++p) list_entry<K, S>(e.x[p], e.f[p], g);
+    for (int p = 0; p < P; ++p) list_entry<K, S, SKIP>(e.x[p], e.f[p], SKIP ? S * P + p : K, g);
 }
 
 // The same, each entry's registers refilled with the next point's (plane term
@@ -257,7 +270,7 @@ __device__ __forceinline__ void entries_list_next(const StepArgs& a, int z, unsi
     for (int p = 0; p < P; ++p) {
         const int x = e.x[p];
         const float f = e.f[p];
-        list_entry<K, S>(x, f, g);
+        list_entry<K, S, true>(x, f, S * P + p, g);
         const long long b = (long long)p * a.L + z;
         e.x[p] = at_off(a.arg + b, o);
         e.f[p] = at_off(a.ph + b, o);
@@ -372,29 +385,29 @@ __device__ __forceinline__ void row_gather(const StepArgs& a, const RowStencil& 
 #pragma unroll
                 for (int p = 0; p < P; ++p) x[p] = at_off(a.arg + ((long long)p * a.L + z), o);
 #pragma unroll
-                for (int p = 0; p < P; ++p) list_entry<K, -1>(x[p], 0.0f, g);
+                for (int p = 0; p < P; ++p) list_entry<K, -1, false>(x[p], 0.0f, K, g);
             }
         };
         RowEntries<P> e;
         ids(0, 4);
         entries_load(a, zD, c, e);
-        entries_list<K, P, 0>(e, g);
+        entries_list<K, P, 0, false>(e, g);
         ids(5, 10);
         entries_load(a, zC, ym, e);
-        entries_list<K, P, 1>(e, g);
+        entries_list<K, P, 1, false>(e, g);
         ids(11, 12);
         entries_load(a, zC, xm, e);
-        entries_list<K, P, 2>(e, g);
+        entries_list<K, P, 2, false>(e, g);
         entries_load(a, zC, c, e);
-        entries_list<K, P, 3>(e, g);
+        entries_list<K, P, 3, false>(e, g);
         entries_load(a, zC, xp, e);
-        entries_list<K, P, 4>(e, g);
+        entries_list<K, P, 4, false>(e, g);
         ids(15, 16);
         entries_load(a, zC, yp, e);
-        entries_list<K, P, 5>(e, g);
+        entries_list<K, P, 5, false>(e, g);
         ids(17, 22);
         entries_load(a, zU, c, e);
-        entries_list<K, P, 6>(e, g);
+        entries_list<K, P, 6, false>(e, g);
         ids(23, 27);
     }
 }
