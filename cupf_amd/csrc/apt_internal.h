@@ -198,7 +198,16 @@ struct NuclArgs {
 
 // Launchers (apt_misc.hip, step_k*_g*.hip).  All enqueue on
 // `stream` and return the hipError_t of the launch.
-// Workgroups of the persistent step kernel that fit the device at once.
+// Step waves launched per wave that fits the device: the dispatcher gives a CU
+// whose wave has ended the next one, which evens out units of unequal cost (a
+// grid of only the waves that fit, each with its share of the units, had its
+// waves done for 10 % of the launch on average); a wave that finds no unit
+// costs ~0.17 ns.  Rounds 1 / 2 / 4 / 6 / 8 / 16 / 64: 256x256x512 at step 150
+// 155 / 154 / 140 / 136 / 138 / 135 / 172 us, at step 450 36 / 34 / 33 / 34 /
+// 34 / 40 / 81; 78 % solid 256^3 window 1003 / 998 / 988 / 983 / 972 / 961 / 994.
+constexpr int kStepRounds = 6;
+
+// Workgroups of the step kernel that fit the device at once.
 int step_kernel_slots(int K, int gather27, int device);
 int batch_kernel_slots(int K, int gather27, int device);
 // Workgroups of the (single or batched) overflow fix-up kernel that fit at once.

@@ -69,7 +69,7 @@ struct pf_ctx {
     unsigned long long nlaunch = 0;  // step launches so far (selects the counter set)
     int nzchunk = 0, items_chunk = 0;
     int tiles_x = 0, tiles_y = 0;   // column tiles (partial ones included)
-    int step_blocks = 0;            // persistent step waves (occupancy x CUs, at most one per unit)
+    int step_blocks = 0;            // step waves (kStepRounds x occupancy x CUs, at most one per unit)
     int fix_blocks = 0;             // fix-up workgroups (occupancy x CUs)
     bool have_coords = false, have_orient = false, have_state = false;
 };
@@ -548,9 +548,11 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
         c->nzchunk = (p.fnz - 2 + c->kchunk - 1) / c->kchunk;
     }
     {
-        // one wave per unit is enough: a small grid does not dispatch idle waves
+        // kStepRounds times the waves that fit, in whole runs of the XCDs'
+        // round; one per unit is enough: a small grid dispatches no idle waves
         const long long units = c->nzchunk * (4LL * c->items_chunk + strip_waves(strip_width(p.fnx, c->tiles_x), p.fny));
-        c->step_blocks = (int)std::min<long long>(step_kernel_slots(p.K, p.gather27, device), units);
+        c->step_blocks = (int)std::min<long long>((long long)kStepRounds * step_kernel_slots(p.K, p.gather27, device),
+                                                  (units + 127) / 128 * 128);
     }
     {
         // at most the workgroups that could have an overflowed point (4 waves
@@ -1357,6 +1359,10 @@ int pf_batch_create(pf_ctx* const* ctxs, int n, pf_batch** out)
     for (pf_ctx* c : b->ctxs)
         b->wl_cap += (size_t)((c->p.fnz - 2 + pf_batch::kMinChunk - 1) / pf_batch::kMinChunk) *
                      c->items_chunk;
+    long long units = 4LL * (long long)b->wl_cap;
+    for (pf_ctx* c : b->ctxs)
+        units += (c->p.fnz - 2LL) * strip_waves(strip_width(c->p.fnx, c->tiles_x), c->p.fny);
+    b->step_blocks = (int)std::min<long long>((long long)kStepRounds * b->step_blocks, (units + 127) / 128 * 128);
     int rc;
     if ((rc = dalloc(&b->sims, (size_t)n)) || (rc = dalloc(&b->wl_sim, b->wl_cap + 1)) ||
         (rc = dalloc(&b->wl_item, b->wl_cap + 1)) || (rc = dalloc(&b->wl_need, b->wl_cap + 1)) ||

@@ -1,4 +1,4 @@
-// step_kernels.h -- the persistent step and fix-up kernels (single simulation
+// step_kernels.h -- the step and fix-up kernels (single simulation
 // and batched), instantiated once per (K, gather variant) by the step_k*_g*.hip
 // files so the large template instantiations compile in parallel.
 #pragma once
@@ -26,7 +26,7 @@ __device__ __forceinline__ unsigned row_place(unsigned W)
 }
 
 // APTrhs_psi (3DgrainMPI/APTPhaseField.cu:178-354) over every interior point:
-// a persistent grid of one-wave workgroups over units, the strip's first, then
+// one-wave workgroups, a few rounds of them, over units, the strip's first, then
 // row r of listed chunk e as unit 4 e + r.  Waves take units by position: an
 // atomic claim per unit (or only for the last two rounds) costs ~17 ns each on
 // one address, which the start-up's 36,000 row planes of 4 us do not afford
