@@ -15,7 +15,10 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
+
+#include <sys/mman.h>
 
 #include "../../include/pf_capi.h"
 #include "apt_internal.h"
@@ -715,7 +718,7 @@ int pf_init_from_phi_alpha(pf_ctx* c, const float* phi0, const int* alpha0)
     if (!phi0 || !alpha0) return fail(PF_E_INVALID, "null initial field");
     const size_t L = c->L;
     HIPCHK(hipMemcpyAsync(c->phi0, phi0, sizeof(float) * L, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->phi, phi0, sizeof(float) * L, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->phi, c->phi0, sizeof(float) * L, hipMemcpyDeviceToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->alpha, alpha0, sizeof(int) * L, hipMemcpyHostToDevice, c->stream));
     c->cur = 0;
     HIPCHK(launch_ini(c->ph[0], c->arg[0], c->ph[1], c->arg[1], c->phi0, c->alpha, c->L, c->p.K,
@@ -741,6 +744,29 @@ int pf_reinit_from_collect(pf_ctx* c)
     return PF_OK;
 }
 
+// Makes the pages of a large result buffer present while the device still
+// works on what goes there.  A fresh array's pages are zeroed one fault at a
+// time, inside the copy otherwise, which then runs at 10 GB/s instead of 25.
+// The contents stay; where the kernel or the mapping does not take the advice,
+// the copy faults as before.  Small buffers are left to the copy.
+static void make_present(std::initializer_list<std::pair<void*, size_t>> bufs)
+{
+    constexpr size_t kSmall = 8u << 20, kPage = 4096, kThreads = 4;
+    std::vector<std::thread> pool;
+    try {
+        for (auto [p, bytes] : bufs) {
+            if (!p || bytes < kSmall) continue;
+            const uintptr_t lo = ((uintptr_t)p + kPage - 1) / kPage * kPage;
+            const uintptr_t hi = ((uintptr_t)p + bytes) / kPage * kPage;
+            const size_t part = ((hi - lo) / kThreads + kSmall - 1) / kSmall * kSmall;
+            for (uintptr_t q = lo; q < hi; q += part)
+                pool.emplace_back([=] { (void)madvise((void*)q, std::min<size_t>(part, hi - q), 23 /* MADV_POPULATE_WRITE */); });
+        }
+    } catch (...) {  // no thread to be had: the copy does the rest
+    }
+    for (auto& t : pool) t.join();
+}
+
 int pf_upload_state(pf_ctx* c, int which, const float* ph, const int* arg)
 {
     int rc = ctx_check(c);
@@ -762,6 +788,7 @@ int pf_download_state(pf_ctx* c, int which, float* ph, int* arg)
     if (rc) return rc;
     const int b = buf_index(c, which);
     const size_t n = (size_t)c->L * c->p.K;
+    make_present({{ph, sizeof(float) * n}, {arg, sizeof(int) * n}});
     if (ph) HIPCHK(hipMemcpyAsync(ph, c->ph[b], sizeof(float) * n, hipMemcpyDeviceToHost, c->stream));
     if (arg) HIPCHK(hipMemcpyAsync(arg, c->arg[b], sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -921,6 +948,7 @@ int pf_collect(pf_ctx* c, int which, int flags, float* phi_out, int* alpha_out)
                               c->stream));
     HIPCHK(launch_collect(c->ph[b], c->arg[b], c->phi, c->alpha, c->L, p.K,
                           (flags & PF_COLLECT_CLEAR_ALPHA) ? 1 : 0, c->stream));
+    make_present({{phi_out, sizeof(float) * c->L}, {alpha_out, sizeof(int) * c->L}});
     if (phi_out)
         HIPCHK(hipMemcpyAsync(phi_out, c->phi, sizeof(float) * c->L, hipMemcpyDeviceToHost, c->stream));
     if (alpha_out)
