@@ -13,7 +13,7 @@
 // instructions per row plane, 16 waves per CU) and by latency and launches in
 // small grids.  Measured against 64x4 tiles with their halo in a three-plane
 // LDS ring (76 KB, 203 registers: 8 waves per CU, every slot staged), step
-// kernel: 256x256x512 at step 6 450 -> 240 us, at 150 259 -> 156, at 450 87 ->
+// kernel: 256x256x512 at step 6 450 -> 215 us, at 150 259 -> 130, at 450 87 ->
 // 36, at 1500 128 -> 55; 64^3 at step 10 108 -> 32, at 900 56 -> 21; 32^3 K=5
 // 62 -> 16; a 78 % solid 256^3 window 1340 -> 1000.  The general path with its
 // values in LDS (14 KB a wave, 10 waves per CU) took 1530 us for that window.
@@ -172,22 +172,35 @@ __device__ __forceinline__ void list_init(RowList<K>& g)
     g.ovf = 0ull;
 }
 
-// Entry (x, f) of a neighbour point, the (before + 1)th of the gather; S: its
-// stencil row, -1 for none; SKIP: leave at once where no lane has an id (pays
+// Entry (x, f) of a neighbour point, its slot `slot`, the (before + 1)th of the
+// gather; S: its stencil row, -1 for none; SKIP: leave at once where no lane has an id (pays
 // with the 7 points, whose entries run up to the largest bound around: 1060 ->
 // 1020 us for a 78 % solid 256^3 window; the 27 points lose 5 %).
-// Only positions that entries so far can have filled are looked at.  Positions
+// Only positions that earlier entries can have filled are looked at.  Positions
 // fill in order, so a pair whose second one is filled in every lane that meets
 // a new id has nothing to take: one branch per pair (256x256x512 at step 150:
 // 162 us with a branch per position or one for all 8, 157 with pairs).
 template <int K, int S, bool SKIP>
-__device__ __forceinline__ void list_entry(int x, float f, int before, RowList<K>& g)
+__device__ __forceinline__ void list_entry(int x, float f, int before, int slot, RowList<K>& g)
 {
     unsigned long long left = __ballot(x != -1);  // lanes that meet a new id
     if (SKIP && left == 0ull) return;
+    // A point and the one above it hold their ids in the order in which the
+    // point below listed them a step ago: their slot's own position first, and
+    // mostly nothing is left to look for (9 of 10 entries in a solid window, 2
+    // of 3 in a start-up; 982 -> 957 us, 227 -> 215; the narrow path loses 4 %,
+    // and as an exit of its own, before the compares, it cost 20 % in copies).
+    constexpr bool HINT = SKIP && (S == 3 || S == 6) && K > 4;
+    if (HINT) {
+        const bool e = g.la[slot] == x;
+        g.v[S < 0 ? 0 : S][slot] = e ? f : g.v[S < 0 ? 0 : S][slot];
+        left &= ~__ballot(e);
+        if (left == 0ull) return;
+    }
 #pragma unroll
     for (int q = 0; q < K; ++q) {
         if (q >= before) break;
+        if (HINT && q == slot) continue;
         const bool e = g.la[q] == x;
         if (S >= 0) g.v[S < 0 ? 0 : S][q] = e ? f : g.v[S < 0 ? 0 : S][q];
         left &= ~__ballot(e);
@@ -256,7 +269,7 @@ template <int K, int P, int S, bool SKIP = true>
 __device__ __forceinline__ void entries_list(const RowEntries<P>& e, RowList<K>& g)
 {
 #pragma unroll
-    for (int p = 0; p < P; ++p) list_entry<K, S, SKIP>(e.x[p], e.f[p], SKIP ? S * P + p : K, g);
+    for (int p = 0; p < P; ++p) list_entry<K, S, SKIP>(e.x[p], e.f[p], SKIP ? S * P + p : K, p, g);
 }
 
 // The same, each entry's registers refilled with the next point's (plane term
@@ -270,7 +283,7 @@ __device__ __forceinline__ void entries_list_next(const StepArgs& a, int z, unsi
     for (int p = 0; p < P; ++p) {
         const int x = e.x[p];
         const float f = e.f[p];
-        list_entry<K, S, true>(x, f, S * P + p, g);
+        list_entry<K, S, true>(x, f, S * P + p, p, g);
         const long long b = (long long)p * a.L + z;
         e.x[p] = at_off(a.arg + b, o);
         e.f[p] = at_off(a.ph + b, o);
@@ -385,7 +398,7 @@ __device__ __forceinline__ void row_gather(const StepArgs& a, const RowStencil& 
 #pragma unroll
                 for (int p = 0; p < P; ++p) x[p] = at_off(a.arg + ((long long)p * a.L + z), o);
 #pragma unroll
-                for (int p = 0; p < P; ++p) list_entry<K, -1, false>(x[p], 0.0f, K, g);
+                for (int p = 0; p < P; ++p) list_entry<K, -1, false>(x[p], 0.0f, K, -1, g);
             }
         };
         RowEntries<P> e;
