@@ -265,8 +265,16 @@ hipError_t launch_bc_fill(float* ph, int* arg, int fnx, int fny, int fnz, int K,
                           int bcy, int bcz, hipStream_t stream);
 hipError_t launch_collect(const float* ph, const int* arg, float* phi, int* alpha, int L, int K,
                           int clear_alpha, hipStream_t stream);
+// Both buffers' maps (activity and row words, new epochs), marked while the
+// buffers are initialised.
+struct IniMaps {
+    unsigned* act[2];
+    unsigned* row[2];
+    unsigned ep[2];
+    int fnx, fny, fnz, ntx, ntiles;
+};
 hipError_t launch_ini(float* ph0, int* arg0, float* ph1, int* arg1, const float* phi0,
-                      const int* alpha0, int L, int K, hipStream_t stream);
+                      const int* alpha0, int L, int K, const IniMaps& maps, hipStream_t stream);
 // Exact sums of planes k_from .. k_to-1 into sums[k_from .. k_to) (the rest untouched).
 hipError_t launch_plane_sums(const float* ph, long long* sums, int fnx, int fny, int fnz, int K,
                              int k_from, int k_to, hipStream_t stream);

@@ -169,9 +169,12 @@ __global__ __launch_bounds__(kBlock) void collect_kernel(const float* __restrict
 
 // set_minus1 + memset(-1) + APTini_PF on both buffers
 // (3DgrainMPI/APTPhaseField.cu:78-89,727-728,817-818).
+// The maps of both buffers are marked on the way: only slot 0 is filled, and
+// every writer of a word writes the same value.  (Reading both buffers back for
+// their maps took 1.5 ms after these 0.7 ms of a 256x256x512, K = 8 domain.)
 __global__ __launch_bounds__(kBlock) void ini_kernel(float* ph0, int* arg0, float* ph1, int* arg1,
                                                      const float* __restrict__ phi0,
-                                                     const int* __restrict__ alpha0, int L, int K)
+                                                     const int* __restrict__ alpha0, int L, int K, IniMaps m)
 {
     const int q = blockIdx.x * kBlock + threadIdx.x;
     if (q >= L * K) return;
@@ -185,6 +188,21 @@ __global__ __launch_bounds__(kBlock) void ini_kernel(float* ph0, int* arg0, floa
     arg0[q] = id;
     ph1[q] = v;
     arg1[q] = id;
+    if (id != -1 || v != -1.0f) {
+        const int A = m.fnx * m.fny;
+        const int k = q / A;
+        const int r = q - k * A;
+        const int j = r / m.fnx;
+        const int i = r - j * m.fnx;
+        if (i >= 1 && i <= m.fnx - 2 && j >= 1 && j <= m.fny - 2 && k >= 1 && k <= m.fnz - 2) {
+            const int x = act_tile_x(i);
+            const int t = k * m.ntiles + x + act_tile_y(j) * m.ntx, w = (k * m.fny + j) * m.ntx + x;
+            m.act[0][t] = m.ep[0];
+            m.act[1][t] = m.ep[1];
+            m.row[0][w] = m.ep[0] << 4 | 1u;
+            m.row[1][w] = m.ep[1] << 4 | 1u;
+        }
+    }
 }
 
 // ave_x (3DgrainMPI/PhaseField.cu:366-378) as an exact fixed-point sum:
@@ -306,64 +324,75 @@ __device__ __forceinline__ float nucl_prob(const NuclArgs& a, float delT, float 
 
 // add_nucl (3DgrainMPI/APTPhaseField.cu:459-536) with a counter-based draw per
 // (seed, coarse cell, call) instead of per-cell cuRAND state.
+// A wave stamps its nuclei one after the other, a lane per point (w^3 of them,
+// one cell's own), and marks each row once per tile: a lane that stamped its
+// own cell was one chain of w^3 stores and atomics (138 us a call for 256^3,
+// the length of a nucleus).
 __global__ __launch_bounds__(kBlock) void nucl_kernel(NuclArgs a)
 {
     const int C = blockIdx.x * kBlock + threadIdx.x;
-    if (C >= a.cnx * a.cny * a.cnz) return;
-    if (a.status[C] != 0) return;
+    const int w = 2 * a.p + 1;
+    const int A = a.fnx * a.fny;
     const int k = C / (a.cnx * a.cny);
     const int r = C - k * a.cnx * a.cny;
     const int j = r / a.cnx;
     const int i = r - j * a.cnx;
-    const int w = 2 * a.p + 1;
     const int gi = w * i + a.p + 1, gj = w * j + a.p + 1, gk = w * k + a.p + 1;
-    const int A = a.fnx * a.fny;
-    const int gC = gk * A + gj * a.fnx + gi;
-    int st = 0;
-    for (int s = 0; s < a.K; ++s)
-        if ((double)a.ph[gC + s * a.L] > kLS) st = 1;
-    if (st) {
-        a.status[C] = 1;
-        return;
+    int id = 0;
+    bool born = false;
+    if (C < a.cnx * a.cny * a.cnz && a.status[C] == 0) {
+        const int gC = gk * A + gj * a.fnx + gi;
+        int st = 0;
+        for (int s = 0; s < a.K; ++s)
+            if ((double)a.ph[gC + s * a.L] > kLS) st = 1;
+        if (!st) {
+            float posb;
+            if (a.use_iuc) {
+                float delT = a.uc0 * 1e6 * (a.t + a.dt);
+                float d_delT = a.uc0 * 1e6 * a.dt;
+                posb = nucl_prob(a, delT, d_delT, a.nuc_Nmax0);
+            } else {
+                const float xx = a.x[gi] - a.X0_mac, yy = a.y[gj] - a.Y0_mac, zz = a.z[gk] - a.Z0_mac;
+                float Tc = interp4(a.T3d, xx, yy, zz, a.t - a.t0_mac, a.Nx, a.Ny, a.Nz, a.Nt, a.Dx_mac,
+                                   a.Dt_mac);
+                float Tcd = interp4(a.T3d, xx, yy, zz, a.t + a.dt - a.t0_mac, a.Nx, a.Ny, a.Nz, a.Nt,
+                                    a.Dx_mac, a.Dt_mac);
+                posb = nucl_prob(a, -Tcd, Tc - Tcd, a.nuc_Nmax);
+            }
+            uint64_t h = mix64(a.seed + 0x9e3779b97f4a7c15ULL);
+            h = mix64(h ^ ((uint64_t)C * 0xd1b54a32d192ed03ULL));
+            h = mix64(h ^ (a.call * 0x8cb92ba72f3d8dd7ULL + 0x632be59bd9b4e019ULL));
+            const float u = (float)((h >> 40) + 1) * (1.0f / 16777216.0f);
+            id = 1 + (int)(((h & 0xffffffffULL) * 0x7ffffffeULL) >> 32);
+            born = u < posb;
+        }
+        if (st || born) a.status[C] = 1;
     }
-    float posb;
-    if (a.use_iuc) {
-        float delT = a.uc0 * 1e6 * (a.t + a.dt);
-        float d_delT = a.uc0 * 1e6 * a.dt;
-        posb = nucl_prob(a, delT, d_delT, a.nuc_Nmax0);
-    } else {
-        const float xx = a.x[gi] - a.X0_mac, yy = a.y[gj] - a.Y0_mac, zz = a.z[gk] - a.Z0_mac;
-        float Tc = interp4(a.T3d, xx, yy, zz, a.t - a.t0_mac, a.Nx, a.Ny, a.Nz, a.Nt, a.Dx_mac,
-                           a.Dt_mac);
-        float Tcd = interp4(a.T3d, xx, yy, zz, a.t + a.dt - a.t0_mac, a.Nx, a.Ny, a.Nz, a.Nt,
-                            a.Dx_mac, a.Dt_mac);
-        posb = nucl_prob(a, -Tcd, Tc - Tcd, a.nuc_Nmax);
-    }
-    uint64_t h = mix64(a.seed + 0x9e3779b97f4a7c15ULL);
-    h = mix64(h ^ ((uint64_t)C * 0xd1b54a32d192ed03ULL));
-    h = mix64(h ^ (a.call * 0x8cb92ba72f3d8dd7ULL + 0x632be59bd9b4e019ULL));
-    const float u = (float)((h >> 40) + 1) * (1.0f / 16777216.0f);
-    const int id = 1 + (int)(((h & 0xffffffffULL) * 0x7ffffffeULL) >> 32);
-    if (u < posb) {
-        int q = 0;
-        for (int lk = -a.p; lk <= a.p; ++lk)
-            for (int lj = -a.p; lj <= a.p; ++lj)
-                for (int li = -a.p; li <= a.p; ++li) {
-                    const int o = gC + lk * A + lj * a.fnx + li;
-                    const float v = a.ball[q++];
-                    a.ph[o] = v;
-                    if (v > -0.9999f) a.arg[o] = id;
-                    a.act[(gk + lk) * a.ntiles + act_tile_x(gi + li) + act_tile_y(gj + lj) * a.ntx] =
-                        a.ep;
-                    atomicMax(a.row + ((gk + lk) * a.fny + gj + lj) * a.ntx + act_tile_x(gi + li), a.ep << 4 | 1u);
-                }
-        a.status[C] = 1;
-        atomicAdd(a.events, 1ull);
+    unsigned long long m = __ballot(born);
+    if (m == 0ull) return;
+    if ((threadIdx.x & 63) == 0) atomicAdd(a.events, (unsigned long long)__popcll(m));
+    for (; m; m &= m - 1) {
+        const int s = __ffsll((long long)m) - 1;
+        const int ci = __shfl(gi, s), cj = __shfl(gj, s), ck = __shfl(gk, s), cid = __shfl(id, s);
+        for (int q = threadIdx.x & 63; q < w * w * w; q += 64) {
+            const int lk = q / (w * w);
+            const int x = ci - a.p + q % w, y = cj - a.p + q / w % w, z = ck - a.p + lk;
+            const int o = z * A + y * a.fnx + x;
+            const float v = a.ball[q];
+            a.ph[o] = v;
+            if (v > -0.9999f) a.arg[o] = cid;
+            if (q % w == 0 || act_tile_x(x) != act_tile_x(x - 1)) {
+                a.act[z * a.ntiles + act_tile_x(x) + act_tile_y(y) * a.ntx] = a.ep;
+                atomicMax(a.row + (z * a.fny + y) * a.ntx + act_tile_x(x), a.ep << 4 | 1u);
+            }
+        }
     }
 }
 
 // Activity and row maps from a buffer's contents (after it was written other
-// than by a step): one lane per interior point, K slots each.
+// than by a step): one wave per row of a tile, every slot of its points in one
+// round trip, no atomics (one lane per point and an atomic per filled point
+// took 1080 us for a solid 256^3 window).
 __global__ __launch_bounds__(kBlock) void act_rebuild_kernel(const float* __restrict__ ph,
                                                              const int* __restrict__ arg,
                                                              unsigned* act, unsigned* row,
@@ -371,20 +400,24 @@ __global__ __launch_bounds__(kBlock) void act_rebuild_kernel(const float* __rest
                                                              int fny, int fnz, int K, int ntx,
                                                              int ntiles)
 {
-    const int nx = fnx - 2, ny = fny - 2;
-    const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (q >= (long long)nx * ny * (fnz - 2)) return;
-    const int k = 1 + (int)(q / ((long long)nx * ny));
-    const int r = (int)(q - (long long)(k - 1) * nx * ny);
-    const int j = 1 + r / nx;
-    const int i = 1 + r - (j - 1) * nx;
+    const int ny = fny - 2;
+    const long long u = (long long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+    if (u >= (long long)ntx * ny * (fnz - 2)) return;
+    const int x = (int)(u % ntx);
+    const int r = (int)(u / ntx);
+    const int j = 1 + r % ny, k = 1 + r / ny;
+    const int i = 1 + x * kTX + (int)(threadIdx.x & 63);
     const int L = fnx * fny * fnz;
-    const int C = i + j * fnx + k * fnx * fny;
+    const int C = min(i, fnx - 2) + j * fnx + k * fnx * fny;
+    bool full[8];  // K <= 8
+#pragma unroll
+    for (int s = 0; s < 8; ++s) full[s] = s < K && ((arg[C + s * L] != -1) | (ph[C + s * L] != -1.0f));
     unsigned bound = 0u;
-    for (int s = 0; s < K; ++s) bound = arg[C + s * L] != -1 || ph[C + s * L] != -1.0f ? s + 1u : bound;
-    if (bound) {
-        act[k * ntiles + act_tile_x(i) + act_tile_y(j) * ntx] = ep;
-        atomicMax(row + (k * fny + j) * ntx + act_tile_x(i), ep << 4 | bound);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) bound = __ballot(full[s]) != 0ull ? s + 1u : bound;
+    if (bound && (threadIdx.x & 63) == 0) {
+        act[k * ntiles + x + act_tile_y(j) * ntx] = ep;
+        row[(k * fny + j) * ntx + x] = ep << 4 | bound;
     }
 }
 
@@ -460,8 +493,8 @@ int fixup_kernel_slots(int K, int gather27, int device, bool batch)
 hipError_t launch_act_rebuild(const float* ph, const int* arg, unsigned* act, unsigned* row, unsigned ep,
                               int fnx, int fny, int fnz, int K, int ntx, int ntiles, hipStream_t stream)
 {
-    const long long n = (long long)(fnx - 2) * (fny - 2) * (fnz - 2);
-    hipLaunchKernelGGL(act_rebuild_kernel, dim3(cdiv(n, kBlock)), dim3(kBlock), 0, stream, ph, arg,
+    const long long n = (long long)ntx * (fny - 2) * (fnz - 2);  // waves
+    hipLaunchKernelGGL(act_rebuild_kernel, dim3(cdiv(n, kBlock / 64)), dim3(kBlock), 0, stream, ph, arg,
                        act, row, ep, fnx, fny, fnz, K, ntx, ntiles);
     return hipGetLastError();
 }
@@ -493,10 +526,10 @@ hipError_t launch_collect(const float* ph, const int* arg, float* phi, int* alph
 }
 
 hipError_t launch_ini(float* ph0, int* arg0, float* ph1, int* arg1, const float* phi0,
-                      const int* alpha0, int L, int K, hipStream_t stream)
+                      const int* alpha0, int L, int K, const IniMaps& maps, hipStream_t stream)
 {
     hipLaunchKernelGGL(ini_kernel, dim3(cdiv((long long)L * K, kBlock)), dim3(kBlock), 0, stream,
-                       ph0, arg0, ph1, arg1, phi0, alpha0, L, K);
+                       ph0, arg0, ph1, arg1, phi0, alpha0, L, K, maps);
     return hipGetLastError();
 }
 

@@ -306,6 +306,16 @@ hipError_t act_rebuild(pf_ctx* c, int b)
                               c->ntx, c->ntiles, c->stream);
 }
 
+// Both buffers and their maps from phi0 and alpha.
+hipError_t init_state(pf_ctx* c)
+{
+    const pf_params& p = c->p;
+    for (int b = 0; b < 2; ++b) c->ep[b] = ++c->ep_ctr;
+    const IniMaps m{{c->act[0], c->act[1]}, {c->row[0], c->row[1]}, {c->ep[0], c->ep[1]},
+                    p.fnx, p.fny, p.fnz, c->ntx, c->ntiles};
+    return launch_ini(c->ph[0], c->arg[0], c->ph[1], c->arg[1], c->phi0, c->alpha, c->L, p.K, m, c->stream);
+}
+
 // The epoch counter's limit: row words hold an epoch and 4 bits of bound.
 constexpr unsigned kEpochMax = 0x07ffffffu;
 
@@ -721,10 +731,7 @@ int pf_init_from_phi_alpha(pf_ctx* c, const float* phi0, const int* alpha0)
     HIPCHK(hipMemcpyAsync(c->phi, c->phi0, sizeof(float) * L, hipMemcpyDeviceToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->alpha, alpha0, sizeof(int) * L, hipMemcpyHostToDevice, c->stream));
     c->cur = 0;
-    HIPCHK(launch_ini(c->ph[0], c->arg[0], c->ph[1], c->arg[1], c->phi0, c->alpha, c->L, c->p.K,
-                      c->stream));
-    HIPCHK(act_rebuild(c, 0));
-    HIPCHK(act_rebuild(c, 1));
+    HIPCHK(init_state(c));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->have_state = true;
     return PF_OK;
@@ -736,10 +743,7 @@ int pf_reinit_from_collect(pf_ctx* c)
     if (rc) return rc;
     if (!c->have_state) return fail(PF_E_STATE, "no initial field");
     c->cur = 0;
-    HIPCHK(launch_ini(c->ph[0], c->arg[0], c->ph[1], c->arg[1], c->phi0, c->alpha, c->L, c->p.K,
-                      c->stream));
-    HIPCHK(act_rebuild(c, 0));
-    HIPCHK(act_rebuild(c, 1));
+    HIPCHK(init_state(c));
     HIPCHK(hipStreamSynchronize(c->stream));
     return PF_OK;
 }
