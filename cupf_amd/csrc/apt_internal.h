@@ -263,8 +263,16 @@ hipError_t launch_qoi_area(const int* alpha, int fnx, int fny, int fnz, int ng, 
                            int* extra, hipStream_t stream);
 hipError_t launch_bc_fill(float* ph, int* arg, int fnx, int fny, int fnz, int K, int bcx,
                           int bcy, int bcz, hipStream_t stream);
+// The buffer's row words for launch_collect (row = nullptr: every slot is
+// read); halo: it was filled from the buffer as it is.
+struct CollectRows {
+    const unsigned* row;
+    unsigned ep;
+    int halo;
+    int fnx, fny, fnz, bcx, bcy, bcz, ntx;
+};
 hipError_t launch_collect(const float* ph, const int* arg, float* phi, int* alpha, int L, int K,
-                          int clear_alpha, hipStream_t stream);
+                          int clear_alpha, const CollectRows& rows, hipStream_t stream);
 // Both buffers' maps (activity and row words, new epochs), marked while the
 // buffers are initialised.
 struct IniMaps {

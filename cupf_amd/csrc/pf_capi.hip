@@ -316,6 +316,15 @@ hipError_t init_state(pf_ctx* c)
     return launch_ini(c->ph[0], c->arg[0], c->ph[1], c->arg[1], c->phi0, c->alpha, c->L, p.K, m, c->stream);
 }
 
+// phi and alpha from buffer b; halo: its halo was filled from it as it is.
+hipError_t collect_fields(pf_ctx* c, int b, bool halo, int clear_alpha)
+{
+    const pf_params& p = c->p;
+    const CollectRows rows{c->use_act ? c->row[b] : nullptr, c->ep[b], halo ? 1 : 0, p.fnx, p.fny, p.fnz,
+                           p.bcx, p.bcy, p.bcz, c->ntx};
+    return launch_collect(c->ph[b], c->arg[b], c->phi, c->alpha, c->L, p.K, clear_alpha, rows, c->stream);
+}
+
 // The epoch counter's limit: row words hold an epoch and 4 bits of bound.
 constexpr unsigned kEpochMax = 0x07ffffffu;
 
@@ -950,8 +959,7 @@ int pf_collect(pf_ctx* c, int which, int flags, float* phi_out, int* alpha_out)
     if (!(flags & PF_COLLECT_NO_BC))
         HIPCHK(launch_bc_fill(c->ph[b], c->arg[b], p.fnx, p.fny, p.fnz, p.K, p.bcx, p.bcy, p.bcz,
                               c->stream));
-    HIPCHK(launch_collect(c->ph[b], c->arg[b], c->phi, c->alpha, c->L, p.K,
-                          (flags & PF_COLLECT_CLEAR_ALPHA) ? 1 : 0, c->stream));
+    HIPCHK(collect_fields(c, b, !(flags & PF_COLLECT_NO_BC), (flags & PF_COLLECT_CLEAR_ALPHA) ? 1 : 0));
     make_present({{phi_out, sizeof(float) * c->L}, {alpha_out, sizeof(int) * c->L}});
     if (phi_out)
         HIPCHK(hipMemcpyAsync(phi_out, c->phi, sizeof(float) * c->L, hipMemcpyDeviceToHost, c->stream));
@@ -1192,7 +1200,7 @@ int pf_md_shift(pf_ctx* c, int move_count)
     const int b = c->cur;
     // APTcollect_PF on the buffer as stored (3DgrainMPI/APTPhaseField.cu:683),
     // then APTmove_frame with the other buffer as scratch, then APTcopy_frame.
-    HIPCHK(launch_collect(c->ph[b], c->arg[b], c->phi, c->alpha, c->L, p.K, 0, c->stream));
+    HIPCHK(collect_fields(c, b, false, 0));
     HIPCHK(launch_move_frame(c->ph[b], c->arg[b], c->ph[1 - b], c->arg[1 - b], c->z, c->zbuf,
                              c->alpha, c->alpha_full, c->loss, move_count, p.fnx, p.fny, p.fnz,
                              p.K, p.num_theta, c->stream));
