@@ -222,8 +222,12 @@ __device__ __forceinline__ float slot_update(const StepArgs& a, int gid, float p
 // which names the next id of the ranking, and drop that id's entries; lanes
 // reduce by DPP within the group.  Then lane q updates slot q.
 //
-// Bound by latency for short lists and by VALU for long ones (~950
-// instructions per wave of 8 points).  One point per lane with a streaming
+// Bound by latency for short lists, by VALU issue and the fetches of the
+// neighbours' lines for long ones (~800 instructions per wave of 8 points).
+// Searching the maximum, its position and its id one after the other took 950,
+// and passing the step's arguments by value spilled scalar registers (97 vector
+// registers against 70): 64^3 K=8 13.4 -> 11.4 us, 96x96x128 K=5 with 27 points
+// 127 -> 108, 256x256x512 133 -> 119.  One point per lane with a streaming
 // top-K (56 dependent pushes and a second pass over the neighbours) was one
 // long chain of loads and compares, and left all but a few CUs idle: the
 // fix-up of a 64^3 K=8 start-up fell from 53-62 to 12-13 us, of 32^3 K=5 from
@@ -237,6 +241,7 @@ struct FixGroup {
     static constexpr int kLanes = G27 ? 16 : 8;   // lanes per point
     static constexpr int kPos = G27 ? 2 : 1;      // neighbour positions per lane
     static constexpr int kPoints = 64 / kLanes;   // points per wave
+    static constexpr int kIds = G27 ? 256 : 64;   // scan positions (padded): LDS words of the ids
 };
 
 // LDS words of one group: the kept ids' phi at the 7 stencil rows by rank
@@ -250,16 +255,8 @@ __device__ __forceinline__ int dpp_get(int v)
     return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false);
 }
 
-// Largest / smallest value over a group of 8 or 16 lanes, on every lane of it
+// Smallest value over a group of 8 or 16 lanes, on every lane of it
 // (all lanes of the wave active): xor 1, xor 2, half-row mirror, row mirror.
-template <bool G27>
-__device__ __forceinline__ int group_max(int v)
-{
-    v = max(v, dpp_get<0xB1>(v));
-    v = max(v, dpp_get<0x4E>(v));
-    v = max(v, dpp_get<0x141>(v));
-    return G27 ? max(v, dpp_get<0x140>(v)) : v;
-}
 template <bool G27>
 __device__ __forceinline__ int group_min(int v)
 {
@@ -275,6 +272,29 @@ __device__ __forceinline__ int phi_key(float x)
 {
     const int b = __float_as_int(x + 0.0f);
     return b ^ ((b >> 31) & 0x7fffffff);
+}
+
+// Ranking keys of the fix-up: doubles 1.mantissa, or below 1.0 (never NaN).
+constexpr unsigned kRankOne = 0x3ff00000u;
+__device__ __forceinline__ double rank_key(unsigned hi, unsigned lo) { return __hiloint2double((int)hi, (int)lo); }
+__device__ __forceinline__ double rank_max(double a, double b)
+{
+    double m;
+    asm("v_max_f64 %0, %1, %2" : "=v"(m) : "v"(a), "v"(b));
+    return m;
+}
+template <int CTRL>
+__device__ __forceinline__ double rank_max_dpp(double a)
+{
+    return rank_max(a, rank_key((unsigned)dpp_get<CTRL>(__double2hiint(a)), (unsigned)dpp_get<CTRL>(__double2loint(a))));
+}
+template <bool G27>
+__device__ __forceinline__ double group_rank_max(double a)
+{
+    a = rank_max_dpp<0xB1>(a);
+    a = rank_max_dpp<0x4E>(a);
+    a = rank_max_dpp<0x141>(a);
+    return G27 ? rank_max_dpp<0x140>(a) : a;
 }
 
 // Orders a wave's LDS accesses (DS operations of a wave complete in order).
@@ -297,8 +317,9 @@ __device__ __forceinline__ void fixup_group(const StepArgs& a, unsigned C, bool 
     const int rem = (int)C - k * A;
     const int j = rem / a.fnx;
     const int i = rem - j * a.fnx;
-    int id[E], key[E];
+    int id[E];
     float ph[E];
+    double key[E];
     int row = -1, rowpos = 0;  // the lane's stencil row (D,B,L,C,R,T,U) and which of its positions it is
 #pragma unroll
     for (int t = 0; t < F::kPos; ++t) {
@@ -333,26 +354,30 @@ __device__ __forceinline__ void fixup_group(const StepArgs& a, unsigned C, bool 
             id[t * K + p] = in ? x : -1;
         }
     }
-#pragma unroll
-    for (int e = 0; e < E; ++e) key[e] = id[e] != -1 ? phi_key(ph[e]) : kNoKey;
+    // An entry's key is its phi's order (32 bits) and below it the scan position
+    // counted backwards (8 bits) in a double's mantissa, so one maximum finds
+    // the largest phi and the earliest entry holding it; entries out of the
+    // ranking lie below 1.0.  Its id is then looked up in LDS.
     const int pos0 = l * K;  // scan position of entry e: pos0 + (16 K for the second position) + slot
+    unsigned* ids = sc + kFixStride;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int pos = pos0 + (e / K) * 16 * K + e % K;
+        const unsigned u = (unsigned)phi_key(ph[e]) ^ 0x80000000u;
+        key[e] = rank_key(id[e] != -1 ? kRankOne | u >> 12 : 0u, u << 20 | (unsigned)(255 - pos) << 12);
+        ids[pos] = (unsigned)id[e];
+    }
+    wave_lds_fence();
     int nk = 0;
 #pragma unroll 1
     for (int r = 0; r < K; ++r) {
-        int m = key[0];
+        double m = key[0];
 #pragma unroll
-        for (int e = 1; e < E; ++e) m = max(m, key[e]);
-        m = group_max<G27>(m);
-        int first = 0x7fffffff;
-#pragma unroll
-        for (int e = E - 1; e >= 0; --e)
-            first = key[e] == m ? pos0 + (e / K) * 16 * K + e % K : first;
-        first = group_min<G27>(first);
-        int kid = kNoKey;
-#pragma unroll
-        for (int e = 0; e < E; ++e) kid = pos0 + (e / K) * 16 * K + e % K == first ? id[e] : kid;
-        kid = group_max<G27>(kid);
-        const bool live = m != kNoKey;
+        for (int e = 1; e < E; ++e) m = rank_max(m, key[e]);
+        m = group_rank_max<G27>(m);
+        const bool live = (unsigned)__double2hiint(m) >= kRankOne;
+        const int top = 255 - ((unsigned)__double2loint(m) >> 12 & 255u);
+        const int kid = live ? (int)ids[top] : kNoKey;
         nk += live ? 1 : 0;
         // the id's entries leave the ranking; its phi at this lane's stencil
         // row is the last entry's, as the reference's overwrite gives it
@@ -360,15 +385,15 @@ __device__ __forceinline__ void fixup_group(const StepArgs& a, unsigned C, bool 
         int fp = 0x7fffffff;
 #pragma unroll
         for (int e = E - 1; e >= 0; --e) {
-            const bool h = live && id[e] == kid;
+            const bool h = id[e] == kid;
             fp = h ? pos0 + (e / K) * 16 * K + e % K : fp;
-            key[e] = h ? kNoKey : key[e];
+            key[e] = rank_key(h ? 0u : (unsigned)__double2hiint(key[e]), (unsigned)__double2loint(key[e]));
         }
 #pragma unroll
         for (int t = 0; t < F::kPos; ++t)
 #pragma unroll
             for (int p = 0; p < K; ++p)
-                v = live && id[t * K + p] == kid && (F::kPos == 1 || rowpos == t) ? ph[t * K + p] : v;
+                v = id[t * K + p] == kid && (F::kPos == 1 || rowpos == t) ? ph[t * K + p] : v;
         fp = group_min<G27>(fp);
         if (row >= 0) sc[kFixVal + 8 * r + row] = __float_as_uint(v);
         if (l == 0) {

@@ -59,6 +59,25 @@ __global__ __launch_bounds__(kRowLanes, 4) void apt_step(StepArgs)
         atomicAdd(a.overflow + kLineWords / 2 * (place % kSpread), (unsigned long long)nres);
 }
 
+// The units of kPoints list entries that wave w of workgroup blk takes: an
+// eighth of the list, in order, for each XCD (workgroups go to the 8 XCDs in
+// turn), because the 8 units of a row's 64 points share their neighbours'
+// lines; and within the eighth the first wave of every workgroup before the
+// second of any, so a short list is spread over the CUs.  (Units in order over
+// all workgroups met in no L2: 7.5 M line fetches against 6.3 M, and 130 against
+// 119 us, for the 270,000 points of the 256x256x512 start-up.)
+struct FixShare {
+    unsigned first, end, step;
+};
+__device__ __forceinline__ FixShare fix_share(unsigned units, int blk, int nblk, int w)
+{
+    const unsigned X = nblk % 8 == 0 ? 8u : 1u;
+    const unsigned x = (unsigned)blk % X, per = (unsigned)nblk / X;
+    const unsigned lo = (unsigned)((unsigned long long)units * x / X);
+    return {lo + (unsigned)w * per + (unsigned)blk / X, (unsigned)((unsigned long long)units * (x + 1u) / X),
+            per * (kFixLanes / 64)};
+}
+
 // Fix-up pass for the points of the last apt_step launch whose neighbourhood
 // overflowed K slots; adds their number to the overflow diagnostic.  The list
 // lives in this step's counter set, which the next-but-one plan kernel
@@ -67,7 +86,7 @@ template <int K, bool G27>
 __device__ __forceinline__ void fixup_run(const StepArgs& a, int blk, int nblk)
 {
     using F = FixGroup<G27>;
-    __shared__ unsigned s_fix[(kFixLanes / F::kLanes) * kFixStride];
+    __shared__ unsigned s_fix[(kFixLanes / F::kLanes) * (kFixStride + F::kIds)];
     __shared__ unsigned s_pre[kSpread + 1], s_cnt[kSpread], s_wave[kFixLanes / 64];
     const unsigned units = fixup_units<F::kPoints>(
         kSpread, [&](int q) { return __atomic_load_n(a.fix_count + kLineWords * q, __ATOMIC_RELAXED); }, s_pre,
@@ -79,23 +98,23 @@ __device__ __forceinline__ void fixup_run(const StepArgs& a, int blk, int nblk)
     const float epsv = -4.0f * a.kin_delta / a_s;
     const int l = threadIdx.x & (F::kLanes - 1), grp = threadIdx.x / F::kLanes;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    // wave units of kPoints entries, the first of every workgroup before the
-    // second of any, so a short list is spread over the CUs
+    const FixShare sh = fix_share(units, blk, nblk, w);
 #pragma unroll 1
-    for (unsigned u = (unsigned)(w * nblk + blk); u < units; u += (unsigned)(nblk * (kFixLanes / 64))) {
+    for (unsigned u = sh.first; u < sh.end; u += sh.step) {
         const int seg = fixup_find(s_pre, kSpread, u);
         const unsigned e0 = (u - s_pre[seg]) * F::kPoints;
         const unsigned e = e0 + (unsigned)(grp & (F::kPoints - 1));
         const bool on = e < s_cnt[seg];
         const unsigned* list = a.fix_list + (unsigned)(seg * a.fix_cap);
-        fixup_group<K, G27>(a, list[on ? e : e0], on, l, s_fix + grp * kFixStride, a_s, epsv);
+        fixup_group<K, G27>(a, list[on ? e : e0], on, l, s_fix + grp * (kFixStride + F::kIds), a_s, epsv);
     }
 }
 
 template <int K, bool G27>
-__global__ __launch_bounds__(kFixLanes) void apt_fixup(StepArgs a)
+__global__ __launch_bounds__(kFixLanes) void apt_fixup(StepArgs)
 {
-    fixup_run<K, G27>(a, (int)blockIdx.x, (int)gridDim.x);
+    CArgs* a = (CArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    fixup_run<K, G27>(*args_ref(a), (int)blockIdx.x, (int)gridDim.x);
 }
 
 // The fix-up of one step and the work-list plan of the next in one launch:
@@ -106,11 +125,13 @@ __global__ __launch_bounds__(kFixLanes) void apt_fixup(StepArgs a)
 // the one after (three sets in turn), so the two halves need no order
 // between them.  Saves one launch and its dispatch gap per step.
 template <int K, bool G27>
-__global__ __launch_bounds__(kBlock) void apt_fixplan(StepArgs fa, StepArgs pa)
+__global__ __launch_bounds__(kBlock) void apt_fixplan(StepArgs, StepArgs)
 {
     static_assert(kFixLanes == kBlock, "one workgroup size for both halves");
-    if ((int)blockIdx.x < fa.fix_blocks) fixup_run<K, G27>(fa, (int)blockIdx.x, fa.fix_blocks);
-    else plan_block(pa, (int)blockIdx.x - fa.fix_blocks);
+    CArgs* args = (CArgs*)__builtin_amdgcn_kernarg_segment_ptr();  // fa, pa
+    const int nfix = args[0].fix_blocks;
+    if ((int)blockIdx.x < nfix) fixup_run<K, G27>(*args_ref(args), (int)blockIdx.x, nfix);
+    else plan_block(*args_ref(args + 1), (int)blockIdx.x - nfix);
 }
 
 // Batched APTrhs_psi: the strip units of every simulation, then the rows of
@@ -159,7 +180,7 @@ template <int K, bool G27>
 __global__ __launch_bounds__(kFixLanes) void batch_fixup(BatchArgs b)
 {
     using F = FixGroup<G27>;
-    __shared__ unsigned s_fix[(kFixLanes / F::kLanes) * kFixStride];
+    __shared__ unsigned s_fix[(kFixLanes / F::kLanes) * (kFixStride + F::kIds)];
     __shared__ unsigned s_pre[kMaxBatch + 1], s_cnt[kMaxBatch], s_wave[kFixLanes / 64];
     typedef const __attribute__((address_space(4))) BatchSim CSim;
     const CSim* sims = (const CSim*)b.sims;
@@ -176,9 +197,9 @@ __global__ __launch_bounds__(kFixLanes) void batch_fixup(BatchArgs b)
                 atomicAdd(b.sims[q / segs].a.overflow + kLineWords / 2 * (q % segs), (unsigned long long)s_cnt[q]);
     const int l = threadIdx.x & (F::kLanes - 1), grp = threadIdx.x / F::kLanes;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const FixShare sh = fix_share(units, (int)blockIdx.x, (int)gridDim.x, w);
 #pragma unroll 1
-    for (unsigned u = (unsigned)(w * (int)gridDim.x + (int)blockIdx.x); u < units;
-         u += (unsigned)((int)gridDim.x * (kFixLanes / 64))) {
+    for (unsigned u = sh.first; u < sh.end; u += sh.step) {
         const int q = fixup_find(s_pre, m, u);
         const StepArgs& a = *(const StepArgs*)&sims[q / segs].a;
         const unsigned e0 = (u - s_pre[q]) * F::kPoints;
@@ -187,7 +208,7 @@ __global__ __launch_bounds__(kFixLanes) void batch_fixup(BatchArgs b)
         const float epsv = -4.0f * a.kin_delta / a_s;
         const bool on = e < s_cnt[q];
         const unsigned* list = a.fix_list + (unsigned)(q % segs * a.fix_cap);
-        fixup_group<K, G27>(a, list[on ? e : e0], on, l, s_fix + grp * kFixStride, a_s, epsv);
+        fixup_group<K, G27>(a, list[on ? e : e0], on, l, s_fix + grp * (kFixStride + F::kIds), a_s, epsv);
     }
 }
 
