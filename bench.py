@@ -11,9 +11,7 @@ Prints one JSON line:
              domain counts, as every one is updated)
   roofline   per-kernel durations of the same window (the run is replayed
              from the initial state with HIP events around every launch on
-             the context's stream): work-list plan, step kernel (in steps
-             with heavy overflow together with the edge kernel that runs
-             beside it on a second stream and joins before the fix-up),
+             the context's stream): work-list plan, step kernel,
              overflow fix-up.  The step kernel skips z planes of 64x4 column tiles
              whose stencil reaches only empty slots and whose destination is
              empty (their result is known without reading anything), so the
@@ -458,7 +456,7 @@ def main() -> int:
     t_all = avg_plan + avg_main + avg_fix
     achieved = bytes_step / (t_all * 1e-3) / 1e9
     achieved_main = bytes_step / (avg_main * 1e-3) / 1e9
-    dominant = "apt_step_tiled<%d,false>" % args.K if avg_main >= avg_fix else "apt_fixup<%d,false>" % args.K
+    dominant = "apt_step<%d,false>" % args.K if avg_main >= avg_fix else "apt_fixup<%d,false>" % args.K
     traffic, traffic_kernels = traffic_from_profiles(f"line-256x256x512:w{args.warmup}:s{args.steps}")
 
     dense = None
@@ -586,7 +584,7 @@ def main() -> int:
             "traffic": traffic,
             "traffic_by_kernel": traffic_kernels,
             "kernel": dominant,
-            "kernels": "apt_plan + apt_step_tiled (+ apt_edge beside it) + apt_fixup (one step)",
+            "kernels": "apt_plan + apt_step + apt_fixup (one step)",
             "step_ms": round(t_all, 4),
             "plan_ms": round(avg_plan, 4),
             "kernel_ms": round(avg_main, 4),

@@ -6,9 +6,9 @@
 
 namespace cupf {
 
-// The LDS path's column tiles are 64 x 4 interior points; a leftover strip at
-// the +x end at least partial_min wide is a partial tile, a narrower one goes
-// to edge items (which are computed, never listed).
+// Column tiles are 64 x 4 interior points; a leftover strip at the +x end at
+// least partial_min wide is a partial tile, a narrower one goes to the strip's
+// waves (which are computed, never listed).
 inline int cap_tiles_x(int fnx, int partial_min)
 {
     const int n = fnx - 2, t = n / 64;
