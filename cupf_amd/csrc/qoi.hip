@@ -20,12 +20,18 @@ __device__ __forceinline__ int interior_index(unsigned s, int nx, int ny, int fn
     return ((int)k + 1) * fnx * fny + ((int)j + 1) * fnx + (int)i + 1;
 }
 
-// Counts per grain id of one workgroup's run of kRun points, in LDS until its
-// end: a large grain's address otherwise takes one global atomic per wave of
+// Counts per grain id of one workgroup's run of points, in LDS until its end: a large grain's address otherwise takes one global atomic per wave of
 // it, ~17 ns each one after the other (858 us for the areas of a solid 256^3
 // window with a few large grains, 158 now).  An id that finds no place in
 // kProbe probes goes to memory at once.
-constexpr int kRun = 8192, kTable = 512, kProbe = 8;
+// Runs are as long as kRunMax where that still gives kRunGroups workgroups
+// (150 workgroups of 8192 points took 85 us for 160x96x80, 38 with shorter
+// ones).
+constexpr int kRunMax = 8192, kRunGroups = 2048, kTable = 512, kProbe = 8;
+inline int run_length(long long n)
+{
+    return (int)min((long long)kRunMax, (n / kRunGroups + kBlock) / kBlock * kBlock);
+}
 
 struct IdTable {
     int key[kTable], sum[kTable], second[kTable];
@@ -61,7 +67,7 @@ __device__ __forceinline__ int table_place(IdTable& t, int id)
 // order and usually hold one or two ids, so the lanes of one id add their
 // count at once; the lowest such lane holds the smallest scan index.
 __global__ __launch_bounds__(kBlock) void qoi_volume_kernel(const int* __restrict__ alpha, int fnx,
-                                                            int fny, int fnz, int max_id,
+                                                            int fny, int fnz, int run, int max_id,
                                                             int* counts, int* first,
                                                             unsigned long long* above)
 {
@@ -71,9 +77,9 @@ __global__ __launch_bounds__(kBlock) void qoi_volume_kernel(const int* __restric
     const int lane = threadIdx.x & 63;
     unsigned long long over = 0ull;
     table_clear(t, 0x7fffffff);
-    const unsigned end = min(n, (blockIdx.x + 1u) * (unsigned)kRun);
+    const unsigned end = min(n, (blockIdx.x + 1u) * (unsigned)run);
     // wave-uniform trip count: every lane reaches the ballots
-    for (unsigned base = blockIdx.x * (unsigned)kRun + (threadIdx.x & ~63u); base < end; base += kBlock) {
+    for (unsigned base = blockIdx.x * (unsigned)run + (threadIdx.x & ~63u); base < end; base += kBlock) {
         const unsigned s = base + lane;
         int a = 0, k;
         if (s < end) a = alpha[interior_index(s, nx, ny, fnx, fny, &k)];
@@ -293,16 +299,16 @@ __global__ __launch_bounds__(kBlock) void qoi_liquid_planes_kernel(const int* __
 // 1..ng, interior points (total) and those above the tip plane (extra), as in
 // qoi_volume_kernel.
 __global__ __launch_bounds__(kBlock) void qoi_area_kernel(const int* __restrict__ alpha, int fnx,
-                                                          int fny, int fnz, int ng, int tip,
-                                                          int* total, int* extra)
+                                                          int fny, int fnz, int run, int ng,
+                                                          int tip, int* total, int* extra)
 {
     __shared__ IdTable t;
     const int nx = fnx - 2, ny = fny - 2, nz = fnz - 2;
     const unsigned n = (unsigned)nx * ny * nz;
     const int lane = threadIdx.x & 63;
     table_clear(t, 0);
-    const unsigned end = min(n, (blockIdx.x + 1u) * (unsigned)kRun);
-    for (unsigned base = blockIdx.x * (unsigned)kRun + (threadIdx.x & ~63u); base < end; base += kBlock) {
+    const unsigned end = min(n, (blockIdx.x + 1u) * (unsigned)run);
+    for (unsigned base = blockIdx.x * (unsigned)run + (threadIdx.x & ~63u); base < end; base += kBlock) {
         const unsigned s = base + lane;
         int a = 0, k = 0;
         if (s < end) a = alpha[interior_index(s, nx, ny, fnx, fny, &k)];
@@ -346,8 +352,8 @@ hipError_t launch_qoi_volume(const int* alpha, int fnx, int fny, int fnz, int ma
                        0x7fffffff);
     hipLaunchKernelGGL(qoi_fill_kernel, dim3(1), dim3(kBlock), 0, stream, (int*)above, 2, 0);
     const long long n = (long long)(fnx - 2) * (fny - 2) * (fnz - 2);
-    hipLaunchKernelGGL(qoi_volume_kernel, dim3(max(1, cdiv(n, kRun))), dim3(kBlock), 0,
-                       stream, alpha, fnx, fny, fnz, max_id, counts, first, above);
+    hipLaunchKernelGGL(qoi_volume_kernel, dim3(max(1, cdiv(n, run_length(n)))), dim3(kBlock), 0,
+                       stream, alpha, fnx, fny, fnz, run_length(n), max_id, counts, first, above);
     return hipGetLastError();
 }
 
@@ -369,8 +375,8 @@ hipError_t launch_qoi_area(const int* alpha, int fnx, int fny, int fnz, int ng, 
     hipLaunchKernelGGL(qoi_fill_kernel, dim3(nb), dim3(kBlock), 0, stream, total, ng, 0);
     hipLaunchKernelGGL(qoi_fill_kernel, dim3(nb), dim3(kBlock), 0, stream, extra, ng, 0);
     const long long n = (long long)(fnx - 2) * (fny - 2) * (fnz - 2);
-    hipLaunchKernelGGL(qoi_area_kernel, dim3(max(1, cdiv(n, kRun))), dim3(kBlock), 0,
-                       stream, alpha, fnx, fny, fnz, ng, tip, total, extra);
+    hipLaunchKernelGGL(qoi_area_kernel, dim3(max(1, cdiv(n, run_length(n)))), dim3(kBlock), 0,
+                       stream, alpha, fnx, fny, fnz, run_length(n), ng, tip, total, extra);
     return hipGetLastError();
 }
 

@@ -23,7 +23,8 @@ def _collected(ph, arg, K, L):
 
 @pytest.mark.parametrize("n,K,bc,ids", [
     ((11, 5, 7), 8, (0, 1, 0), 60),        # odd field size, one partial row
-    ((130, 9, 20), 5, (1, 0, 1), 4000),    # two tiles and a strip, more ids than a table holds
+    ((130, 9, 20), 5, (1, 0, 1), 4000),    # two tiles and a strip, a table half full
+    ((130, 100, 90), 5, (1, 0, 1), 4000),  # longer runs, more ids than a table holds
     ((62, 30, 14), 8, (1, 1, 0), 900),     # field size a multiple of four
 ])
 def test_collect_and_counts(n, K, bc, ids):
