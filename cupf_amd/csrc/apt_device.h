@@ -227,7 +227,7 @@ __device__ __forceinline__ float slot_update(const StepArgs& a, int gid, float p
 // Searching the maximum, its position and its id one after the other took 950,
 // and passing the step's arguments by value spilled scalar registers (97 vector
 // registers against 70): 64^3 K=8 13.4 -> 11.4 us, 96x96x128 K=5 with 27 points
-// 127 -> 108, 256x256x512 133 -> 119.  One point per lane with a streaming
+// 127 -> 108, 256x256x512 133 -> 119 (89 with segments by region).  One point per lane with a streaming
 // top-K (56 dependent pushes and a second pass over the neighbours) was one
 // long chain of loads and compares, and left all but a few CUs idle: the
 // fix-up of a 64^3 K=8 start-up fell from 53-62 to 12-13 us, of 32^3 K=5 from
@@ -455,14 +455,18 @@ constexpr int kTX = 64, kTY = 4;
 __device__ __forceinline__ int act_tile_x(int i) { return (i - 1) / kTX; }
 __device__ __forceinline__ int act_tile_y(int j) { return (j - 1) / kTY; }
 
-// Append the lanes of a wave in m (not 0) to its row plane's segment of the
-// fix-up list (one atomic per wave); row: its index (capacity.h),
-// wave-uniform.
-__device__ __forceinline__ void fixup_append(const StepArgs& a, unsigned long long m, unsigned point, int row)
+// Append the lanes of a wave in m (not 0) to the fix-up list (one atomic per
+// wave); j, k: its first row, wave-uniform.  A segment holds a few y rows of
+// every plane (capacity.h), so the fix-up's XCDs, an eighth of the list each,
+// meet most of their points' neighbours in their own L2 (segments of every 64th
+// row: 640 MB fetched for the 256x256x512 start-up's list in 119 us, 356 in 89).
+__device__ __forceinline__ void fixup_append(const StepArgs& a, unsigned long long m, unsigned point, int j, int k)
 {
     const int lane = threadIdx.x & 63;
     const int leader = __ffsll((long long)m) - 1;
-    const int seg = row & (a.fix_segs - 1);
+    const unsigned nz = (unsigned)a.fnz - 2u;
+    const unsigned part = ((unsigned)(a.fny - 2) * nz + 63u) / 64u;
+    const int seg = (int)(((unsigned)(j - 1) * nz + (unsigned)(k - 1)) / part) * a.fix_segs / 64;
     unsigned base = 0;
     if (lane == leader) base = atomicAdd(a.fix_count + kLineWords * seg, (unsigned)__popcll(m));
     base = __shfl(base, leader);

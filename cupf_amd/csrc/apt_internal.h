@@ -28,8 +28,8 @@ constexpr int kPartialMin = 16;
 // Atomics of a whole grid on one address go through one at a time, ~17 ns each
 // (the start-up of a 256x256x512 simulation hands over points from ~25,000 row
 // planes of a 400 us step), so the fix-up list and the overflow count are
-// spread over kSpread counters on cache lines of their own: by row for the
-// list, whose segments hold every point of their rows.  (One counter each
+// spread over kSpread counters on cache lines of their own: the list's by
+// equal shares of the rows, y-major (capacity.h).  (One counter each
 // before; step kernel at step 6: 400 -> 266 us; 64^3 at step 10 45 -> 34; the
 // 27-point gather at 96x96x128 115 -> 80.)
 constexpr int kSpread = 64;

@@ -505,11 +505,8 @@ __device__ __forceinline__ void wide_plane(const StepArgs& a, const RowLane& r, 
     if (tx >= 0) row_mark_tile(a, r, k, tx, g.ovf != 0ull ? K : nm);
     else row_mark_strip(a, r, k, in_mask(g.ovf) ? K : list_len(g));
     if (g.ovf != 0ull) {
-        const int j = __builtin_amdgcn_readfirstlane(r.j);  // the row, or a strip wave's first
-        const int ex = strip_width(a.fnx, a.tiles_x);
-        const int row = tx >= 0 ? (k * a.fny + j) * a.tiles_x + tx
-                                : a.fnz * a.fny * a.tiles_x + k * strip_waves(ex, a.fny) + (j - 1) / (64 / max(ex, 1));
-        fixup_append(a, g.ovf, (unsigned)t.zC + (t.c >> 2), row);
+        // the row's, or a strip wave's first
+        fixup_append(a, g.ovf, (unsigned)t.zC + (t.c >> 2), __builtin_amdgcn_readfirstlane(r.j), k);
     }
 }
 

@@ -40,16 +40,22 @@ inline int cap_strip_waves(int fnx, int fny, int partial_min)
     return ex > 0 ? (fny - 2 + 64 / ex - 1) / (64 / ex) : 0;
 }
 
-// Entries of one of `segs` (a power of two up to 64) segments of that list:
-// the points of a row plane (64 at most) go to the segment of its index, the
-// tiles' rows first, (k * fny + j) * tiles + tile, then the strip's waves,
-// k * waves + wave.  A quarter as many segments hold four of the full split's
-// each, so every split fits the full one's list.
+// Entries of one of `segs` (a power of two up to 64) segments of that list: the
+// interior rows, y-major ((j - 1) * (fnz - 2) + k - 1), are cut into 64 equal
+// parts, and a wave's points (64 at most: a row of a tile, or its part of the
+// strip) go to the part of its first row.  A quarter as many segments hold four
+// parts each, so every split fits the full one's list.
 inline long long fix_segment_cap(int fnx, int fny, int fnz, int partial_min, int segs)
 {
-    const long long rows = (long long)cap_tiles_x(fnx, partial_min) * fny * fnz +
-                           (long long)cap_strip_waves(fnx, fny, partial_min) * fnz;
-    return (rows + 63) / 64 * 64 * (64 / segs);
+    const long long nz = fnz - 2, part = ((fny - 2) * nz + 63) / 64;
+    long long waves = cap_tiles_x(fnx, partial_min) * part;
+    if (cap_strip_waves(fnx, fny, partial_min)) {
+        const int per = 64 / ((fnx - 2) % 64);  // y rows of a strip wave
+        const long long js = (part + nz - 1) / nz + 1;  // y rows that a part touches at most
+        const long long strip = (js + per - 1) / per * nz;
+        waves += strip < part ? strip : part;
+    }
+    return waves * 64 * (64 / segs);
 }
 
 }  // namespace cupf
