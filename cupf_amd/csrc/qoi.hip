@@ -22,12 +22,15 @@ __device__ __forceinline__ int interior_index(unsigned s, int nx, int ny, int fn
 
 // Counts per grain id of one workgroup's run of points, in LDS until its end: a large grain's address otherwise takes one global atomic per wave of
 // it, ~17 ns each one after the other (858 us for the areas of a solid 256^3
-// window with a few large grains, 158 now).  An id that finds no place in
+// window with a few large grains, 180 now).  An id that finds no place in
 // kProbe probes goes to memory at once.
 // Runs are as long as kRunMax where that still gives kRunGroups workgroups
 // (150 workgroups of 8192 points took 85 us for 160x96x80, 38 with shorter
-// ones).
-constexpr int kRunMax = 8192, kRunGroups = 2048, kTable = 512, kProbe = 8;
+// ones).  Longer runs save atomics of large grains but leave a thin layer of
+// many small ones to few workgroups: with 512 / 1024 / 2048 / 4096 / 8192, the
+// area call of that window takes 528 / 344 / 265 / 241 / 243 us, that of a
+// 256x256x512 start-up 202 / 187 / 182 / 217 / 383 (191 with an atomic per wave).
+constexpr int kRunMax = 2048, kRunGroups = 2048, kTable = 512, kProbe = 8;
 inline int run_length(long long n)
 {
     return (int)min((long long)kRunMax, (n / kRunGroups + kBlock) / kBlock * kBlock);
