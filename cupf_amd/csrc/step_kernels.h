@@ -15,9 +15,10 @@ namespace {
 // A wave's place among W waves that take units u, u + W, ...: kXcdRun
 // neighbouring places on one XCD (workgroups go to the 8 XCDs in turn), so that
 // the rows of a tile plane and its neighbours in x meet in one L2, and every
-// XCD has the same share of a last, partly filled round.  (1 / 4 / 16: 407 /
-// 405 / 401 us for the 256x256x512 start-up, 79 / 79 / 77 us at step 1500; one
-// run of W / 8 per XCD: 460 and 86 us, the last round falls on few XCDs.)
+// XCD has the same share of a last, partly filled round.  (Runs of 4 / 16 / 64 /
+// 128 / 512: 243 / 241 / 249 / 284 / 305 us for the 256x256x512 start-up, 57 /
+// 55 / 57 / 64 / 66 at step 1500, 1014 / 1000 / 987 / 987 / 1168 for a solid
+// 256^3 window, whose line fetches beyond the L2s fall by 39 %.)
 constexpr unsigned kXcdRun = 16u;
 __device__ __forceinline__ unsigned row_place(unsigned W)
 {
@@ -30,7 +31,8 @@ __device__ __forceinline__ unsigned row_place(unsigned W)
 // row r of listed chunk e as unit 4 e + r.  Waves take units by position: an
 // atomic claim per unit (or only for the last two rounds) costs ~17 ns each on
 // one address, which the start-up's 36,000 row planes of 4 us do not afford
-// (256x256x512: 407 us by position, 498 with claims in the last two rounds).
+// (256x256x512, before the entries got cheaper: 407 us by position, 498 with
+// claims in the last two rounds).
 template <int K, bool G27>
 __global__ __launch_bounds__(kRowLanes, 4) void apt_step(StepArgs)
 {
