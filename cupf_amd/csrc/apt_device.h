@@ -266,7 +266,7 @@ __device__ __forceinline__ int group_min(int v)
     return G27 ? min(v, dpp_get<0x140>(v)) : v;
 }
 
-// phi as an integer of the same order (-0 as +0, below every float: kNoKey).
+// phi, no NaN, as an integer of the same order (-0 as +0, below every float: kNoKey).
 constexpr int kNoKey = (int)0x80000000;
 __device__ __forceinline__ int phi_key(float x)
 {
@@ -357,17 +357,25 @@ __device__ __forceinline__ void fixup_group(const StepArgs& a, unsigned C, bool 
     // An entry's key is its phi's order (32 bits) and below it the scan position
     // counted backwards (8 bits) in a double's mantissa, so one maximum finds
     // the largest phi and the earliest entry holding it; entries out of the
-    // ranking lie below 1.0.  Its id is then looked up in LDS.
+    // ranking lie below 1.0.  Its id is then looked up in LDS.  A NaN ranks below
+    // every other entry, but nothing is larger than it either: as the first
+    // entry left it is taken, whatever the maximum (`nan`: the wave has one; the
+    // tests for it cost 99.1 -> 100.4 us for 96x96x128 K=5 with 27 points, 11.6 ->
+    // 11.7 at 64^3).
     const int pos0 = l * K;  // scan position of entry e: pos0 + (16 K for the second position) + slot
     unsigned* ids = sc + kFixStride;
+    unsigned odd = 0u;  // this lane's NaN entries
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int pos = pos0 + (e / K) * 16 * K + e % K;
-        const unsigned u = (unsigned)phi_key(ph[e]) ^ 0x80000000u;
+        const bool ordered = ph[e] == ph[e];
+        const unsigned u = ordered ? (unsigned)phi_key(ph[e]) ^ 0x80000000u : 0u;
+        odd |= id[e] != -1 && !ordered ? 1u << e : 0u;
         key[e] = rank_key(id[e] != -1 ? kRankOne | u >> 12 : 0u, u << 20 | (unsigned)(255 - pos) << 12);
         ids[pos] = (unsigned)id[e];
     }
     wave_lds_fence();
+    const bool nan = __ballot(odd != 0u) != 0ull;
     int nk = 0;
 #pragma unroll 1
     for (int r = 0; r < K; ++r) {
@@ -376,7 +384,18 @@ __device__ __forceinline__ void fixup_group(const StepArgs& a, unsigned C, bool 
         for (int e = 1; e < E; ++e) m = rank_max(m, key[e]);
         m = group_rank_max<G27>(m);
         const bool live = (unsigned)__double2hiint(m) >= kRankOne;
-        const int top = 255 - ((unsigned)__double2loint(m) >> 12 & 255u);
+        int top = 255 - ((unsigned)__double2loint(m) >> 12 & 255u);
+        if (nan) {
+            unsigned left = 0u;  // its entries not taken
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                left |= (unsigned)__double2hiint(key[e]) >= kRankOne ? 1u << e : 0u;
+            // 2 * position of the first entry left, + 1 for a NaN
+            const int e = __ffs((int)left) - 1;
+            int first = left ? 2 * (pos0 + (e / K) * 16 * K + e % K) + (int)(odd >> e & 1u) : 0x7fffffff;
+            first = group_min<G27>(first);
+            if (live && (first & 1)) top = first >> 1;
+        }
         const int kid = live ? (int)ids[top] : kNoKey;
         nk += live ? 1 : 0;
         // the id's entries leave the ranking; its phi at this lane's stencil

@@ -112,8 +112,14 @@ __device__ __forceinline__ void fixup_run(const StepArgs& a, int blk, int nblk)
     }
 }
 
+// Waves per SIMD that the registers of the 7-point fix-up have to leave room
+// for: as many as its LDS lets in (unasked, the cold NaN branch took 8 more
+// vector registers, 78, and a wave away).  The 27-point kernels get there by
+// themselves (94 registers at K = 5) or not at all (143 at K = 8).
+constexpr int fix_waves(bool g27) { return g27 ? 1 : 7; }
+
 template <int K, bool G27>
-__global__ __launch_bounds__(kFixLanes) void apt_fixup(StepArgs)
+__global__ __launch_bounds__(kFixLanes, fix_waves(G27)) void apt_fixup(StepArgs)
 {
     CArgs* a = (CArgs*)__builtin_amdgcn_kernarg_segment_ptr();
     fixup_run<K, G27>(*args_ref(a), (int)blockIdx.x, (int)gridDim.x);
@@ -127,7 +133,7 @@ __global__ __launch_bounds__(kFixLanes) void apt_fixup(StepArgs)
 // the one after (three sets in turn), so the two halves need no order
 // between them.  Saves one launch and its dispatch gap per step.
 template <int K, bool G27>
-__global__ __launch_bounds__(kBlock) void apt_fixplan(StepArgs, StepArgs)
+__global__ __launch_bounds__(kBlock, fix_waves(G27)) void apt_fixplan(StepArgs, StepArgs)
 {
     static_assert(kFixLanes == kBlock, "one workgroup size for both halves");
     CArgs* args = (CArgs*)__builtin_amdgcn_kernarg_segment_ptr();  // fa, pa
@@ -178,8 +184,9 @@ __global__ __launch_bounds__(kRowLanes, 4) void batch_step(BatchArgs b)
 // Batched fix-up: the list segments of all simulations (fix_segs each) form
 // one index space of wave units (prefix sums in LDS) that the grid strides
 // over, so long and short lists alike are spread over every workgroup.
+// (Four waves per SIMD: 126 registers for 27 points at K = 8, 138 unasked.)
 template <int K, bool G27>
-__global__ __launch_bounds__(kFixLanes) void batch_fixup(BatchArgs b)
+__global__ __launch_bounds__(kFixLanes, 4) void batch_fixup(BatchArgs b)
 {
     using F = FixGroup<G27>;
     __shared__ unsigned s_fix[(kFixLanes / F::kLanes) * (kFixStride + F::kIds)];
