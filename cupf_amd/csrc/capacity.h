@@ -1,7 +1,7 @@
 // capacity.h -- worst-case entries of a step's work lists, recomputed from
 // the grid and the chunk depth alone (not from the values pf_create derived
-// and stored), for the host check before every launch.  Plain C++: the CPU
-// tests compile it on its own.
+// and stored), for the host check before every launch; and the range of the
+// epochs.  Plain C++: the CPU tests compile it on its own.
 #pragma once
 
 namespace cupf {
@@ -57,5 +57,17 @@ inline long long fix_segment_cap(int fnx, int fny, int fnz, int partial_min, int
     }
     return waves * 64 * (64 / segs);
 }
+
+// The epoch counter's limit: row words hold an epoch and 4 bits of bound, and
+// a few epochs are taken between two looks at the counter (new states).
+constexpr unsigned kEpochMax = 0x07ffffffu;
+
+// Whether the counter may still take `ahead` epochs; the maps are renewed
+// otherwise, and it starts again.
+inline bool epochs_left(unsigned ctr, unsigned ahead) { return ahead < kEpochMax && ctr < kEpochMax - ahead; }
+
+// Steps of a batched run that has `left` to go before the next look at its
+// members' counters (a run takes an epoch per step).
+inline int epoch_run(int left) { return left < (1 << 26) ? left : 1 << 26; }
 
 }  // namespace cupf

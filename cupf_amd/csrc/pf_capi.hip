@@ -325,16 +325,13 @@ hipError_t collect_fields(pf_ctx* c, int b, bool halo, int clear_alpha)
     return launch_collect(c->ph[b], c->arg[b], c->phi, c->alpha, c->L, p.K, clear_alpha, rows, c->stream);
 }
 
-// The epoch counter's limit: row words hold an epoch and 4 bits of bound.
-constexpr unsigned kEpochMax = 0x07ffffffu;
-
 size_t row_words(const pf_params& p) { return (size_t)((p.fnx - 2 + 63) / 64) * p.fny * p.fnz; }
 
 // Before the epoch counter could pass its limit within the next `ahead`
 // steps: clear the maps and rebuild them.
 hipError_t act_renew_if_needed(pf_ctx* c, unsigned ahead = 1u)
 {
-    if (c->ep_ctr < kEpochMax - ahead) return hipSuccess;
+    if (epochs_left(c->ep_ctr, ahead)) return hipSuccess;
     const size_t n = (size_t)c->ntiles * c->p.fnz;
     hipError_t e;
     for (int b = 0; b < 2; ++b) {
@@ -868,7 +865,7 @@ static int step_impl(pf_ctx* c, int nsteps, int first_step, int flags)
         c->cur = 1 - c->cur;
         // an activity-map renewal (epoch counter near its end) must come
         // between this step and the next plan: no fused launch then
-        have = !nucl && s + 1 < end && c->ep_ctr < kEpochMax - 1u;
+        have = !nucl && s + 1 < end && epochs_left(c->ep_ctr, 1u);
         if (have) {
             a = make_step_args(c, c->cur, (s + 1) * p.dt * p.tau0, use_iuc);
         }
@@ -1461,7 +1458,15 @@ int pf_batch_step(pf_batch* b, int nsteps, const int* first_step, int flags)
     const bool use_graph = (flags & PF_BATCH_GRAPH) != 0;
     std::vector<int> fs(first_step, first_step + b->ctxs.size());
     int left = nsteps;
-    if (!(flags & PF_BATCH_AUTOTUNE)) return batch_run(b, left, fs, use_iuc, use_graph);
+    if (!(flags & PF_BATCH_AUTOTUNE)) {
+        int rc = PF_OK;
+        while (left > 0 && rc == PF_OK) {
+            const int seg = epoch_run(left);
+            rc = batch_run(b, seg, fs, use_iuc, use_graph);
+            left -= seg;
+        }
+        return rc;
+    }
     // The chunk depth changes only how the work is cut, never the results.
     // Every kTuneEvery steps, time a few real steps with each candidate and
     // keep the fastest for the rest of the segment: the best depth moves as
