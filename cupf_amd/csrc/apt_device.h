@@ -485,12 +485,12 @@ __device__ __forceinline__ void fixup_append(const StepArgs& a, unsigned long lo
     const int leader = __ffsll((long long)m) - 1;
     const unsigned nz = (unsigned)a.fnz - 2u;
     const unsigned part = ((unsigned)(a.fny - 2) * nz + 63u) / 64u;
-    const int seg = (int)(((unsigned)(j - 1) * nz + (unsigned)(k - 1)) / part) * a.fix_segs / 64;
+    const int seg = (int)(((unsigned)(j - 1) * nz + (unsigned)(k - 1)) / part) >> a.fix_shift;
     unsigned base = 0;
     if (lane == leader) base = atomicAdd(a.fix_count + kLineWords * seg, (unsigned)__popcll(m));
     base = __shfl(base, leader);
     if ((m >> lane) & 1ull)
-        a.fix_list[(unsigned)(seg * a.fix_cap) + base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = point;
+        a.fix_list[fix_segment_base(seg, a.fix_shift, a.fix_cap) + base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = point;
 }
 
 // Counts of m fix-up segments (count(q), m <= kMaxBatch) into s_cnt and the

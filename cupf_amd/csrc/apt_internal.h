@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "capacity.h"
+
 namespace cupf {
 
 // LS = -0.995 (3DgrainMPI/APTPhaseField.cu:25) is a double literal in the
@@ -53,11 +55,12 @@ struct StepArgs {
     const float* psi_mac;  // type-4 thermal field
     unsigned long long* overflow;  // points with > K distinct ids: the sum of kSpread counts,
                                    // kLineWords / 2 apart
-    // Interior points left to the fix-up pass: fix_segs segments (a power of
-    // two) of fix_cap entries; a row plane's points go to the segment of its
-    // index (capacity.h).
+    // Interior points left to the fix-up pass: 64 equal parts of fix_cap entries
+    // by the index of a row plane (capacity.h), a segment of the list each, or
+    // (a batch) 2^fix_shift of them to a segment.
     unsigned* fix_list;
-    int fix_segs, fix_cap;
+    int fix_shift;
+    unsigned fix_cap;
     // Counters of this step: fix_count[kLineWords * s] entries in segment s;
     // wl_count (below) points into the same set (kSetWords).  Steps take three sets in turn;
     // cnt_next is the next step's, cleared by this step's plan kernel (its

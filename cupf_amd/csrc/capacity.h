@@ -33,29 +33,32 @@ inline long long worst_fix_entries(int fnx, int fny, int fnz)
     return (long long)(fnx - 2) * (fny - 2) * (fnz - 2);
 }
 
-// Waves of the +x strip of one plane (its columns, 64 / width rows to a wave).
-inline int cap_strip_waves(int fnx, int fny, int partial_min)
-{
-    const int ex = (fnx - 2) - 64 * cap_tiles_x(fnx, partial_min);
-    return ex > 0 ? (fny - 2 + 64 / ex - 1) / (64 / ex) : 0;
-}
-
 // Entries of one of `segs` (a power of two up to 64) segments of that list: the
 // interior rows, y-major ((j - 1) * (fnz - 2) + k - 1), are cut into 64 equal
-// parts, and a wave's points (64 at most: a row of a tile, or its part of the
-// strip) go to the part of its first row.  A quarter as many segments hold four
-// parts each, so every split fits the full one's list.
+// parts, and a wave's points (the columns of a row of a tile, or its part of
+// the strip: 64 / width rows) go to the part of its first row.  A quarter as
+// many segments hold four parts each, so every split fits the full one's list.
+// (64 entries to a wave, whatever its columns, made the list 2.05 times the
+// interior at 32^3 and 4 times for 16 columns; now 1.06 and 1.0.)
 inline long long fix_segment_cap(int fnx, int fny, int fnz, int partial_min, int segs)
 {
-    const long long nz = fnz - 2, part = ((fny - 2) * nz + 63) / 64;
-    long long waves = cap_tiles_x(fnx, partial_min) * part;
-    if (cap_strip_waves(fnx, fny, partial_min)) {
-        const int per = 64 / ((fnx - 2) % 64);  // y rows of a strip wave
+    const long long ny = fny - 2, nz = fnz - 2, part = (ny * nz + 63) / 64;
+    const int tiled = 64 * cap_tiles_x(fnx, partial_min), ex = fnx - 2 - tiled;
+    long long points = part * (ex > 0 ? tiled : fnx - 2);
+    if (ex > 0) {
+        const long long per = 64 / ex;  // y rows of a strip wave
         const long long js = (part + nz - 1) / nz + 1;  // y rows that a part touches at most
-        const long long strip = (js + per - 1) / per * nz;
-        waves += strip < part ? strip : part;
+        const long long waves = (js + per - 1) / per * nz;
+        points += (waves < part ? waves : part) * ex * (per < ny ? per : ny);
     }
-    return waves * 64 * (64 / segs);
+    return points * (64 / segs);
+}
+
+// First entry of segment `seg` of 2^shift parts of `cap` entries.  The list of a
+// narrow, long grid (4 x 66 x 1.6 M points, one strip) passes 32 bits.
+constexpr unsigned long long fix_segment_base(int seg, int shift, unsigned cap)
+{
+    return ((unsigned long long)seg << shift) * cap;
 }
 
 // The epoch counter's limit: row words hold an epoch and 4 bits of bound, and

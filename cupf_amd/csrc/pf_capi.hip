@@ -22,7 +22,6 @@
 
 #include "../../include/pf_capi.h"
 #include "apt_internal.h"
-#include "capacity.h"
 
 using namespace cupf;
 
@@ -43,7 +42,7 @@ struct pf_ctx {
     float* phi = nullptr;           // collect target
     int* alpha = nullptr;           // collect target / initial alpha (alpha_m)
     unsigned long long* counters = nullptr;  // overflow counts (kSpread lines), then nucleation events
-    unsigned* fix_list = nullptr;   // overflow fix-up list, one entry per interior point
+    unsigned* fix_list = nullptr;   // overflow fix-up list, kSpread segments (capacity.h)
     unsigned* fix_count = nullptr;  // three counter sets (kSetWords each), used by steps in turn
     long long* sums = nullptr;
     std::vector<long long> h_sums;
@@ -168,8 +167,8 @@ StepArgs make_step_args(pf_ctx* c, int src, float t, int use_iuc)
     a.psi_mac = c->psi_mac;
     a.overflow = c->counters;
     a.fix_list = c->fix_list;
-    a.fix_segs = kSpread;
-    a.fix_cap = (int)fix_segment_cap(p.fnx, p.fny, p.fnz, kPartialMin, kSpread);
+    a.fix_shift = 0;
+    a.fix_cap = (unsigned)fix_segment_cap(p.fnx, p.fny, p.fnz, kPartialMin, kSpread);
     {
         // three sets in turn (advanced once the launch succeeded): this step's
         // plan clears the next step's set, whose last user (two steps back) has
@@ -416,8 +415,7 @@ int batch_upload(pf_batch* b, const std::vector<int>& first_step, int use_iuc, B
         m.a.nzchunk = (p.fnz - 2 + b->kchunk - 1) / b->kchunk;
         m.a.step_blocks = b->step_blocks;
         m.a.fix_blocks = b->fix_blocks;
-        m.a.fix_segs = b->fix_segs;
-        m.a.fix_cap = (int)fix_segment_cap(p.fnx, p.fny, p.fnz, kPartialMin, b->fix_segs);
+        while (b->fix_segs << m.a.fix_shift < kSpread) ++m.a.fix_shift;
         for (int q = 0; q < 2; ++q) {
             m.ph[q] = c->ph[q];
             m.arg[q] = c->arg[q];

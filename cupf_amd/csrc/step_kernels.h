@@ -107,7 +107,7 @@ __device__ __forceinline__ void fixup_run(const StepArgs& a, int blk, int nblk)
         const unsigned e0 = (u - s_pre[seg]) * F::kPoints;
         const unsigned e = e0 + (unsigned)(grp & (F::kPoints - 1));
         const bool on = e < s_cnt[seg];
-        const unsigned* list = a.fix_list + (unsigned)(seg * a.fix_cap);
+        const unsigned* list = a.fix_list + fix_segment_base(seg, 0, a.fix_cap);
         fixup_group<K, G27>(a, list[on ? e : e0], on, l, s_fix + grp * (kFixStride + F::kIds), a_s, epsv);
     }
 }
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(kFixLanes, 4) void batch_fixup(BatchArgs b)
         const float a_s = 1.0f + 3.0f * a.kin_delta;
         const float epsv = -4.0f * a.kin_delta / a_s;
         const bool on = e < s_cnt[q];
-        const unsigned* list = a.fix_list + (unsigned)(q % segs * a.fix_cap);
+        const unsigned* list = a.fix_list + fix_segment_base(q % segs, a.fix_shift, a.fix_cap);
         fixup_group<K, G27>(a, list[on ? e : e0], on, l, s_fix + grp * (kFixStride + F::kIds), a_s, epsv);
     }
 }
