@@ -61,6 +61,22 @@ constexpr unsigned long long fix_segment_base(int seg, int shift, unsigned cap)
     return ((unsigned long long)seg << shift) * cap;
 }
 
+// Elements of a context's large arrays: a slot buffer's phi or ids, a field, the
+// fix-up list, a buffer's activity and row maps, the work list.
+struct ContextSizes {
+    long long slots, field, fix, act, row, items;
+};
+inline ContextSizes context_sizes(int fnx, int fny, int fnz, int K, int kchunk, int partial_min)
+{
+    const long long field = (long long)fnx * fny * fnz, columns = (fnx - 2 + 63) / 64;
+    return {K * field,
+            field,
+            64 * fix_segment_cap(fnx, fny, fnz, partial_min, 64),
+            columns * cap_tiles_y(fny) * fnz,
+            columns * fny * fnz,
+            worst_list_items(fnx, fny, fnz, kchunk, partial_min) + 1};
+}
+
 // The epoch counter's limit: row words hold an epoch and 4 bits of bound, and
 // a few epochs are taken between two looks at the counter (new states).
 constexpr unsigned kEpochMax = 0x07ffffffu;

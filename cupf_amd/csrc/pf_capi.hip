@@ -53,7 +53,7 @@ struct pf_ctx {
     float* ball = nullptr;
     int cnx = 0, cny = 0, cnz = 0;
     unsigned long long ncall = 0;
-    long long wl_alloc = 0;         // entries allocated for wl_item / wl_need / wl_act
+    long long wl_alloc = 0;         // entries allocated for wl_item / wl_need
     long long fix_alloc = 0;        // entries allocated for fix_list
     int kchunk = 1;                 // z planes per work item
     // Activity map per buffer (one word per 64x4 column tile and z plane), row
@@ -324,19 +324,17 @@ hipError_t collect_fields(pf_ctx* c, int b, bool halo, int clear_alpha)
     return launch_collect(c->ph[b], c->arg[b], c->phi, c->alpha, c->L, p.K, clear_alpha, rows, c->stream);
 }
 
-size_t row_words(const pf_params& p) { return (size_t)((p.fnx - 2 + 63) / 64) * p.fny * p.fnz; }
-
 // Before the epoch counter could pass its limit within the next `ahead`
 // steps: clear the maps and rebuild them.
 hipError_t act_renew_if_needed(pf_ctx* c, unsigned ahead = 1u)
 {
     if (epochs_left(c->ep_ctr, ahead)) return hipSuccess;
-    const size_t n = (size_t)c->ntiles * c->p.fnz;
+    const pf_params& p = c->p;
+    const ContextSizes n = context_sizes(p.fnx, p.fny, p.fnz, p.K, c->kchunk, kPartialMin);
     hipError_t e;
     for (int b = 0; b < 2; ++b) {
-        if ((e = hipMemsetAsync(c->act[b], 0, n * sizeof(unsigned), c->stream)) != hipSuccess) return e;
-        if ((e = hipMemsetAsync(c->row[b], 0, row_words(c->p) * sizeof(unsigned), c->stream)) != hipSuccess)
-            return e;
+        if ((e = hipMemsetAsync(c->act[b], 0, (size_t)n.act * sizeof(unsigned), c->stream)) != hipSuccess) return e;
+        if ((e = hipMemsetAsync(c->row[b], 0, (size_t)n.row * sizeof(unsigned), c->stream)) != hipSuccess) return e;
     }
     c->ep_ctr = 1u;
     if ((e = act_rebuild(c, 0)) != hipSuccess) return e;
@@ -600,21 +598,21 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
         return bail(fail(PF_E_HIP, "hipStreamCreate failed"));
     if (hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess)
         return bail(fail(PF_E_HIP, "hipEventCreate failed"));
-    const size_t nst = (size_t)L * p.K;
+    const ContextSizes n = context_sizes(p.fnx, p.fny, p.fnz, p.K, c->kchunk, kPartialMin);
+    const size_t nst = (size_t)n.slots;
     for (int b = 0; b < 2; ++b) {
         if ((rc = dalloc(&c->ph[b], nst)) || (rc = dalloc(&c->arg[b], nst))) return bail(rc);
     }
+    c->fix_alloc = n.fix;
+    c->wl_alloc = n.items;
     if ((rc = dalloc(&c->x, p.fnx)) || (rc = dalloc(&c->y, p.fny)) || (rc = dalloc(&c->z, p.fnz)) ||
-        (rc = dalloc(&c->zbuf, p.fnz)) || (rc = dalloc(&c->phi0, (size_t)L)) ||
-        (rc = dalloc(&c->phi, (size_t)L)) || (rc = dalloc(&c->alpha, (size_t)L)) ||
+        (rc = dalloc(&c->zbuf, p.fnz)) || (rc = dalloc(&c->phi0, (size_t)n.field)) ||
+        (rc = dalloc(&c->phi, (size_t)n.field)) || (rc = dalloc(&c->alpha, (size_t)n.field)) ||
         (rc = dalloc(&c->counters, kOverflowWords + 1)) || (rc = dalloc(&c->sums, p.fnz)) ||
-        (rc = dalloc(&c->fix_list, (size_t)(c->fix_alloc = kSpread * fix_segment_cap(p.fnx, p.fny, p.fnz, kPartialMin, kSpread)))) ||
-        (rc = dalloc(&c->fix_count, 3 * kSetWords)) ||
-        (rc = dalloc(&c->act[0], (size_t)c->ntiles * p.fnz)) ||
-        (rc = dalloc(&c->act[1], (size_t)c->ntiles * p.fnz)) ||
-        (rc = dalloc(&c->row[0], row_words(p))) || (rc = dalloc(&c->row[1], row_words(p))) ||
-        (rc = dalloc(&c->wl_item, (size_t)(c->wl_alloc = (long long)c->nzchunk * c->items_chunk + 1))) ||
-        (rc = dalloc(&c->wl_need, (size_t)c->nzchunk * c->items_chunk + 1)))
+        (rc = dalloc(&c->fix_list, (size_t)n.fix)) || (rc = dalloc(&c->fix_count, 3 * kSetWords)) ||
+        (rc = dalloc(&c->act[0], (size_t)n.act)) || (rc = dalloc(&c->act[1], (size_t)n.act)) ||
+        (rc = dalloc(&c->row[0], (size_t)n.row)) || (rc = dalloc(&c->row[1], (size_t)n.row)) ||
+        (rc = dalloc(&c->wl_item, (size_t)n.items)) || (rc = dalloc(&c->wl_need, (size_t)n.items)))
         return bail(rc);
     c->h_sums.resize(p.fnz);
     for (int b = 0; b < 2; ++b) {
@@ -625,10 +623,10 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
     if (hipMemsetAsync(c->counters, 0, (kOverflowWords + 1) * sizeof(unsigned long long), c->stream) != hipSuccess ||
         hipMemsetAsync(c->fix_count, 0, 3 * kSetWords * sizeof(unsigned), c->stream) != hipSuccess ||
         hipMemsetAsync(c->alpha, 0, L * sizeof(int), c->stream) != hipSuccess ||
-        hipMemsetAsync(c->act[0], 0, (size_t)c->ntiles * p.fnz * sizeof(unsigned), c->stream) != hipSuccess ||
-        hipMemsetAsync(c->act[1], 0, (size_t)c->ntiles * p.fnz * sizeof(unsigned), c->stream) != hipSuccess ||
-        hipMemsetAsync(c->row[0], 0, row_words(p) * sizeof(unsigned), c->stream) != hipSuccess ||
-        hipMemsetAsync(c->row[1], 0, row_words(p) * sizeof(unsigned), c->stream) != hipSuccess ||
+        hipMemsetAsync(c->act[0], 0, (size_t)n.act * sizeof(unsigned), c->stream) != hipSuccess ||
+        hipMemsetAsync(c->act[1], 0, (size_t)n.act * sizeof(unsigned), c->stream) != hipSuccess ||
+        hipMemsetAsync(c->row[0], 0, (size_t)n.row * sizeof(unsigned), c->stream) != hipSuccess ||
+        hipMemsetAsync(c->row[1], 0, (size_t)n.row * sizeof(unsigned), c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
         return bail(fail(PF_E_HIP, "initial fill failed"));
     *out = c;

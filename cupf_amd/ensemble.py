@@ -40,12 +40,48 @@ class SimSpec:
     arrival: float = 0.0  # s after the start of a served stream
 
     def footprint(self, K: int = 8) -> int:
-        """Device bytes of a context: two K-slot buffers (phi + id), the single
-        fields and the fix-up list."""
-        fnx, fny, fnz = self.n[0] + 3, self.n[1] + 3, self.n[2] + 3
-        L = fnx * fny * fnz
-        interior = (fnx - 2) * (fny - 2) * (fnz - 2)
-        return 16 * K * L + 12 * L + 4 * interior
+        """Device bytes that the simulation takes as a member of a batch: the
+        allocations of its context, as large as the device makes them, and its
+        entries of the batch's work list."""
+        lists = 16 * (_context_sizes(self.n, K, 2)["items"] - 1)  # the batch's smallest chunk depth
+        return lists + sum(_on_device(b) for b in _context_allocations(self.n, K, self.grains))
+
+
+def _context_sizes(n, K: int, kchunk: int = 1) -> dict:
+    """Elements of a context's large arrays, as context_sizes of csrc/capacity.h
+    has them (kPartialMin = 16)."""
+    fnx, fny, fnz = n[0] + 3, n[1] + 3, n[2] + 3
+    ix, iy, iz = fnx - 2, fny - 2, fnz - 2
+    tiles = ix // 64 + (1 if ix % 64 >= 16 else 0)
+    strip = ix - 64 * tiles
+    part = -(-iy * iz // 64)
+    cap = part * (64 * tiles if strip > 0 else ix)
+    if strip > 0:
+        per = 64 // strip
+        rows = -(-part // iz) + 1
+        cap += min(-(-rows // per) * iz, part) * strip * min(per, iy)
+    columns, tiles_y = -(-ix // 64), -(-iy // 4)
+    return dict(slots=K * fnx * fny * fnz, field=fnx * fny * fnz, fix=64 * cap, act=columns * tiles_y * fnz,
+                row=columns * fny * fnz, items=tiles * tiles_y * -(-iz // kchunk) + 1)
+
+
+def _context_allocations(n, K: int, grains: int) -> list:
+    """Bytes of the allocations that a context makes (pf_create, the
+    orientation table)."""
+    s = _context_sizes(n, K)
+    fnx, fny, fnz = n[0] + 3, n[1] + 3, n[2] + 3
+    per_buffer = [4 * s["slots"], 4 * s["slots"], 4 * s["act"], 4 * s["row"]]
+    counters = [8 * 1025, 3 * 4 * 65 * 32]  # the overflow counts and events, three counter sets
+    return (per_buffer * 2 + [4 * s["field"]] * 3 + [4 * s["fix"], 4 * s["items"], 8 * s["items"]] + counters
+            + [4 * fnx, 4 * fny, 4 * fnz, 4 * fnz, 8 * fnz, 48 * (grains + 1)])
+
+
+def _on_device(b: int) -> int:
+    """An allocation's size on the device: whole 64 KiB, one MiB from half of
+    one on, whole 2 MiB from one on (free memory before and after 20 contexts of
+    16^3 to 128x128x256: 0 to 6 % below the sum of these)."""
+    unit = 1 << 16 if b < 1 << 19 else 1 << 20 if b < 1 << 20 else 1 << 21
+    return -(-b // unit) * unit
 
 
 def _grains(n) -> int:
