@@ -15,13 +15,11 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
-#include <thread>
 #include <vector>
-
-#include <sys/mman.h>
 
 #include "../../include/pf_capi.h"
 #include "apt_internal.h"
+#include "host_pages.h"
 
 using namespace cupf;
 
@@ -748,29 +746,6 @@ int pf_reinit_from_collect(pf_ctx* c)
     HIPCHK(init_state(c));
     HIPCHK(hipStreamSynchronize(c->stream));
     return PF_OK;
-}
-
-// Makes the pages of a large result buffer present while the device still
-// works on what goes there.  A fresh array's pages are zeroed one fault at a
-// time, inside the copy otherwise, which then runs at 10 GB/s instead of 25.
-// The contents stay; where the kernel or the mapping does not take the advice,
-// the copy faults as before.  Small buffers are left to the copy.
-static void make_present(std::initializer_list<std::pair<void*, size_t>> bufs)
-{
-    constexpr size_t kSmall = 8u << 20, kPage = 4096, kThreads = 4;
-    std::vector<std::thread> pool;
-    try {
-        for (auto [p, bytes] : bufs) {
-            if (!p || bytes < kSmall) continue;
-            const uintptr_t lo = ((uintptr_t)p + kPage - 1) / kPage * kPage;
-            const uintptr_t hi = ((uintptr_t)p + bytes) / kPage * kPage;
-            const size_t part = ((hi - lo) / kThreads + kSmall - 1) / kSmall * kSmall;
-            for (uintptr_t q = lo; q < hi; q += part)
-                pool.emplace_back([=] { (void)madvise((void*)q, std::min<size_t>(part, hi - q), 23 /* MADV_POPULATE_WRITE */); });
-        }
-    } catch (...) {  // no thread to be had: the copy does the rest
-    }
-    for (auto& t : pool) t.join();
 }
 
 int pf_upload_state(pf_ctx* c, int which, const float* ph, const int* arg)
