@@ -12,13 +12,12 @@ namespace cupf {
 // LS = -0.995 (3DgrainMPI/APTPhaseField.cu:25) is a double literal in the
 // reference: every `phi > LS` test compares in double.
 constexpr double kLS = -0.995;
-// Slot kill threshold (3DgrainMPI/APTPhaseField.cu:341), also a double compare.
-constexpr double kKill = -0.9999;
-// The same two comparisons in float, exact for every float x:
-// (double)x > -0.995 <=> x > -0.995f, because -0.995f is the largest float not
-// above -0.995; (double)x < -0.9999 <=> x < -0.9999f, because -0.9999f is the
-// smallest float not below -0.9999 (checked exhaustively on [-1, -0.99] by
-// tests/test_oracle.py).
+// The same comparison and that with the slot kill threshold -0.9999
+// (3DgrainMPI/APTPhaseField.cu:341, also a double) in float, exact for every
+// float x: (double)x > -0.995 <=> x > -0.995f, because -0.995f is the largest
+// float not above -0.995; (double)x < -0.9999 <=> x < -0.9999f, because -0.9999f
+// is the smallest float not below -0.9999 (checked exhaustively on [-1, -0.99]
+// by tests/test_oracle.py).
 constexpr float kLSf = -0.995f;
 constexpr float kKillf = -0.9999f;
 
@@ -78,7 +77,7 @@ struct StepArgs {
     unsigned ep_dst;       // epoch the destination buffer had before this step
     unsigned ep_new;       // epoch the destination buffer gets from this step
     int use_act;           // 0: process every plane (the map is still maintained)
-    int ntx, nty, ntiles;  // activity tiles (64x4, partial ones included)
+    int ntx, ntiles;       // activity tiles in x and in all (64x4, partial ones included)
     // Row map: one word per (row of a column tile, z plane) and buffer, epoch
     // << 4 | bound.  A row of a buffer may hold anything but empty pairs only
     // if its word's epoch is >= the buffer's, and then only in slots below
@@ -97,7 +96,7 @@ struct StepArgs {
     int fnx, fny, fnz;
     int L;                 // slot stride fnx*fny*fnz
     int nzchunk, kchunk;   // z-chunks per column, planes per chunk
-    int tiles_x, tiles_y;  // 64x4 column tiles (partial ones at the +x/+y end included;
+    int tiles_x;           // 64x4 column tiles in x (one partial at the +x end included;
                            // see kPartialMin)
     int bcx, bcy, bcz;
     int num_theta;
@@ -215,7 +214,7 @@ int step_kernel_slots(int K, int gather27, int device);
 int batch_kernel_slots(int K, int gather27, int device);
 // Workgroups of the (single or batched) overflow fix-up kernel that fit at once.
 int fixup_kernel_slots(int K, int gather27, int device, bool batch);
-// Batched step: plan, persistent step, fix-up and advance kernels.
+// Batched step: plan, step, fix-up and advance kernels.
 hipError_t launch_batch_step(const BatchArgs& b, int K, int gather27, hipStream_t stream);
 // Pieces shared by the per-K launchers.
 hipError_t launch_plan(const StepArgs& a, hipStream_t stream);

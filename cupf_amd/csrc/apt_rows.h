@@ -29,8 +29,11 @@ constexpr int kRowLanes = 64;  // one wave per workgroup: rows need no barrier
 
 // Step arguments through a pointer the compiler cannot look through: fields
 // are scalar loads where they are used, instead of ~100 uniform values held in
-// (and spilled from) scalar registers across the whole kernel (174 spills and
-// 123 vector registers before, none and 110 with it, for the general path).
+// (and spilled from) scalar registers across the whole kernel (174 scalar
+// spills at first).  apt_step now, by the compiler's report, under the 128
+// vector registers of 4 waves per SIMD: K = 5 115 registers and 5 scalar spills
+// (27 points 111 and none); K = 8 128 with 24 scalar and 4 vector spills, 20 B of
+// scratch a lane (27 points 5, 5 and 24 B).
 typedef const __attribute__((address_space(4))) StepArgs CArgs;
 __device__ __forceinline__ const StepArgs* args_ref(CArgs* p)
 {

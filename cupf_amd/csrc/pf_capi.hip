@@ -62,13 +62,13 @@ struct pf_ctx {
     unsigned ep[2] = {1u, 1u};
     unsigned ep_ctr = 1u;
     int use_act = 1;
-    int ntx = 0, nty = 0, ntiles = 0;
+    int ntx = 0, ntiles = 0;
     // Work list of the step (filled by the plan kernel).
     int* wl_item = nullptr;
     unsigned long long* wl_need = nullptr;
     unsigned long long nlaunch = 0;  // step launches so far (selects the counter set)
     int nzchunk = 0, items_chunk = 0;
-    int tiles_x = 0, tiles_y = 0;   // column tiles (partial ones included)
+    int tiles_x = 0;                // column tiles in x (a partial one included)
     int step_blocks = 0;            // step waves (kStepRounds x occupancy x CUs, at most one per unit)
     int fix_blocks = 0;             // fix-up workgroups (occupancy x CUs)
     bool have_coords = false, have_orient = false, have_state = false;
@@ -184,7 +184,6 @@ StepArgs make_step_args(pf_ctx* c, int src, float t, int use_iuc)
     a.kchunk = c->kchunk;
     a.nzchunk = c->nzchunk;
     a.tiles_x = c->tiles_x;
-    a.tiles_y = c->tiles_y;
     a.act_src = c->act[src];
     a.act_dst = c->act[1 - src];
     a.row_src = c->row[src];
@@ -194,7 +193,6 @@ StepArgs make_step_args(pf_ctx* c, int src, float t, int use_iuc)
     a.ep_new = ++c->ep_ctr;
     a.use_act = c->use_act;
     a.ntx = c->ntx;
-    a.nty = c->nty;
     a.ntiles = c->ntiles;
     a.items_chunk = c->items_chunk;
     a.step_blocks = c->step_blocks;
@@ -362,7 +360,7 @@ struct pf_batch {
     std::vector<pf_ctx*> ctxs;
     int device = 0, K = 0, g27 = 0;
     hipStream_t stream = nullptr;
-    int kchunk = 4;
+    int kchunk = 4;                 // planes per work item (64 mixed simulations: depth 2 2.207 s, 4 2.249, 8 2.269, 16 2.322)
     int step_blocks = 0;
     int fix_blocks = 0;
     BatchSim* sims = nullptr;       // device array, n entries
@@ -547,8 +545,7 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
     }
     if (const char* na = getenv("CUPF_NO_ACTIVITY")) c->use_act = atoi(na) ? 0 : 1;
     c->ntx = (p.fnx - 2 + 63) / 64;
-    c->nty = (p.fny - 2 + 3) / 4;
-    c->ntiles = c->ntx * c->nty;
+    c->ntiles = c->ntx * cap_tiles_y(p.fny);
     {
         // 64x4 column tiles, a partial one where the +x leftover is at least
         // kPartialMin wide and always in y; a narrower +x leftover is the strip
@@ -556,8 +553,7 @@ int pf_create(const pf_params* params, int device, pf_ctx** out)
         const int ex = (p.fnx - 2) - tiles_x * 64;
         if (ex >= kPartialMin) ++tiles_x;
         c->tiles_x = tiles_x;
-        c->tiles_y = (p.fny - 2 + 3) / 4;
-        c->items_chunk = c->tiles_x * c->tiles_y;
+        c->items_chunk = c->tiles_x * cap_tiles_y(p.fny);
         c->nzchunk = (p.fnz - 2 + c->kchunk - 1) / c->kchunk;
     }
     {
@@ -1345,8 +1341,8 @@ int pf_batch_create(pf_ctx* const* ctxs, int n, pf_batch** out)
     }
     b->step_blocks = batch_kernel_slots(b->K, b->g27, b->device);
     while (b->fix_segs < kSpread && 2 * b->fix_segs * n <= kBatchSpread) b->fix_segs *= 2;
-    // 2 fix-up workgroups per CU (3.60 s for the 64-simulation ensemble, against 3.63-3.65 s
-    // with the 4 or 6 per CU that fit)
+    // 2 fix-up workgroups per CU (2.231 s for 64 simulations of 2000 steps at depth 4, 2.255 s
+    // with one per CU, 2.232 / 2.241 / 2.246 with 3, 4 and the 5 that fit)
     {
         int ncu = 0;
         if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, b->device) == hipSuccess)

@@ -20,10 +20,11 @@ __device__ __forceinline__ int interior_index(unsigned s, int nx, int ny, int fn
     return ((int)k + 1) * fnx * fny + ((int)j + 1) * fnx + (int)i + 1;
 }
 
-// Counts per grain id of one workgroup's run of points, in LDS until its end: a large grain's address otherwise takes one global atomic per wave of
-// it, ~17 ns each one after the other (858 us for the areas of a solid 256^3
-// window with a few large grains, 180 now).  An id that finds no place in
-// kProbe probes goes to memory at once.
+// Counts per grain id of one workgroup's run of points, in LDS until its end: a
+// large grain's address otherwise takes one global atomic per wave of it, ~17 ns
+// each one after the other (area call of a solid 256^3 window with a few large
+// grains: 980 -> 256 us).  An id that finds no place in kProbe probes goes to
+// memory at once.
 // Runs are as long as kRunMax where that still gives kRunGroups workgroups
 // (150 workgroups of 8192 points took 85 us for 160x96x80, 38 with shorter
 // ones).  Longer runs save atomics of large grains but leave a thin layer of

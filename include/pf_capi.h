@@ -241,7 +241,7 @@ int pf_activity(pf_ctx* ctx, int which, unsigned char* map, long long* active, l
  * No counterpart in the reference, which runs one simulation per process
  * (3Dgrain/createcmd:1 launches them one after another).  A batch steps
  * several contexts of one device (same K and gather variant; grids, thermal
- * parameters and seeds may differ) with one plan, one persistent step, one
+ * parameters and seeds may differ) with one plan, one step, one
  * fix-up and one advance kernel per time step over all of them, so small
  * simulations share the GPU instead of each being launch-bound.  Every member
  * gets exactly the bits pf_step would give it: batching changes the schedule,
